@@ -35,6 +35,8 @@ SOURCES = [
     ("sq8_convrot.hip", "sq8_convrot", []),
     ("sq8_w8a8.hip", "sq8_w8a8", []),
     ("sq8_i8_inst.hip", "sq8_i8_inst", []),
+    ("sq8_group_inst.hip", "sq8_group_i8_nk", ["-DSQ8_MATH=1", "-DSQ8_WT=0", "-DSQ8_WL=1"]),
+    ("sq8_group_inst.hip", "sq8_group_i8_packed", ["-DSQ8_MATH=1", "-DSQ8_WT=0", "-DSQ8_WL=2"]),
     ("sq8_blocks.hip", "sq8_blocks", []),
     ("sq8_api.hip", "sq8_api", []),
 ]

@@ -35,6 +35,7 @@ struct sq8_ctx {
     rocblas_handle blas;    // the bf16-weight product's library GEMM (created on its first call)
     int wd_tile;            // measurement knobs, read once at sq8_create (SQ8_TILE, SQ8_Q8_TILE, SQ8_SPLITS): a
     int q8_tile;            // forced weight-direct / block-scale tile, or -1 (the product's own choice); the
+    int i8_tile;            // the W8A8 tile SQ8_TILE forces (the K-group tiles only), or -1
     int splits;             // skinny kernel's K split count (1: none, the default)
     int cus;                // the device's compute units, read once here: the tile rules' rounds
 };
@@ -91,6 +92,13 @@ int knob(const char *value, std::initializer_list<KnobValue> table) {
     for (const KnobValue &v : table)
         if (strcmp(value, v.name) == 0) return v.tile;
     return -1;
+}
+
+// A K-group tile's knob name → its tile id, or `other`.
+int group_knob(const char *value, int other) {
+    for (int i = 0; value && i < sq8::kGroupShapes; ++i)
+        if (strcmp(value, sq8::group_shapes[i].name) == 0) return sq8::GROUP_TILE0 + i;
+    return other;
 }
 
 bool is_glu(int epilogue) { return epilogue == SQ8_EPI_SILU_GLU || epilogue == SQ8_EPI_SITU_GLU; }
@@ -524,7 +532,11 @@ int run_w8a8(sq8_ctx *ctx, const W8A8 &q, double *gpu_seconds) {
         p.w = static_cast<const uint8_t *>(ctx->wpack);
         p.kt_w = (q.k + 63) / 64;
     }
-    e = sq8::launch_i8gemm(p, wl, q.residual ? sq8::EPI_RESIDUAL : q.epilogue,
+    int tile = ctx->i8_tile >= 0 ? ctx->i8_tile : sq8::choose_i8_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, p.kt);
+    // A forced tile of an odd number of 32-column blocks cannot hold a GLU pair.
+    if (is_glu(q.epilogue) && tile >= sq8::GROUP_TILE0 && sq8::group_shapes[tile - sq8::GROUP_TILE0].cols % 64 != 0)
+        tile = sq8::I8_128x256;
+    e = sq8::launch_i8gemm(p, tile, wl, q.residual ? sq8::EPI_RESIDUAL : q.epilogue,
                            q.c_dtype == SQ8_F32 ? sq8::OUT_F32 : sq8::OUT_BF16, ctx->stream);
     if (e != hipSuccess) return hip_status(e);
     if (gpu_seconds) {
@@ -781,6 +793,7 @@ int sq8_create(int device, void *stream, sq8_ctx **out) {
                                              {"32", sq8::WD_32}, {"64n", sq8::WD_64N}, {"64x192", sq8::WD_64x192}, {"s64", sq8::WD_SKINNY64}, {"s32", sq8::WD_SKINNY32},
                                              {"gemv", sq8::WD_GEMV}, {"k32x32", sq8::WD_K32x32}, {"k32x64", sq8::WD_K32x64},
                                              {"k64x64", sq8::WD_K64x64}, {"k64x128", sq8::WD_K64x128}, {"k64x192", sq8::WD_K64x192}});
+    ctx->i8_tile = group_knob(getenv("SQ8_TILE"), knob(getenv("SQ8_TILE"), {{"128", sq8::I8_128x256}}));
     ctx->q8_tile = knob(getenv("SQ8_Q8_TILE"), {{"256", sq8::BL_64x256}, {"512", sq8::BL_64x512},
                                                 {"128x256", sq8::BL_128x256}, {"128x128", sq8::BL_128x128}});
     const char *splits = getenv("SQ8_SPLITS");

@@ -37,6 +37,7 @@ struct GemmArgs {
     int splits;             // > 1: the skinny kernel's K steps split over this many workgroups per tile, whose
                             // sums a second launch adds in split order before the epilogue
     int cus;                // the device's compute units (0: 256), for launch shapes chosen per product
+    int epi, out;           // set by the launcher of a kernel that reads them at run time (sq8_group_kernel.h)
 };
 
 enum Tile { TILE_256x256 = 0, TILE_128x128 = 1 };
@@ -76,6 +77,32 @@ __host__ __device__ constexpr bool gemv_x_in_lds(int m, int kt) {
 // Bytes of the partial sums of a split skinny product (tile height bm, `splits` splits).
 int64_t skinny_part_bytes(int M, int N, bool glu, int bm, int splits);
 hipError_t launch_wdirect(const GemmArgs &p, int tile, int wt, int wl, int epi, int out, hipStream_t stream);
+
+// The K-group kernels (sq8_group_kernel.h): `rows` × `cols` tiles (cols: weight columns) whose K steps split over
+// `groups` wave groups; GLU products take those of an even number of 32-column blocks. What a round of tiles on
+// the CUs, one a CU, takes on W8A8 operands: us + us_step · (K steps of 128) microseconds, fitted to 256 and 512
+// tiles at K = 1024, 3072 and 8192 (graph launches, the launch's own 2.5 µs taken off).
+struct GroupShape {
+    int rows, cols, groups;
+    float us, us_step;
+    const char *name;  // the SQ8_TILE knob's name for it
+};
+constexpr int GROUP_TILE0 = 100;  // tile ids of the K-group kernels: GROUP_TILE0 + index into group_shapes
+constexpr GroupShape group_shapes[] = {
+    {32, 32, 8, 0.65f, 0.104f, "g32x32k8"},
+    {32, 64, 8, 0.55f, 0.165f, "g32x64k8"},
+    {64, 64, 4, 1.60f, 0.204f, "g64x64k4"},
+    {64, 96, 4, 2.65f, 0.243f, "g64x96k4"},
+    {64, 128, 4, 2.30f, 0.325f, "g64x128k4"},
+    {96, 96, 4, 3.60f, 0.312f, "g96x96k4"},
+    {96, 128, 4, 4.40f, 0.408f, "g96x128k4"},
+    {128, 96, 4, 4.70f, 0.402f, "g128x96k4"},
+    {128, 128, 2, 6.30f, 0.493f, "g128x128k2"},
+    {96, 192, 2, 6.30f, 0.560f, "g96x192k2"},
+    {128, 192, 2, 8.70f, 0.694f, "g128x192k2"},
+};
+constexpr int kGroupShapes = (int)(sizeof(group_shapes) / sizeof(group_shapes[0]));
+hipError_t launch_group_i8(const GemmArgs &p, int shape, int wl, int epi, int out, hipStream_t stream);
 
 // Bytes of the packed layout of a weight with k rows of K and n columns (GLU: n = 2h, packed in
 // pairs of 32-column blocks of the two halves).
@@ -137,7 +164,10 @@ hipError_t launch_quantize_rows(const void *x, bool x_bf16, int64_t ldx, int row
                                 int64_t ldq, int k_pad, float *scales, hipStream_t stream);
 hipError_t launch_pad_codes(const int8_t *src, int64_t ld_src, int8_t *dst, int64_t ld_dst, int64_t rows, int k, int k_pad,
                             hipStream_t stream);
-hipError_t launch_i8gemm(const GemmArgs &p, int wl, int epi, int out, hipStream_t stream);
+// `tile`: choose_i8_tile's: I8_128x256 (128 × 256, two workgroups a CU) or a K-group tile's id. kt: K steps of 128.
+constexpr int I8_128x256 = 0;
+int choose_i8_tile(int M, int N, bool glu, int cus, int kt);
+hipError_t launch_i8gemm(const GemmArgs &p, int tile, int wl, int epi, int out, hipStream_t stream);
 
 // The DiT block's elementwise passes (sq8_block.hip).
 hipError_t launch_norm_modulate(const float *x, int64_t ldx, const float *w, const float *scale, const float *shift,

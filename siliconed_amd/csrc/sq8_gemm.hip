@@ -19,6 +19,13 @@ hipError_t launch_wdirect(const GemmArgs &p, int tile, int wt, int wl, int epi, 
     return wl == W_NK ? launch_wdirect_1_1(p, tile, epi, out, stream) : launch_wdirect_1_2(p, tile, epi, out, stream);
 }
 
+hipError_t launch_group_1_0_1(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+hipError_t launch_group_1_0_2(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+
+hipError_t launch_group_i8(const GemmArgs &p, int shape, int wl, int epi, int out, hipStream_t stream) {
+    return wl == W_NK ? launch_group_1_0_1(p, shape, epi, out, stream) : launch_group_1_0_2(p, shape, epi, out, stream);
+}
+
 // The tile before the K-group tiles are considered.
 static int base_wd_tile(int M, int N, bool glu, int cus) {
     // Tiles of 256 columns (four 64-column slabs; GLU: 32 output columns a slab), as tall as keeps
@@ -113,6 +120,42 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int kt) {
             most = count(c);
         }
     return best;
+}
+
+// Microseconds of `tiles` workgroups, `cus` at a time, `round` each: a last, partly filled round is shorter (its
+// workgroups share the memory system with fewer others: half the CUs 0.83 of a full round).
+static float rounds_us(long tiles, int cus, float round) {
+    const long full = tiles / cus, rest = tiles % cus;
+    return round * ((float)full + (rest ? 0.66f + 0.34f * (float)rest / (float)cus : 0.0f));
+}
+
+int choose_i8_tile(int M, int N, bool glu, int cus, int kt) {
+    // The tile of the least estimated time. Every tile gives the same bits (int32 sums), so only time decides; the
+    // 128 × 256 kernel's rounds (two workgroups a CU: 11.2 + 1.70 µs a K step; one: 9.6 + 0.91) are measured as the
+    // K-group tiles' (GroupShape). It has the least operand traffic per output and wins where its tiles fill the
+    // chip (K = 3072: 4096 × 12288 150 µs against 203 in 128 × 192); with fewer the K-group tiles spread the work
+    // over more CUs and hold more loads in flight a CU. Measured, K = 3072, product alone, µs, 128 × 256 tiles
+    // against the rule's: 1 × 3072 20.8 → 4.9, 77 × 12288 22.6 → 12.9, 512 × 3072 23.0 → 10.8, 1021 × 3072 24.5 →
+    // 17.0, 333 × 9216 25.0 → 20.0; K = 12288, 68 × 512 62.9 → 9.7.
+    if (cus <= 0) cus = 256;
+    const long blocks = glu ? 2 * (((long)N / 2 + 31) / 32) : ((long)N + 31) / 32;  // 32-column blocks
+    const long big = (long)((M + 127) / 128) * ((blocks + 7) / 8), slots = 2L * cus;
+    const float two = 11.2f + 1.70f * (float)kt, one = 9.6f + 0.91f * (float)kt;
+    const long rest = big % slots;
+    float best = (float)(big / slots) * two + (rest > cus ? two : rounds_us(rest, cus, one));
+    int tile = I8_128x256;
+    for (int i = 0; i < kGroupShapes; ++i) {
+        const GroupShape &g = group_shapes[i];
+        const int nw = g.cols / 32;
+        if (glu && nw % 2 != 0) continue;
+        const float us = rounds_us((long)((M + g.rows - 1) / g.rows) * ((blocks + nw - 1) / nw), cus,
+                                   g.us + g.us_step * (float)kt);
+        if (us < best) {
+            best = us;
+            tile = GROUP_TILE0 + i;
+        }
+    }
+    return tile;
 }
 
 int64_t skinny_part_bytes(int M, int N, bool glu, int bm, int splits) {

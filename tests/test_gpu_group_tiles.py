@@ -1,0 +1,55 @@
+"""The K-group tiles (the K steps split over wave groups, the groups' sums added in LDS) on an MI355X: every tile at
+its edges — one row, a row and a column past the tile, a K with fewer steps than groups, one that does not divide
+among them and one that does —, each epilogue, output type, output layout and weight layout, bit for bit against the
+128 × 256 kernel on the same operands (W8A8 sums are exact integers: any split of K gives the same bits)."""
+import pytest
+import torch
+
+from test_gpu_parity import DEV, dev
+
+pytestmark = pytest.mark.gpu
+
+W8A8_TILES = ["g32x32k8", "g32x64k8", "g64x64k4", "g64x96k4", "g64x128k4", "g96x96k4", "g96x128k4", "g128x96k4",
+              "g128x128k2", "g96x192k2", "g128x192k2"]
+
+
+def _w8a8_operands(m, k, n, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    codes = torch.randint(-128, 128, (m, k), dtype=torch.int8, device=DEV, generator=g)
+    w = torch.randint(-127, 128, (n, k), dtype=torch.int8, device=DEV, generator=g)
+    sx, s = (torch.rand(size, device=DEV, generator=g) * 1e-2 + 1e-3 for size in (m, n))
+    return codes, sx, w, s, torch.randn(n, device=DEV, generator=g)
+
+
+@pytest.mark.parametrize("tile", W8A8_TILES)
+def test_w8a8_group_tile_same_bits(tile_gemm, tile):
+    bm, bn = (int(v) for v in tile[1:].split("k")[0].split("x"))
+    got, want = tile_gemm(tile), tile_gemm("128")
+    cases = [(1, 128, bn, None, torch.float32, False), (bm + 1, 640, bn + 32, "gelu_tanh", torch.bfloat16, False),
+             (bm, 1024, bn + 4, None, torch.bfloat16, True), (2 * bm - 1, 1152, 2 * bn + 1, None, torch.float32, False),
+             (bm - 1, 200, bn - 3, "gelu_tanh", torch.float32, False)]
+    if bn % 64 == 0:
+        cases += [(bm + 3, 640, 2 * (bn // 2 + 5), "silu_glu", torch.bfloat16, False),
+                  (bm, 1024, 2 * bn, "situ_glu", torch.float32, False)]
+    for m, k, n, epi, out, nk in cases:
+        print(f"{tile}: {m} x {k} x {n} {epi} {out} {'nk' if nk else 'packed'}", flush=True)
+        codes, sx, w, s, b = _w8a8_operands(m, k, n, m + k + n)
+        if not nk:
+            w = want.pack(w, layout="nk", glu=epi in ("silu_glu", "situ_glu"))
+        ys = [g.product_w8a8(codes, sx, w, s, bias=b, epilogue=epi, out_dtype=out) for g in (got, want)]
+        torch.cuda.synchronize()
+        assert torch.equal(*ys)
+    # Three outputs (row-major, head-major), and the residual stream in place.
+    m, k, d = bm + 2, 1024, 128
+    codes, sx, w, s, b = _w8a8_operands(m, k, 3 * d, 7)
+    w = want.pack(w, layout="nk")
+    for head_dim in (0, 32):
+        parts = [g.product_w8a8_qkv(codes, sx, w, s, bias=b, head_dim=head_dim) for g in (got, want)]
+        torch.cuda.synchronize()
+        assert all(torch.equal(x, y) for x, y in zip(*parts))
+    gate = torch.linspace(-1.0, 1.0, 3 * d, device=DEV)
+    streams = [torch.ones((m, 3 * d), device=DEV) for _ in range(2)]
+    for g, x in zip((got, want), streams):
+        g.product_w8a8_residual(x, codes, sx, w, s, bias=b, gate=gate)
+    torch.cuda.synchronize()
+    assert torch.equal(*streams)
