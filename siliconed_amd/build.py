@@ -38,6 +38,7 @@ SOURCES = [
     ("sq8_group_inst.hip", "sq8_group_i8_nk", ["-DSQ8_MATH=1", "-DSQ8_WT=0", "-DSQ8_WL=1"]),
     ("sq8_group_inst.hip", "sq8_group_i8_packed", ["-DSQ8_MATH=1", "-DSQ8_WT=0", "-DSQ8_WL=2"]),
     ("sq8_blocks.hip", "sq8_blocks", []),
+    ("sq8_blocks16_inst.hip", "sq8_blocks16_inst", []),
     ("sq8_api.hip", "sq8_api", []),
 ]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -659,9 +659,9 @@ int run_blocks(sq8_ctx *ctx, const Blocks &q, double *gpu_seconds) {
     p.glu_half = is_glu(q.epilogue) ? q.n / 2 : 0;
     const size_t esz = q.c_dtype == SQ8_F32 ? 4 : 2;
     p.c_vec16 = aligned(q.c, 16) && (q.ldc % (int64_t)(16 / esz)) == 0;
-    // 128-row tiles of one 32-column block per wave (the codes widened once for twice the rows);
-    // the GLU epilogues pair both blocks of a slab in one wave: 64-row tiles.
-    const int tile = ctx->q8_tile >= 0 ? ctx->q8_tile : is_glu(q.epilogue) ? sq8::BL_64x256 : sq8::BL_128x256;
+    p.c_vec = aligned(q.c, 4 * esz) && (q.ldc % 4) == 0;
+    p.sb_vec = !p.bias || (aligned(p.bias, 16) && (p.glu_half % 4) == 0);
+    const int tile = ctx->q8_tile >= 0 ? ctx->q8_tile : sq8::choose_blocks_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, p.kt);
     hipError_t e = sq8::launch_blocks_product(p, tile, q.epilogue, q.c_dtype == SQ8_F32 ? sq8::OUT_F32 : sq8::OUT_BF16,
                                   ctx->stream);
     if (e != hipSuccess) return hip_status(e);
@@ -794,8 +794,10 @@ int sq8_create(int device, void *stream, sq8_ctx **out) {
                                              {"gemv", sq8::WD_GEMV}, {"k32x32", sq8::WD_K32x32}, {"k32x64", sq8::WD_K32x64},
                                              {"k64x64", sq8::WD_K64x64}, {"k64x128", sq8::WD_K64x128}, {"k64x192", sq8::WD_K64x192}});
     ctx->i8_tile = group_knob(getenv("SQ8_TILE"), knob(getenv("SQ8_TILE"), {{"128", sq8::I8_128x256}}));
-    ctx->q8_tile = knob(getenv("SQ8_Q8_TILE"), {{"256", sq8::BL_64x256}, {"512", sq8::BL_64x512},
-                                                {"128x256", sq8::BL_128x256}, {"128x128", sq8::BL_128x128}});
+    ctx->q8_tile = knob(getenv("SQ8_Q8_TILE"), {{"128x256", sq8::BL_128x256}, {"128x128", sq8::BL_128x128},
+                                                {"16", sq8::BLOCKS16_ROWS + 16}, {"32", sq8::BLOCKS16_ROWS + 32},
+                                                {"48", sq8::BLOCKS16_ROWS + 48}, {"64", sq8::BLOCKS16_ROWS + 64},
+                                                {"80", sq8::BLOCKS16_ROWS + 80}});
     const char *splits = getenv("SQ8_SPLITS");
     ctx->splits = splits && atoi(splits) >= 1 ? atoi(splits) : 1;
     uint8_t *unused = nullptr;

@@ -9,7 +9,7 @@ namespace sq8 {
 
 namespace {
 
-constexpr int S_BF16 = 1, S_F32 = 2, S_F16 = 5;  // numbered as the C ABI's sq8_dtype
+constexpr int S_BF16 = 1, S_F16 = 5;  // numbered as the C ABI's sq8_dtype (2, fp32, otherwise)
 
 __device__ __forceinline__ float scale_value(const void *s, int kind, int64_t i) {
     if (kind == S_BF16) return __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(s)[i] << 16);
@@ -77,24 +77,6 @@ int grid_of(int64_t count) {
     return (int)(blocks < 8192 ? (blocks > 0 ? blocks : 1) : 8192);
 }
 
-template <int BM, int NW, int OCC, int NB>
-hipError_t dispatch(const GemmArgs &p, int epi, int out, hipStream_t stream) {
-#define SQ8_CASE(E, O)                                                                            \
-    if (epi == E && out == O) return blk::launch_blocks_product<BM, NW, OCC, NB, W_INT8, E, O>(p, stream);
-    SQ8_CASE(EPI_NONE, OUT_BF16)
-    SQ8_CASE(EPI_NONE, OUT_F32)
-    SQ8_CASE(EPI_GELU, OUT_BF16)
-    SQ8_CASE(EPI_GELU, OUT_F32)
-    if constexpr (NB == 2) {
-        SQ8_CASE(EPI_SILU_GLU, OUT_BF16)
-        SQ8_CASE(EPI_SILU_GLU, OUT_F32)
-        SQ8_CASE(EPI_SITU_GLU, OUT_BF16)
-        SQ8_CASE(EPI_SITU_GLU, OUT_F32)
-    }
-#undef SQ8_CASE
-    return hipErrorInvalidValue;
-}
-
 }  // namespace
 
 int64_t packed_blocks_bytes(int k, int n, bool glu) {
@@ -115,11 +97,9 @@ hipError_t launch_pack_blocks(const uint8_t *w, int wl, int64_t ldw, const void 
 }
 
 hipError_t launch_blocks_product(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream) {
-    const bool glu = epi == EPI_SILU_GLU || epi == EPI_SITU_GLU;
-    if (tile == BL_128x256 && !glu) return dispatch<128, 8, 1, 1>(p, epi, out, stream);
-    if (tile == BL_128x128 && !glu) return dispatch<128, 4, 2, 1>(p, epi, out, stream);
-    if (tile == BL_64x512) return dispatch<64, 8, 1, 2>(p, epi, out, stream);
-    return dispatch<64, 4, 2, 2>(p, epi, out, stream);
+    if (tile > BLOCKS16_ROWS) return launch_blocks16(p, tile - BLOCKS16_ROWS, epi, out, stream);
+    if (tile == BL_128x128) return blk::launch_blocks_product<128, 4>(p, epi, out, stream);
+    return blk::launch_blocks_product<128, 8>(p, epi, out, stream);
 }
 
 }  // namespace sq8

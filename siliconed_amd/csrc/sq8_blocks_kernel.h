@@ -12,16 +12,28 @@
 // equal to the reference's sum in exact arithmetic, rounded differently: one fp32 product and sum
 // per block instead of one fp32 product per weight.
 //
-// The weight-direct kernel's structure (sq8_wdirect_kernel.h: activation tiles through a 2-stage
-// LDS ring, each wave streaming its 64-column slab of packed codes straight into registers) with
-// three differences:
+// The weight-direct kernel's structure (sq8_wdirect_kernel.h: activation tiles through an LDS ring, each wave
+// streaming its packed codes straight into registers) with these differences:
 //   * the activation is the MFMA's first operand and the codes the second, so each lane's 16
 //     results of a 32 × 32 block share one column (lane & 31) and one scale per block of K;
 //   * a 64-step's K order keeps each block of 32 in two MFMA sub-steps: sub-step ks takes
 //     k ∈ [16·ks, 16·ks + 16), lane half h the 8 at 16·ks + 8·h — the packed Q8 layout stores the
 //     codes in that order, the activation fragment of (ks, h) is LDS chunk 2·ks + h;
-//   * per block: P = MFMA(A, q) over its two sub-steps (from zero), then acc += P · s (fp32 FMA),
-//     the scales of the step (two blocks × the lane's two 32-column blocks) one 16-byte load.
+//   * per block: P = MFMA(A, q) over its two sub-steps (from zero), then acc += P · s (fp32 FMA).
+//
+// What bounds it, and the schedule. Per MFMA (32 cycles of a SIMD's matrix core) a wave issues 8 rescale FMAs and
+// 3 widening operations, 44 cycles of the vector ALU: the kernel can only approach the vector ALU's time if the two
+// run side by side, and waves that run all their MFMAs and then all their FMAs, in step with each other between
+// barriers, add them (measured: 32 + 54 cycles). So the step is cut into four groups of one K block × two row
+// blocks: a group issues its four MFMAs (P of this group), and between them the 32 FMAs of the group before (whose P
+// is complete), a quarter of the widening and the next group's four fragment reads; the groups run on across steps
+// (the next step's first fragments and codes are taken during the last group). The order of every sum is unchanged.
+// Measured (µs, the groups against the plain order): one row of tiles alone, K = 3072, 52.4 → 46.5 in 128 × 256 and
+// 33.6 in 128 × 128; 1021 × 3072 × 3072 54.9 → 40.3 (128 × 128, two workgroups a CU: one's epilogue under the other's
+// MFMAs). On a full chip the clock follows the power (4096 × 3072 × 12288, the same 780 k cycles: 403 µs, with every
+// activation zero 349, with every code zero 321), so there the cycles saved come back as 2.5 % (400 → 391 µs).
+// Measured and not kept: eight activation stages with a barrier every two steps (402 against 406 µs, two registers
+// spilled).
 //
 // Packed Q8 layout (sq8_pack_blocks): the codes as the packed layout's chunks — chunk c =
 // ((slab·kt + t)·4 + j)·64 + lane, 16 bytes: k = 64t + 32(j&1) + 8h + [0, 8) then
@@ -31,7 +43,7 @@
 // the slab's 32 output columns of each half). Zeros past K and past the columns.
 #pragma once
 
-#include "sq8_wdirect_kernel.h"
+#include "sq8_group_kernel.h"
 
 namespace sq8 {
 namespace blk {
@@ -47,53 +59,19 @@ using wd::widen8;
 // Byte offset of the packed scales of a weight of kt steps and `slabs` slabs from the packed base.
 __host__ __device__ inline int64_t scales_offset(int64_t slabs, int64_t kt) { return slabs * kt * 4096; }
 
-// Bias, activation and store of one 32 × 32 block a wave holds in the transposed order (lane l,
-// register r: row 8·(r >> 2) + 4·(l >> 5) + (r & 3), column l & 31): written value by value into the
-// wave's LDS region, then stored as the weight-direct epilogue stores (flush_region).
-template <int EPI, int OUT>
-__device__ __forceinline__ void store_block_t(const GemmArgs &p, const f32x16 &x, float bx, const f32x16 &u, float bu,
-                                              int col0, int m_first, int n_out, uint8_t *region, int lane) {
-    constexpr bool GLU = EPI == EPI_SILU_GLU || EPI == EPI_SITU_GLU;
-    constexpr int ESZ = OUT == OUT_BF16 ? 2 : 4;
-    constexpr int PITCH = 32 * ESZ + 16;
-    const int h = lane >> 5, c = lane & 31;
-    wd::ResidualPre pre;
-    if constexpr (EPI == EPI_RESIDUAL) wd::load_residual(p, col0, m_first, n_out, lane, pre);
-    static_for<0, 16>([&](auto rc) {
-        constexpr int r = decltype(rc)::value;
-        float v = __fadd_rn(x[r], bx);
-        if constexpr (EPI == EPI_GELU) {
-            v = gelu_tanh(v);
-        } else if constexpr (GLU) {
-            const float w = __fadd_rn(u[r], bu);
-            v = EPI == EPI_SILU_GLU ? silu_glu(v, w) : situ(v, w);
-        }
-        uint8_t *dst = region + (8 * (r >> 2) + 4 * h + (r & 3)) * PITCH + c * ESZ;
-        if constexpr (OUT == OUT_BF16)
-            *reinterpret_cast<uint16_t *>(dst) = (uint16_t)round_bf16(v);
-        else
-            *reinterpret_cast<float *>(dst) = v;
-    });
-    wd::flush_region<EPI, OUT>(p, col0, m_first, n_out, region, lane, EPI == EPI_RESIDUAL ? &pre : nullptr);
-}
-
-// NB: 32-column blocks per wave — 2 (the wave owns a 64-column slab) or 1 (waves in pairs share a
-// slab, wave w taking block w & 1: half the registers per row block, so twice the rows fit).
-template <int BM, int NW, int OCC, int NB, int WT, int EPI, int OUT>
-__global__ void __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW), amdgpu_waves_per_eu(OCC, OCC)))
+template <int BM, int NW>
+__global__ void __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW), amdgpu_waves_per_eu(2, 2)))
 gemm_blocks_kernel(const GemmArgs p) {
-    static_assert(NB == 1 || NB == 2, "one or two 32-column blocks a wave");
-    static_assert(NB == 2 || NW % 2 == 0, "waves in pairs");
-    constexpr bool GLU = EPI == EPI_SILU_GLU || EPI == EPI_SITU_GLU;
+    static_assert(NW % 2 == 0, "wave w: block w & 1 of slab w ÷ 2 of the tile's");
     constexpr int FM = BM / 32;
+    static_assert(FM % 2 == 0, "row blocks in pairs");
+    constexpr int NAS = 4;                    // activation stages and code buffers
     constexpr int SA = BM * 128;
-    constexpr int A_BLOCKS = BM / 8;
-    constexpr int A_PER_WAVE = A_BLOCKS / NW;
-    static_assert(A_BLOCKS % NW == 0, "the activation blocks split evenly over the waves");
-    constexpr int WLOADS = 2 * NB + 1;  // code loads + the scale load per step
-    static_assert(A_PER_WAVE + WLOADS < 64, "vmcnt budget");
-    constexpr int REGION = 32 * (32 * (OUT == OUT_BF16 ? 2 : 4) + 16);
-    constexpr int LDS_BYTES = NW * REGION > 2 * SA ? NW * REGION : 2 * SA;  // epilogue regions over the stages
+    constexpr int A_PER_WAVE = BM / 8 / NW;
+    static_assert(BM / 8 % NW == 0, "the activation blocks split evenly over the waves");
+    constexpr int GROUPS = FM;                // groups a step: two K blocks × FM/2 pairs of row blocks
+    constexpr int WLOADS = 3;                 // two code loads and a scale load per step
+    constexpr int LDS_BYTES = NAS * SA > NW * grp::SLOT ? NAS * SA : NW * grp::SLOT;
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_BYTES];
 
@@ -102,51 +80,46 @@ gemm_blocks_kernel(const GemmArgs p) {
     int tm, tn;
     kern::tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
     const int m0 = tm * BM;
-    const int slabs = GLU ? (p.glu_half + 31) / 32 : (p.N + 63) / 64;
-    constexpr int SLABS_PER_WG = NB == 2 ? NW : NW / 2;
-    const int slab = tn * SLABS_PER_WG + (NB == 2 ? wave : wave >> 1);
-    const int b0 = NB == 2 ? 0 : (wave & 1);  // the wave's first 32-column block in the slab
-    const int rslab = slab < slabs ? slab : slabs - 1;  // a wave past the last slab reads the last
-    const kern::gbytes Ag = (kern::gbytes)p.a;
+    const bool glu = p.glu_half > 0;
+    const int slabs = glu ? (p.glu_half + 31) / 32 : (p.N + 63) / 64;
+    const int slab = min(tn * (NW / 2) + (wave >> 1), slabs - 1);  // a wave past the last slab reads the last
+    const int b0 = wave & 1;
     const kern::gbytes Wg = (kern::gbytes)p.w;
     const int KT = p.kt;
 
     uint32_t a_goff[A_PER_WAVE];
 #pragma unroll
     for (int i = 0; i < A_PER_WAVE; ++i) {
-        const int b = wave + NW * i;
-        const int r = 8 * b + (lane >> 3);
+        const int r = 8 * (wave + NW * i) + (lane >> 3);
         const int lc = (lane & 7) ^ ((r ^ (r >> 3)) & 7);
-        const int row = min(m0 + r, p.M - 1);
-        a_goff[i] = (uint32_t)((int64_t)row * p.lda * 2) + lc * 16;
+        a_goff[i] = (uint32_t)((int64_t)min(m0 + r, p.M - 1) * p.lda * 2) + lc * 16;
     }
+    const wd::i32x4 a_rsrc = wd::buffer_rsrc(p.a);
+    auto issue_a1 = [&](int t, auto stage, auto ic) {  // load ic of step t
+        constexpr int S = decltype(stage)::value, i = decltype(ic)::value;
+        const int soff = __builtin_amdgcn_readfirstlane((int)((uint32_t)min(t, KT - 1) * 128));
+        wd::raw_buffer_load_lds(a_rsrc, (wd::lds_u32)(lds + S * SA + (wave + NW * i) * 1024), 16, (int)a_goff[i], soff, 0, 0);
+    };
     auto issue_a = [&](int t, auto stage) {
-        constexpr int S = decltype(stage)::value;
-        const kern::gbytes base = Ag + (uint32_t)min(t, KT - 1) * (BK * 2);
-#pragma unroll
-        for (int i = 0; i < A_PER_WAVE; ++i)
-            __builtin_amdgcn_global_load_lds((glb_ptr)(base + a_goff[i]), (lds_ptr)(lds + S * SA + (wave + NW * i) * 1024),
-                                             16, 0, 0);
+        static_for<0, A_PER_WAVE>([&](auto ic) { issue_a1(t, stage, ic); });
     };
 
-    // Codes: 4 × 16 bytes per lane per step; scales: 16 bytes per lane per step (lanes l and l + 32
-    // read the same).
-    // The weight's K steps: KT, or kt_w when the activation holds several parts along K that each face
-    // the whole weight (the fp32 route), the weight's step then t modulo kt_w.
+    // Codes: 2 × 16 bytes per lane per step (the two K blocks); scales: the lane's column's two, 8 bytes. The weight's
+    // K steps: KT, or kt_w when the activation holds several parts along K that each face the whole weight (the fp32
+    // route), the weight's step then t modulo kt_w.
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
     const int KW = p.kt_w > 0 ? p.kt_w : KT;
-    const uint32_t w_base = (uint32_t)((int64_t)rslab * KW * 4096) + lane * 16;
-    const uint32_t s_base = (uint32_t)(scales_offset(slabs, KW) + (int64_t)rslab * KW * 512) + (lane & 31) * 16;
-    // raw[B][2·b + kb]: the codes of the wave's block b (0..NB−1 from b0), K block kb of the step.
-    constexpr int NLOAD = 2 * NB;
-    u32x4 raw[2][NLOAD];
-    f32x4 sraw[2];
+    const uint32_t w_off = (uint32_t)((int64_t)slab * KW * 4096) + b0 * 2048 + lane * 16;
+    const uint32_t s_off = (uint32_t)(scales_offset(slabs, KW) + (int64_t)slab * KW * 512) + (lane & 31) * 16 + 8 * b0;
+    u32x4 raw[NAS][2];
+    f32x2 sraw[NAS];
     auto issue_w = [&](int t, auto buf) {
         constexpr int B = decltype(buf)::value;
         const int tt = wd::weight_step(p, min(t, KT - 1));
         const kern::gbytes base = Wg + (uint32_t)tt * 4096;
-#pragma unroll
-        for (int j = 0; j < NLOAD; ++j) raw[B][j] = kern::gld<u32x4>(base, w_base + (2 * b0 + j) * 1024);
-        sraw[B] = kern::gld<f32x4>(Wg + (uint32_t)tt * 512, s_base);
+        raw[B][0] = kern::gld<u32x4>(base, w_off);
+        raw[B][1] = kern::gld<u32x4>(base, w_off + 1024);
+        sraw[B] = kern::gld<f32x2>(Wg + (uint32_t)tt * 512, s_off);
     };
 
     const int h = lane >> 5;
@@ -156,142 +129,165 @@ gemm_blocks_kernel(const GemmArgs p) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) xo[par][ks] = swz(32 * par + (lane & 31), 2 * ks + h) - 32 * 128 * par;
 
-    f32x16 acc[NB][FM];
+    f32x16 acc[FM];
+    f32x16 pp[2][2];       // [group & 1][row block of the pair]
+    bf16x8 xf[2][2][2];    // [group & 1][row block of the pair][sub-step of the K block]
+    bf16x8 wk[2][2];       // [K block][sub-step]
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+    for (int bm = 0; bm < FM; ++bm)
 #pragma unroll
-        for (int bm = 0; bm < FM; ++bm)
+        for (int r = 0; r < 16; ++r) acc[bm][r] = 0.0f;
+    // The first step's "group before": sums of zero.
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[b][bm][r] = 0.0f;
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) pp[1][i][r] = 0.0f;
+    float sp = 0.0f;       // the scale of the group before
 
+    auto read_x = [&](auto stage, auto gc, auto dst) {  // group gc's fragments
+        constexpr int S = decltype(stage)::value, g = decltype(gc)::value, D = decltype(dst)::value;
+        constexpr int kb = g / (FM / 2), pair = g % (FM / 2);
+        static_for<0, 2>([&](auto kc) {
+            constexpr int ks = decltype(kc)::value;
+            static_for<0, 2>([&](auto ic) {
+                constexpr int i = decltype(ic)::value;
+                xf[D][i][ks] = kern::lds_load_frag(lds + S * SA + 32 * 128 * (2 * pair + i), xo[i][2 * kb + ks]);
+            });
+        });
+    };
+    auto widen = [&](auto buf, auto bc, auto kc) {
+        constexpr int B = decltype(buf)::value, kb = decltype(bc)::value, ks = decltype(kc)::value;
+        wk[kb][ks] = widen8<W_INT8>(raw[B][kb][2 * ks], raw[B][kb][2 * ks + 1]);
+    };
+    auto rescale = [&](auto gc, float s) {  // group gc's P into the totals
+        constexpr int g = decltype(gc)::value, pair = g % (FM / 2);
+        static_for<0, 2>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[2 * pair + i][r] = __builtin_fmaf(pp[g & 1][i][r], s, acc[2 * pair + i][r]);
+        });
+    };
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
 
-    issue_a(0, I0{});
-    issue_w(0, I0{});
-    issue_w(1, I1{});
-    wait_vmcnt<WLOADS>();
+    // Prologue: W(0 .. 2) and A(0 .. 2), all landed (the compiler's own waits for the codes of the first steps then
+    // count from here; behind loads in flight they would drain the loop's prefetch too).
+    static_for<0, NAS - 1>([&](auto vc) { issue_w(decltype(vc)::value, vc); });
+    static_for<0, NAS - 1>([&](auto vc) { issue_a(decltype(vc)::value, vc); });
+    wait_vmcnt<0>();
     step_barrier();
+    read_x(I0{}, I0{}, I0{});
+    widen(I0{}, I0{}, I0{});
+    widen(I0{}, I0{}, I1{});
 
-    auto step = [&](int t, auto par) {
-        constexpr int P = decltype(par)::value;
-        bf16x8 wk[2][NB];  // [ks & 1][block]
-        bf16x8 xf[2][FM];
-        f32x16 pp[NB][FM];
-        const f32x4 sv = sraw[P];
-        auto widen_ks = [&](auto kc) {
-            constexpr int ks = decltype(kc)::value;
-            static_for<0, NB>([&](auto bc) {
-                constexpr int b = decltype(bc)::value;
-                const u32x4 &r = raw[P][2 * b + (ks >> 1)];
-                wk[ks & 1][b] = widen8<WT>(r[2 * (ks & 1)], r[2 * (ks & 1) + 1]);
-            });
-        };
-        auto read_x = [&](auto kc) {
-            constexpr int ks = decltype(kc)::value;
-            static_for<0, FM>([&](auto bmc) {
-                constexpr int bm = decltype(bmc)::value;
-                xf[ks & 1][bm] = kern::lds_load_frag(lds + P * SA + 32 * 128 * bm, xo[bm & 1][ks]);
-            });
-        };
-        __builtin_amdgcn_sched_barrier(0);
-        read_x(I0{});
-        widen_ks(I0{});
-        issue_a(t + 1, std::integral_constant<int, 1 - P>{});
-        static_for<0, 4>([&](auto kc) {
-            constexpr int ks = decltype(kc)::value;
-            if constexpr (ks < 3) {
-                read_x(std::integral_constant<int, ks + 1>{});
-                widen_ks(std::integral_constant<int, ks + 1>{});
+    // Step t on stage and code buffer U = t mod 4.
+    auto step = [&](int t, auto uc) {
+        constexpr int U = decltype(uc)::value;
+        using SU = std::integral_constant<int, U>;
+        using S1 = std::integral_constant<int, (U + 1) % NAS>;
+        using S3 = std::integral_constant<int, (U + 3) % NAS>;
+        static_for<0, GROUPS>([&](auto gc) {
+            constexpr int g = decltype(gc)::value, kb = g / (FM / 2), pair = g % (FM / 2);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (g + 1 < GROUPS)
+                read_x(SU{}, std::integral_constant<int, g + 1>{}, std::integral_constant<int, (g + 1) & 1>{});
+            else
+                read_x(S1{}, I0{}, I0{});  // the next step's first
+            // The next K block's codes: one sub-step each in the K block's last two groups.
+            if constexpr (pair >= FM / 2 - 2) {
+                using KS = std::integral_constant<int, pair - (FM / 2 - 2)>;
+                if constexpr (kb == 0) widen(SU{}, I1{}, KS{});
+                else widen(S1{}, I0{}, KS{});
             }
-            if constexpr (ks == 2) {
-                __builtin_amdgcn_sched_barrier(0);
-                issue_w(t + 2, std::integral_constant<int, P>{});
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            static_for<0, NB>([&](auto bc) {
-                constexpr int b = decltype(bc)::value;
-                static_for<0, FM>([&](auto bmc) {
-                    constexpr int bm = decltype(bmc)::value;
-                    if constexpr ((ks & 1) == 0)
-                        pp[b][bm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[ks & 1][bm], wk[ks & 1][b],
-                                                                            f32x16{}, 0, 0, 0);
+            // Into the stage and buffer last read during step t − 1 (its barrier saw every wave's reads).
+            if constexpr (g < A_PER_WAVE) issue_a1(t + 3, S3{}, gc);
+            if constexpr (g == GROUPS - 1) issue_w(t + 3, S3{});
+            static_for<0, 2>([&](auto kc) {
+                constexpr int ks = decltype(kc)::value;
+                static_for<0, 2>([&](auto ic) {
+                    constexpr int i = decltype(ic)::value;
+                    if constexpr (ks == 0)
+                        pp[g & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[g & 1][i][0], wk[kb][0], f32x16{}, 0, 0, 0);
                     else
-                        pp[b][bm] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[ks & 1][bm], wk[ks & 1][b], pp[b][bm],
-                                                                            0, 0, 0);
+                        pp[g & 1][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[g & 1][i][1], wk[kb][1], pp[g & 1][i], 0, 0, 0);
                 });
             });
-            if constexpr ((ks & 1) == 1) {
-                // The block of K ends: its partial sums scaled into the totals.
-                static_for<0, NB>([&](auto bc) {
-                    constexpr int b = decltype(bc)::value;
-                    const float s = NB == 2 ? sv[2 * b + (ks >> 1)] : (b0 ? sv[2 + (ks >> 1)] : sv[ks >> 1]);
-                    static_for<0, FM>([&](auto bmc) {
-                        constexpr int bm = decltype(bmc)::value;
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[b][bm][r] = __builtin_fmaf(pp[b][bm][r], s, acc[b][bm][r]);
-                    });
-                });
-            }
+            rescale(std::integral_constant<int, (g + GROUPS - 1) % GROUPS>{}, sp);
+            sp = sraw[U][kb];
+            static_for<0, 4>([&](auto) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            });
+            __builtin_amdgcn_sched_barrier(0);
         });
-        __builtin_amdgcn_sched_barrier(0);
-        wait_vmcnt<WLOADS>();
+        // A(t + 2) landed: W(t + 2) and step t + 3's loads may fly.
+        wait_vmcnt<A_PER_WAVE + 2 * WLOADS>();
         step_barrier();
     };
     int t = 0;
-    for (; t + 1 < KT; t += 2) {
-        step(t, I0{});
-        step(t + 1, I1{});
-    }
-    if (t < KT) step(t, I0{});
-
-    const bool has_bias = p.bias != nullptr;
-    const int n_out = GLU ? p.glu_half : p.N;
-    float bias[NB];
-    static_for<0, NB>([&](auto bc) {
-        const int b = b0 + decltype(bc)::value;
-        const int oc = GLU ? slab * 32 + (lane & 31) : slab * 64 + 32 * b + (lane & 31);
-        const int col = GLU ? min(oc, n_out - 1) + b * p.glu_half : min(oc, n_out - 1);
-        bias[decltype(bc)::value] = has_bias ? p.bias[col] : 0.0f;
+    for (; t + NAS <= KT; t += NAS) static_for<0, NAS>([&](auto uc) { step(t + decltype(uc)::value, uc); });
+    static_for<0, NAS - 1>([&](auto uc) {
+        if (t + decltype(uc)::value < KT) step(t + decltype(uc)::value, uc);
     });
+    rescale(std::integral_constant<int, GROUPS - 1>{}, sp);
     wait_vmcnt<0>();
-    step_barrier();
+    __syncthreads();
 
-    uint8_t *region = lds + wave * REGION;
-    if constexpr (NB == 2) {
-        static_for<0, FM>([&](auto bmc) {
-            constexpr int bm = decltype(bmc)::value;
-            static_for<0, GLU ? 1 : 2>([&](auto bc) {
-                constexpr int b = decltype(bc)::value;
-                const int col0 = GLU ? slab * 32 : slab * 64 + 32 * b;
-                if (col0 < n_out)
-                    store_block_t<EPI, OUT>(p, acc[b][bm], bias[b], acc[GLU ? 1 : b][bm], bias[GLU ? 1 : b], col0,
-                                            m0 + 32 * bm, n_out, region, lane);
-            });
-        });
-    } else {
-        static_assert(!GLU, "a GLU pair needs both blocks of the slab in one wave");
-        const int col0 = slab * 64 + 32 * b0;
-        static_for<0, FM>([&](auto bmc) {
-            constexpr int bm = decltype(bmc)::value;
-            if (col0 < n_out)
-                store_block_t<EPI, OUT>(p, acc[0][bm], bias[0], acc[0][bm], bias[0], col0, m0 + 32 * bm, n_out, region,
-                                        lane);
-        });
+    // ---- epilogue: 32 rows at a time through LDS, then four columns a thread, whole rows of the tile ----------
+    // A thread's column (and so its bias) is the same for every row block.
+    const int n_out = glu ? p.glu_half : p.N;
+    const int cols = (glu ? 16 : 32) * NW, per_row = cols / 4;
+    const int chunk = tid % per_row;
+    const int col = tn * cols + 4 * chunk, blk = chunk >> 3;   // blk: the 32-column output block
+    const bool has_bias = p.bias != nullptr;
+    float bi[4], bu[4];
+    if (col < n_out) {
+        grp::column4(p.bias, true, p.sb_vec, col, n_out, 0, bi);
+        if (glu) grp::column4(p.bias, true, p.sb_vec, col, n_out, p.glu_half, bu);
     }
+    static_for<0, FM>([&](auto bmc) {
+        constexpr int bm = decltype(bmc)::value;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)  // row 8·(r >> 2) + 4h + (r & 3), column lane & 31 of the wave's block
+            *reinterpret_cast<float *>(lds + wave * grp::SLOT + (8 * (r >> 2) + 4 * h + (r & 3)) * grp::PITCH + (lane & 31) * 4) =
+                acc[bm][r];
+        __syncthreads();
+        if (col < n_out) {
+            const uint8_t *src = lds + (glu ? 2 * blk : blk) * grp::SLOT + (chunk & 7) * 16;
+            for (int row = tid / per_row; row < 32; row += 64 * NW / per_row) {
+                const int m = m0 + 32 * bm + row;
+                if (m >= p.M) break;
+                const f32x4 x = *reinterpret_cast<const f32x4 *>(src + row * grp::PITCH);
+                float v[4], u[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = has_bias ? __fadd_rn(x[e], bi[e]) : x[e];
+                if (glu) {
+                    const f32x4 y = *reinterpret_cast<const f32x4 *>(src + grp::SLOT + row * grp::PITCH);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) u[e] = has_bias ? __fadd_rn(y[e], bu[e]) : y[e];
+                }
+                grp::activate4(p.epi, v, u);
+                grp::store4(p, m, col, n_out, v);
+            }
+        }
+        if constexpr (bm + 1 < FM) __syncthreads();
+    });
 }
 
-template <int BM, int NW, int OCC, int NB, int WT, int EPI, int OUT>
-hipError_t launch_blocks_product(const GemmArgs &args, hipStream_t stream) {
-    constexpr bool GLU = EPI == EPI_SILU_GLU || EPI == EPI_SITU_GLU;
+template <int BM, int NW>
+hipError_t launch_blocks_product(const GemmArgs &args, int epi, int out, hipStream_t stream) {
     GemmArgs p = args;
+    p.epi = epi;
+    p.out = out;
     p.tiles_m = (p.M + BM - 1) / BM;
-    const int slabs = GLU ? (p.glu_half + 31) / 32 : (p.N + 63) / 64;
-    constexpr int SLABS_PER_WG = NB == 2 ? NW : NW / 2;
-    p.tiles_n = (slabs + SLABS_PER_WG - 1) / SLABS_PER_WG;
+    const int slabs = p.glu_half > 0 ? (p.glu_half + 31) / 32 : (p.N + 63) / 64;
+    p.tiles_n = (slabs + NW / 2 - 1) / (NW / 2);
     const int blocks = p.tiles_m * p.tiles_n;
     if (blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL((gemm_blocks_kernel<BM, NW, OCC, NB, WT, EPI, OUT>), dim3(blocks), dim3(64 * NW), 0, stream, p);
+    hipLaunchKernelGGL((gemm_blocks_kernel<BM, NW>), dim3(blocks), dim3(64 * NW), 0, stream, p);
     return hipGetLastError();
 }
 

@@ -116,14 +116,19 @@ hipError_t launch_pack(const uint8_t *w, int wl, int64_t ldw, int k, int n, bool
 
 // Codes with a scale per block of rows and column (GGUF Q8_0; sq8_blocks.hip): the packed Q8 layout
 // (codes in block-aligned K order, then fp32 scales per step and column) and its product, int8
-// codes, K a multiple of 64, A aligned for 16-byte loads. `tile`: BL_64x256 (two workgroups per CU),
-// BL_64x512 (one), BL_128x256 / BL_128x128 (eight waves of one 32-column block each, one or two
-// workgroups per CU; not for GLU epilogues, which then take BL_64x256). Scales [K/B, N] for W_KN codes, [N, K/B] for W_NK; B a multiple of 32
-// dividing K; scale dtype numbered as the C ABI's (fp32, bf16, fp16).
-enum BlocksTile { BL_64x256 = 0, BL_64x512 = 1, BL_128x256 = 2, BL_128x128 = 3 };
+// codes, K a multiple of 64, A aligned for 16-byte loads. `tile`: choose_blocks_tile's: BL_128x256 (eight waves of one
+// 32-column block each, one workgroup per CU), BL_128x128 (four, two per CU), or BLOCKS16_ROWS + rows (below). Scales
+// [K/B, N] for W_KN codes, [N, K/B] for W_NK; B a multiple of 32 dividing K; scale dtype numbered as the C ABI's
+// (fp32, bf16, fp16).
+enum BlocksTile { BL_128x256 = 0, BL_128x128 = 1 };
 int64_t packed_blocks_bytes(int k, int n, bool glu);
 hipError_t launch_pack_blocks(const uint8_t *w, int wl, int64_t ldw, const void *scale, int scale_dtype, int block,
                               int k, int n, bool glu, uint8_t *out, hipStream_t stream);
+// Tiles of BLOCKS16_ROWS + rows: the narrow-wave kernel (sq8_blocks16_kernel.h: 16, 32, 48, 64 or 80 rows × 64
+// columns, waves of 16 columns).
+constexpr int BLOCKS16_ROWS = 100;
+int choose_blocks_tile(int M, int N, bool glu, int cus, int kt);
+hipError_t launch_blocks16(const GemmArgs &p, int rows, int epi, int out, hipStream_t stream);
 hipError_t launch_blocks_product(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 
 // Auxiliary kernels (sq8_aux.hip).

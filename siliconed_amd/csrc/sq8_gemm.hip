@@ -2,6 +2,8 @@
 // allow them (sq8_gemm_inst.hip), the guarded ones otherwise (sq8_gemm_general.hip).
 #include "sq8_gemm.h"
 
+#include <math.h>
+
 namespace sq8 {
 
 hipError_t launch_fast_0_0(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
@@ -153,6 +155,34 @@ int choose_i8_tile(int M, int N, bool glu, int cus, int kt) {
         if (us < best) {
             best = us;
             tile = GROUP_TILE0 + i;
+        }
+    }
+    return tile;
+}
+
+int choose_blocks_tile(int M, int N, bool glu, int cus, int kt) {
+    // Every tile gives the same bits (each sum in K order), so only time decides: the least estimate of a workgroup's
+    // chain of K steps (µs a step, one workgroup a CU) against the CU's throughput (µs a step and workgroup), both
+    // measured at K = 3072 on full and nearly empty chips. Narrow waves (16 … 80 rows × 64 columns) where the wide
+    // kernel's tiles are few; measured against it (old → rule, µs, K = 3072): 77 × 12288 54 → 22, 512 × 3072 54 → 25,
+    // 16 × 128 (K = 2816) 48 → 11; K = 9728, 148 × 960 152 → 31. Wide: 128 × 128, two workgroups a CU (1021 × 3072
+    // 54.9 → 40.3, 333 × 9216 55 → 39.6), and 128 × 256 from four rounds of them on (GELU, 4096 × 12288 385 against
+    // 396: one activation tile for twice the columns; level at two rounds).
+    if (cus <= 0) cus = 256;
+    const float steps = (float)kt;
+    const long slabs = glu ? ((long)N / 2 + 31) / 32 : ((long)N + 63) / 64;
+    auto a_cu = [&](int rows, long per) { return (float)(((long)((M + rows - 1) / rows) * ((slabs + per - 1) / per) + cus - 1) / cus); };
+    struct Narrow { int rows; float chain, work; };
+    static const Narrow narrow[] = {{16, 0.175f, 0.13f}, {32, 0.208f, 0.15f}, {48, 0.26f, 0.195f}, {64, 0.3125f, 0.238f},
+                                    {80, 0.375f, 0.294f}};
+    if (a_cu(128, 4) >= 4.0f) return BL_128x256;
+    float best = fmaxf(6.0f + 0.66f * steps, 4.0f + a_cu(128, 2) * 0.655f * steps);
+    int tile = BL_128x128;
+    for (const Narrow &w : narrow) {
+        const float us = steps * fmaxf(w.chain, a_cu(w.rows, 1) * w.work);
+        if (us < best) {
+            best = us;
+            tile = BLOCKS16_ROWS + w.rows;
         }
     }
     return tile;

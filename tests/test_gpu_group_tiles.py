@@ -53,3 +53,58 @@ def test_w8a8_group_tile_same_bits(tile_gemm, tile):
         g.product_w8a8_residual(x, codes, sx, w, s, bias=b, gate=gate)
     torch.cuda.synchronize()
     assert torch.equal(*streams)
+
+
+Q8_TILES = {"16": (16, 64), "32": (32, 64), "48": (48, 64), "64": (64, 64), "80": (80, 64), "128x128": (128, 128),
+            "128x256": (128, 256)}
+
+
+@pytest.fixture(scope="module")
+def q8_gemm(gemm):
+    """Block-scale contexts on a forced tile (SQ8_Q8_TILE)."""
+    import os
+    import siliconed_amd as sq
+    made = {}
+    for name in Q8_TILES:
+        os.environ["SQ8_Q8_TILE"] = name
+        try:
+            made[name] = sq.TensorGEMM.make(0)
+        finally:
+            del os.environ["SQ8_Q8_TILE"]
+    return made
+
+
+@pytest.mark.parametrize("tile", Q8_TILES)
+def test_q8_tile_sums_in_k_order(gemm, q8_gemm, tile):
+    """Block scales at every tile's edges (one row, a row and a column past the tile; one K step, counts that leave each
+    remainder of the kernels' unrolled steps; a K of 32·odd), plain and GLU, bf16 and fp32 out, the rounded and the fp32
+    route. Integer activations make each block's sum exact, so acc = fl(P·d + acc) per block in K order, then the bias,
+    is the whole arithmetic: restated in float64 (which holds P·d + acc exactly), bit for bit on fp32 outputs; the
+    activations' outputs bit for bit against the 16-row tile's."""
+    bm, bn = Q8_TILES[tile]
+    ctx = q8_gemm[tile]
+    for m, k, n, epi, out, exact in [
+            (1, 64, 8, None, torch.float32, False), (bm + 1, 320, bn + 4, None, torch.float32, False),
+            (bm, 96, bn + 1, None, torch.float32, False), (2 * bm - 1, 704, bn, None, torch.float32, False),
+            (bm - 1, 576, 130, None, torch.float32, True), (bm + 3, 448, 2 * (bn // 2 + 5), "silu_glu", torch.bfloat16, False),
+            (bm + 2, 1024, 2 * bn, "situ_glu", torch.float32, False), (bm + 5, 832, bn + 2, "gelu_tanh", torch.bfloat16, False)]:
+        print(f"q8 tile {tile}: {m} x {k} x {n} {epi} {out} {'fp32 route' if exact else ''}", flush=True)
+        g = torch.Generator(device=DEV).manual_seed(m + k + n)
+        x = torch.randint(-5, 6, (m, k), device=DEV, generator=g).float()
+        q = torch.randint(-127, 128, (n, k), device=DEV, generator=g, dtype=torch.int8)
+        d = (torch.rand((n, k // 32), device=DEV, generator=g) * 0.02 + 1e-3).half()
+        b = torch.randn(n, device=DEV, generator=g)
+        w = ctx.pack_blocks(q, d, 32, layout="nk", glu=epi in ("silu_glu", "situ_glu"))
+        a = x if exact else x.bfloat16()
+        y = ctx.product_blocks(a, w, bias=b, epilogue=epi, out_dtype=out, rounding=not exact)
+        torch.cuda.synchronize()
+        if epi is None:
+            acc = torch.zeros((m, n), device=DEV)
+            for i in range(k // 32):
+                part = x[:, 32 * i:32 * i + 32].double() @ q[:, 32 * i:32 * i + 32].double().t()
+                acc = (part * d[:, i].double() + acc.double()).float()
+            assert torch.equal(y, acc + b)
+        else:
+            z = q8_gemm["16"].product_blocks(a, w, bias=b, epilogue=epi, out_dtype=out, rounding=not exact)
+            torch.cuda.synchronize()
+            assert torch.equal(y, z)
