@@ -18,23 +18,35 @@ CSRC = os.path.join(PKG, "csrc")
 OBJ = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libsiliconed_q8.so")
 # (source, object name, extra defines): the FAST kernel set is one source compiled per weight type
-# and layout, so the sets compile in parallel.
+# and layout, so the sets compile in parallel, the longest first.
 SOURCES = [
+    ("sq8_wdirect_inst.hip", "sq8_wdirect_i8_nk", ["-DSQ8_WT=0", "-DSQ8_WL=1"]),
+    ("sq8_wdirect_inst.hip", "sq8_wdirect_i8_packed", ["-DSQ8_WT=0", "-DSQ8_WL=2"]),
+    ("sq8_wdirect_inst.hip", "sq8_wdirect_f8_nk", ["-DSQ8_WT=1", "-DSQ8_WL=1"]),
+    ("sq8_wdirect_inst.hip", "sq8_wdirect_f8_packed", ["-DSQ8_WT=1", "-DSQ8_WL=2"]),
+    ("sq8_short_inst.hip", "sq8_short_i8_nk", ["-DSQ8_WT=0", "-DSQ8_WL=1"]),
+    ("sq8_short_inst.hip", "sq8_short_i8_packed", ["-DSQ8_WT=0", "-DSQ8_WL=2"]),
+    ("sq8_short_inst.hip", "sq8_short_f8_nk", ["-DSQ8_WT=1", "-DSQ8_WL=1"]),
+    ("sq8_short_inst.hip", "sq8_short_f8_packed", ["-DSQ8_WT=1", "-DSQ8_WL=2"]),
     ("sq8_gemm.hip", "sq8_gemm", []),
     ("sq8_gemm_general.hip", "sq8_gemm_general", []),
     ("sq8_gemm_inst.hip", "sq8_gemm_i8_kn", ["-DSQ8_WT=0", "-DSQ8_WL=0"]),
     ("sq8_gemm_inst.hip", "sq8_gemm_i8_nk", ["-DSQ8_WT=0", "-DSQ8_WL=1"]),
     ("sq8_gemm_inst.hip", "sq8_gemm_f8_kn", ["-DSQ8_WT=1", "-DSQ8_WL=0"]),
     ("sq8_gemm_inst.hip", "sq8_gemm_f8_nk", ["-DSQ8_WT=1", "-DSQ8_WL=1"]),
-    ("sq8_wdirect_inst.hip", "sq8_wdirect_i8_nk", ["-DSQ8_WT=0", "-DSQ8_WL=1"]),
-    ("sq8_wdirect_inst.hip", "sq8_wdirect_i8_packed", ["-DSQ8_WT=0", "-DSQ8_WL=2"]),
-    ("sq8_wdirect_inst.hip", "sq8_wdirect_f8_nk", ["-DSQ8_WT=1", "-DSQ8_WL=1"]),
-    ("sq8_wdirect_inst.hip", "sq8_wdirect_f8_packed", ["-DSQ8_WT=1", "-DSQ8_WL=2"]),
     ("sq8_aux.hip", "sq8_aux", []),
     ("sq8_block.hip", "sq8_block", []),
     ("sq8_convrot.hip", "sq8_convrot", []),
     ("sq8_w8a8.hip", "sq8_w8a8", []),
     ("sq8_i8_inst.hip", "sq8_i8_inst", []),
+    ("sq8_group_inst.hip", "sq8_group_bf16_i8_nk", ["-DSQ8_MATH=0", "-DSQ8_WT=0", "-DSQ8_WL=1"]),
+    ("sq8_group_inst.hip", "sq8_group_bf16_i8_packed", ["-DSQ8_MATH=0", "-DSQ8_WT=0", "-DSQ8_WL=2"]),
+    ("sq8_group_inst.hip", "sq8_group_bf16_f8_nk", ["-DSQ8_MATH=0", "-DSQ8_WT=1", "-DSQ8_WL=1"]),
+    ("sq8_group_inst.hip", "sq8_group_bf16_f8_packed", ["-DSQ8_MATH=0", "-DSQ8_WT=1", "-DSQ8_WL=2"]),
+    ("sq8_group_inst.hip", "sq8_group_f32_i8_nk", ["-DSQ8_MATH=2", "-DSQ8_WT=0", "-DSQ8_WL=1"]),
+    ("sq8_group_inst.hip", "sq8_group_f32_i8_packed", ["-DSQ8_MATH=2", "-DSQ8_WT=0", "-DSQ8_WL=2"]),
+    ("sq8_group_inst.hip", "sq8_group_f32_f8_nk", ["-DSQ8_MATH=2", "-DSQ8_WT=1", "-DSQ8_WL=1"]),
+    ("sq8_group_inst.hip", "sq8_group_f32_f8_packed", ["-DSQ8_MATH=2", "-DSQ8_WT=1", "-DSQ8_WL=2"]),
     ("sq8_group_inst.hip", "sq8_group_i8_nk", ["-DSQ8_MATH=1", "-DSQ8_WT=0", "-DSQ8_WL=1"]),
     ("sq8_group_inst.hip", "sq8_group_i8_packed", ["-DSQ8_MATH=1", "-DSQ8_WT=0", "-DSQ8_WL=2"]),
     ("sq8_blocks.hip", "sq8_blocks", []),
@@ -88,7 +100,7 @@ def build(verbose: bool = False, incremental: bool = False) -> str:
     unless `incremental` (then only those whose object is older than the source or a header)."""
     os.makedirs(OBJ, exist_ok=True)
     todo = [it for it in SOURCES if _stale(it)] if incremental else SOURCES
-    with concurrent.futures.ThreadPoolExecutor(max_workers=max(len(todo), 1)) as pool:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=max(1, min(len(todo), os.cpu_count() or 1))) as pool:
         list(pool.map(_compile, todo))
     objs = [os.path.join(OBJ, name + ".o") for _, name, _ in SOURCES]
     tmp = LIB + ".tmp"

@@ -101,6 +101,26 @@ int group_knob(const char *value, int other) {
     return other;
 }
 
+// True when K-group tile `tile` is built for products of kind `math` (a GLU pair takes an even number of blocks).
+bool group_serves(int tile, int math, bool glu) {
+    const sq8::GroupShape &g = sq8::group_shapes[tile - sq8::GROUP_TILE0];
+    return g.cost[math].us_step > 0.0f && !(glu && g.cols % 64 != 0);
+}
+
+// The knobs "k32x32" … "k64x192": the K-group tile of that shape where K/64 divides among its groups, else the tile of
+// the same height without groups (GLU: a tile of an even number of 32-column blocks, of as many groups).
+constexpr int KNOB_K = 1000;
+int wd_knob_tile(int knob, bool glu, int steps, bool f32) {
+    if (knob < sq8::GROUP_TILE0) return knob;
+    if (knob < KNOB_K) return group_serves(knob, f32 ? sq8::GM_F32 : sq8::GM_BF16, glu) ? knob : sq8::WD_128;
+    static const struct { const char *group; int groups, plain, glu; } of[] = {
+        {"g32x32k4", 4, sq8::WD_32, sq8::WD_32}, {"g32x64k4", 4, sq8::WD_32, sq8::WD_32}, {"g64x64k4", 4, sq8::WD_64N, sq8::WD_32},
+        {"g64x128k2", 2, sq8::WD_64N, sq8::WD_32}, {"g64x192k2", 2, sq8::WD_64x192, sq8::WD_64}};
+    const auto &k = of[knob - KNOB_K];
+    if (steps % k.groups != 0) return glu ? k.glu : k.plain;
+    return group_knob(glu && knob == KNOB_K ? "g32x64k4" : k.group, sq8::WD_128);
+}
+
 bool is_glu(int epilogue) { return epilogue == SQ8_EPI_SILU_GLU || epilogue == SQ8_EPI_SITU_GLU; }
 
 bool is_packed(int w_layout) { return w_layout == SQ8_PACKED || w_layout == SQ8_PACKED_GLU; }
@@ -362,7 +382,10 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
         // The weight-direct kernels: packed codes, or [N, K] rows read as they lie.
         if (!p.a_vec || !k_steps) return SQ8_EUNSUPPORTED;  // K = 0, or an activation not 16-byte aligned
         const int wl = is_packed(wl_run) ? sq8::W_PACKED : sq8::W_NK;
-        const int tile = ctx->wd_tile >= 0 ? ctx->wd_tile : sq8::choose_wd_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, p.kt);
+        const int steps = q.exact ? p.kt_w : p.kt;
+        const int tile = ctx->wd_tile >= 0 ? wd_knob_tile(ctx->wd_tile, is_glu(q.epilogue), steps, q.exact)
+                                           : sq8::choose_wd_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, steps, q.exact,
+                                                                 sq8::w256_fits(p, epi, out));
         if ((tile == sq8::WD_SKINNY32 || tile == sq8::WD_SKINNY64) && ctx->splits > 1) {
             // Short M with the SQ8_SPLITS knob: the K steps split over several workgroups per tile, partial
             // sums in the context's buffer, added in split order by a second launch. Not the default: the
@@ -533,9 +556,7 @@ int run_w8a8(sq8_ctx *ctx, const W8A8 &q, double *gpu_seconds) {
         p.kt_w = (q.k + 63) / 64;
     }
     int tile = ctx->i8_tile >= 0 ? ctx->i8_tile : sq8::choose_i8_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, p.kt);
-    // A forced tile of an odd number of 32-column blocks cannot hold a GLU pair.
-    if (is_glu(q.epilogue) && tile >= sq8::GROUP_TILE0 && sq8::group_shapes[tile - sq8::GROUP_TILE0].cols % 64 != 0)
-        tile = sq8::I8_128x256;
+    if (tile >= sq8::GROUP_TILE0 && !group_serves(tile, sq8::GM_I8, is_glu(q.epilogue))) tile = sq8::I8_128x256;
     e = sq8::launch_i8gemm(p, tile, wl, q.residual ? sq8::EPI_RESIDUAL : q.epilogue,
                            q.c_dtype == SQ8_F32 ? sq8::OUT_F32 : sq8::OUT_BF16, ctx->stream);
     if (e != hipSuccess) return hip_status(e);
@@ -789,10 +810,11 @@ int sq8_create(int device, void *stream, sq8_ctx **out) {
     ctx->device = device;
     ctx->stream = static_cast<hipStream_t>(stream);
     ctx->cus = prop.multiProcessorCount;
-    ctx->wd_tile = knob(getenv("SQ8_TILE"), {{"256", sq8::WD_256}, {"224", sq8::WD_224}, {"128", sq8::WD_128}, {"64", sq8::WD_64},
-                                             {"32", sq8::WD_32}, {"64n", sq8::WD_64N}, {"64x192", sq8::WD_64x192}, {"s64", sq8::WD_SKINNY64}, {"s32", sq8::WD_SKINNY32},
-                                             {"gemv", sq8::WD_GEMV}, {"k32x32", sq8::WD_K32x32}, {"k32x64", sq8::WD_K32x64},
-                                             {"k64x64", sq8::WD_K64x64}, {"k64x128", sq8::WD_K64x128}, {"k64x192", sq8::WD_K64x192}});
+    ctx->wd_tile = group_knob(getenv("SQ8_TILE"), knob(getenv("SQ8_TILE"), {
+        {"256", sq8::WD_256}, {"224", sq8::WD_224}, {"128", sq8::WD_128}, {"64", sq8::WD_64}, {"32", sq8::WD_32},
+        {"64n", sq8::WD_64N}, {"64x192", sq8::WD_64x192}, {"s64", sq8::WD_SKINNY64}, {"s32", sq8::WD_SKINNY32},
+        {"gemv", sq8::WD_GEMV}, {"k32x32", KNOB_K + 0}, {"k32x64", KNOB_K + 1}, {"k64x64", KNOB_K + 2},
+        {"k64x128", KNOB_K + 3}, {"k64x192", KNOB_K + 4}}));
     ctx->i8_tile = group_knob(getenv("SQ8_TILE"), knob(getenv("SQ8_TILE"), {{"128", sq8::I8_128x256}}));
     ctx->q8_tile = knob(getenv("SQ8_Q8_TILE"), {{"128x256", sq8::BL_128x256}, {"128x128", sq8::BL_128x128},
                                                 {"16", sq8::BLOCKS16_ROWS + 16}, {"32", sq8::BLOCKS16_ROWS + 32},

@@ -120,22 +120,29 @@ gemm_blocks16_kernel(const GemmArgs p) {
         });
     };
 
-    // Prologue: the loads of the steps before the loop in its issue order — A(0), A(1), then A(s), W(s) pairs.
+    // Prologue: the loads of the steps before the loop in its issue order — A(0), A(1), then A(s), W(s) pairs
+    // (kept in it: the compiler would move the codes' loads past the others, and the waits count on the order).
+    __builtin_amdgcn_sched_barrier(0);
     issue_a(0, std::integral_constant<int, 0>{});
     issue_a(1, std::integral_constant<int, 1>{});
+    __builtin_amdgcn_sched_barrier(0);
     static_for<0, PF>([&](auto vc_) {
         constexpr int v = decltype(vc_)::value;
         // W(v) belongs to step v − PF, whose A is A(v − PF + NAS − 1).
         constexpr int a = v - PF + NAS - 1;
         if constexpr (a >= 2) issue_a(a, std::integral_constant<int, a>{});
+        __builtin_amdgcn_sched_barrier(0);
         issue_w(v, vc_);
+        __builtin_amdgcn_sched_barrier(0);
     });
     wait_vmcnt<STEP_WAIT>();
     step_barrier();
     read_x(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
 
-    // Step t: activation stage t mod NAS, code buffer t mod PF, fragments t mod 2.
-    auto step = [&](int t, auto uc) {
+    // Step t: activation stage t mod NAS, code buffer t mod PF, fragments t mod 2. TAIL: one of the last steps, whose code
+    // loads no later step uses and the compiler drops: the wait counts the activation's loads only.
+    auto step = [&](int t, auto uc, auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
         constexpr int U = decltype(uc)::value;
         constexpr int S = U % NAS, P = U % PF, D = U & 1;
         __builtin_amdgcn_sched_barrier(0);
@@ -164,17 +171,17 @@ gemm_blocks16_kernel(const GemmArgs p) {
         __builtin_amdgcn_sched_barrier(0);
         issue_w(t + PF, std::integral_constant<int, P>{});
         __builtin_amdgcn_sched_barrier(0);
-        wait_vmcnt<STEP_WAIT>();
+        wait_vmcnt<TAIL ? (NAS - 3) * A_PER_WAVE : STEP_WAIT>();
         step_barrier();
     };
     // The stages, buffers and fragment halves repeat every lcm(NAS, PF, 2) steps.
     constexpr int CYCLE = PF % NAS == 0 && PF % 2 == 0 ? PF : 2 * NAS * PF;
     static_assert(CYCLE <= 16, "unrolled steps");
     int t = 0;
-    for (; t + CYCLE <= KT; t += CYCLE) static_for<0, CYCLE>([&](auto uc) { step(t + decltype(uc)::value, uc); });
+    for (; t + CYCLE <= KT; t += CYCLE) static_for<0, CYCLE>([&](auto uc) { step(t + decltype(uc)::value, uc, std::false_type{}); });
     static_for<0, CYCLE - 1>([&](auto uc) {
         constexpr int u = decltype(uc)::value;
-        if (t + u < KT) step(t + u, uc);
+        if (t + u < KT) step(t + u, uc, std::true_type{});
     });
     wait_vmcnt<0>();
     __syncthreads();

@@ -180,8 +180,10 @@ gemm_blocks_kernel(const GemmArgs p) {
     widen(I0{}, I0{}, I0{});
     widen(I0{}, I0{}, I1{});
 
-    // Step t on stage and code buffer U = t mod 4.
-    auto step = [&](int t, auto uc) {
+    // Step t on stage and code buffer U = t mod 4. TAIL: one of the last steps, whose code loads no later step uses and the
+    // compiler drops: the wait counts the activation's loads only (as if every code load had been dropped).
+    auto step = [&](int t, auto uc, auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
         constexpr int U = decltype(uc)::value;
         using SU = std::integral_constant<int, U>;
         using S1 = std::integral_constant<int, (U + 1) % NAS>;
@@ -224,13 +226,13 @@ gemm_blocks_kernel(const GemmArgs p) {
             __builtin_amdgcn_sched_barrier(0);
         });
         // A(t + 2) landed: W(t + 2) and step t + 3's loads may fly.
-        wait_vmcnt<A_PER_WAVE + 2 * WLOADS>();
+        wait_vmcnt<A_PER_WAVE + (TAIL ? 0 : 2 * WLOADS)>();
         step_barrier();
     };
     int t = 0;
-    for (; t + NAS <= KT; t += NAS) static_for<0, NAS>([&](auto uc) { step(t + decltype(uc)::value, uc); });
+    for (; t + NAS <= KT; t += NAS) static_for<0, NAS>([&](auto uc) { step(t + decltype(uc)::value, uc, std::false_type{}); });
     static_for<0, NAS - 1>([&](auto uc) {
-        if (t + decltype(uc)::value < KT) step(t + decltype(uc)::value, uc);
+        if (t + decltype(uc)::value < KT) step(t + decltype(uc)::value, uc, std::true_type{});
     });
     rescale(std::integral_constant<int, GROUPS - 1>{}, sp);
     wait_vmcnt<0>();

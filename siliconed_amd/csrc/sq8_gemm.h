@@ -50,22 +50,29 @@ hipError_t launch_gemm(const GemmArgs &p, bool fast, int tile, int wt, int wl, i
 
 // The weight-direct kernels (sq8_wdirect_inst.hip): [N, K] or packed weights, K a multiple of 64,
 // A aligned for 16-byte loads. `tile`: WD_256 (256 × 256, one workgroup per CU), WD_224 (224 × 256, the
-// same kernel), WD_128 (128 × 256, two workgroups per CU), WD_64 (64 × 256, one per CU), WD_32 (32 × 256,
-// two per CU), WD_64N (64 × 128, a 32-column block a wave, two per CU; not GLU), WD_64x192 (64 × 192, six
-// waves of one 32-column block; not GLU), or the skinny-M kernel with 64- or 32-row tiles of one 64-column
-// slab and the K steps split over four waves (WD_SKINNY64, WD_SKINNY32), or M ≤ 64 in 16-column groups on
-// 16 × 16 MFMAs, every K step's loads issued far ahead (WD_GEMV), or tiles of one-block waves whose K steps
-// split over two or four wave groups (WD_K32x32, WD_K32x64, WD_K64x64: four groups; WD_K64x128, WD_K64x192:
-// two; not GLU, K/64 a multiple of the groups).
+// same kernel), WD_128 (128 × 256, two workgroups per CU), WD_GEMV (M ≤ 16 in 16-column groups on 16 × 16 MFMAs, every
+// K step's loads issued far ahead), the skinny-M kernel with 64- or 32-row tiles of one 64-column slab and the K steps
+// split over four waves (WD_SKINNY64, WD_SKINNY32), or a K-group tile's id (below). By the SQ8_TILE knob only: WD_64
+// (64 × 256, one per CU), WD_32 (32 × 256, two per CU), WD_64N (64 × 128, a 32-column block a wave, two per CU; not
+// GLU), WD_64x192 (64 × 192, six waves of one 32-column block; not GLU): the K-group tiles' shapes without groups, in
+// WD_128's order of sums.
 enum WdTile { WD_256 = 0, WD_128 = 1, WD_SKINNY64 = 2, WD_SKINNY32 = 3, WD_64 = 4, WD_32 = 5, WD_224 = 6, WD_64N = 7, WD_64x192 = 8,
-              WD_GEMV = 9, WD_K32x32 = 10, WD_K32x64 = 11, WD_K64x64 = 12, WD_K64x128 = 13, WD_K64x192 = 14 };
-// The tile for an M × N product (GLU: N = 2h): 256 or 224 rows × 256 while those tiles occupy more than
-// half the 256 CUs (the height whose rounds of 256 tiles cover the fewest rows; launch_wdirect takes
-// 128-row tiles where that kernel cannot serve the product), else the tallest of 128, 64 and 32 rows
-// whose tiles number at least 144 (enough to occupy the 256 CUs), else the skinny kernel; below the 128-row
-// tiles the K-group tiles where one fits a round (up to 16 rows only where the short-M kernel would read the
-// activation from global memory). `kt`: the product's K steps of 64.
-int choose_wd_tile(int M, int N, bool glu, int cus, int kt);
+              WD_GEMV = 9 };
+// The tile for an M × N product (GLU: N = 2h) of `steps` weight K steps of 64, `f32` on the fp32 route (three parts of
+// an fp32 activation), `w256`: the 256-row kernel serves it (w256_fits).
+int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32, bool w256);
+// True when the 256- and 224-row kernel runs this product: whole 64-column slabs (GLU: whole 32-column
+// slabs of each half) and 16-byte scale/bias loads; for the slab epilogue (bf16 out, no activation or
+// GELU) also slabs that each lie in one output (and one head) and 16-byte stores. The fp32 route's three
+// parts along K (kt_w > 0) face the weight's steps in turn (weight_step).
+inline bool w256_fits(const GemmArgs &p, int epi, int out) {
+    if (!p.sb_vec) return false;
+    if (p.glu_half > 0 ? p.glu_half % 32 != 0 : p.N % 64 != 0) return false;
+    if (epi == EPI_RESIDUAL && out != OUT_F32) return false;
+    if ((epi == EPI_NONE || epi == EPI_GELU) && out == OUT_BF16)
+        return p.split % 64 == 0 && p.head_dim % 64 == 0 && p.c_vec16;
+    return true;
+}
 // The short-M kernel (sq8_gemv_kernel.h): the activation staged in LDS (M rows of K' = kt · 64 bf16, rows
 // gemv_xpitch bytes apart: 16 more than a row, so the 16 rows a fragment read touches start on different banks)
 // when it fits GEMV_XLDS bytes and each row is whole 1 KB runs (K' a multiple of 512), the unit of a direct load.
@@ -80,29 +87,37 @@ hipError_t launch_wdirect(const GemmArgs &p, int tile, int wt, int wl, int epi, 
 
 // The K-group kernels (sq8_group_kernel.h): `rows` × `cols` tiles (cols: weight columns) whose K steps split over
 // `groups` wave groups; GLU products take those of an even number of 32-column blocks. What a round of tiles on
-// the CUs, one a CU, takes on W8A8 operands: us + us_step · (K steps of 128) microseconds, fitted to 256 and 512
-// tiles at K = 1024, 3072 and 8192 (graph launches, the launch's own 2.5 µs taken off).
+// the CUs, one a CU, takes by kind of product: us + us_step · (weight K steps) microseconds, fitted to 256 and 512
+// tiles at K = 1024, 3072 and 8192 (graph launches, the launch's own 2.5 µs taken off); us_step 0: not built for it.
+enum GroupMath { GM_BF16 = 0, GM_I8 = 1, GM_F32 = 2 };
+struct GroupCost {
+    float us, us_step;
+};
 struct GroupShape {
     int rows, cols, groups;
-    float us, us_step;
-    const char *name;  // the SQ8_TILE knob's name for it
+    const char *name;   // the SQ8_TILE knob's name for it
+    GroupCost cost[3];  // by GroupMath
 };
 constexpr int GROUP_TILE0 = 100;  // tile ids of the K-group kernels: GROUP_TILE0 + index into group_shapes
 constexpr GroupShape group_shapes[] = {
-    {32, 32, 8, 0.65f, 0.104f, "g32x32k8"},
-    {32, 64, 8, 0.55f, 0.165f, "g32x64k8"},
-    {64, 64, 4, 1.60f, 0.204f, "g64x64k4"},
-    {64, 96, 4, 2.65f, 0.243f, "g64x96k4"},
-    {64, 128, 4, 2.30f, 0.325f, "g64x128k4"},
-    {96, 96, 4, 3.60f, 0.312f, "g96x96k4"},
-    {96, 128, 4, 4.40f, 0.408f, "g96x128k4"},
-    {128, 96, 4, 4.70f, 0.402f, "g128x96k4"},
-    {128, 128, 2, 6.30f, 0.493f, "g128x128k2"},
-    {96, 192, 2, 6.30f, 0.560f, "g96x192k2"},
-    {128, 192, 2, 8.70f, 0.694f, "g128x192k2"},
+    {32, 32, 8, "g32x32k8", {{}, {0.65f, 0.104f}, {}}},
+    {32, 64, 8, "g32x64k8", {{}, {0.55f, 0.165f}, {}}},
+    {32, 32, 4, "g32x32k4", {{1.16f, 0.064f}, {}, {2.20f, 0.277f}}},
+    {32, 64, 4, "g32x64k4", {{1.74f, 0.089f}, {}, {2.11f, 0.352f}}},
+    {64, 64, 4, "g64x64k4", {{2.64f, 0.151f}, {1.60f, 0.204f}, {5.15f, 0.511f}}},
+    {64, 96, 4, "g64x96k4", {{3.42f, 0.212f}, {2.65f, 0.243f}, {6.26f, 0.620f}}},
+    {64, 128, 4, "g64x128k4", {{2.81f, 0.284f}, {2.30f, 0.325f}, {7.01f, 0.746f}}},
+    {64, 128, 2, "g64x128k2", {{2.56f, 0.290f}, {}, {6.77f, 0.752f}}},
+    {64, 192, 2, "g64x192k2", {{3.79f, 0.407f}, {}, {8.56f, 1.032f}}},
+    {96, 96, 4, "g96x96k4", {{3.88f, 0.299f}, {3.60f, 0.312f}, {9.95f, 0.822f}}},
+    {96, 128, 4, "g96x128k4", {{4.23f, 0.371f}, {4.40f, 0.408f}, {}}},
+    {128, 96, 4, "g128x96k4", {{4.59f, 0.382f}, {4.70f, 0.402f}, {}}},
+    {128, 128, 2, "g128x128k2", {{5.61f, 0.482f}, {6.30f, 0.493f}, {14.93f, 1.284f}}},
+    {96, 192, 2, "g96x192k2", {{6.10f, 0.520f}, {6.30f, 0.560f}, {11.95f, 1.425f}}},
+    {128, 192, 2, "g128x192k2", {{7.80f, 0.656f}, {8.70f, 0.694f}, {13.96f, 1.848f}}},
 };
 constexpr int kGroupShapes = (int)(sizeof(group_shapes) / sizeof(group_shapes[0]));
-hipError_t launch_group_i8(const GemmArgs &p, int shape, int wl, int epi, int out, hipStream_t stream);
+hipError_t launch_group(const GemmArgs &p, int math, int shape, int wt, int wl, int epi, int out, hipStream_t stream);
 
 // Bytes of the packed layout of a weight with k rows of K and n columns (GLU: n = 2h, packed in
 // pairs of 32-column blocks of the two halves).

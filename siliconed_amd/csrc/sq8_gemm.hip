@@ -11,124 +11,136 @@ hipError_t launch_fast_0_1(const GemmArgs &p, int tile, int epi, int out, hipStr
 hipError_t launch_fast_1_0(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 hipError_t launch_fast_1_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 hipError_t launch_general(const GemmArgs &p, int wt, int wl, int epi, int out, hipStream_t stream);
+hipError_t launch_short_0_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
+hipError_t launch_short_0_2(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
+hipError_t launch_short_1_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
+hipError_t launch_short_1_2(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 hipError_t launch_wdirect_0_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 hipError_t launch_wdirect_0_2(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 hipError_t launch_wdirect_1_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 hipError_t launch_wdirect_1_2(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 
 hipError_t launch_wdirect(const GemmArgs &p, int tile, int wt, int wl, int epi, int out, hipStream_t stream) {
-    if (wt == W_INT8) return wl == W_NK ? launch_wdirect_0_1(p, tile, epi, out, stream) : launch_wdirect_0_2(p, tile, epi, out, stream);
-    return wl == W_NK ? launch_wdirect_1_1(p, tile, epi, out, stream) : launch_wdirect_1_2(p, tile, epi, out, stream);
+    if (tile >= GROUP_TILE0)
+        return launch_group(p, p.kt_w > 0 ? GM_F32 : GM_BF16, tile - GROUP_TILE0, wt, wl, epi, out, stream);
+    const bool shorter = tile == WD_GEMV || tile == WD_SKINNY64 || tile == WD_SKINNY32;
+#define SQ8_CASE(T, L)                                                                                          \
+    if (wt == T && wl == L)                                                                                     \
+        return shorter ? launch_short_##T##_##L(p, tile, epi, out, stream) : launch_wdirect_##T##_##L(p, tile, epi, out, stream);
+    SQ8_CASE(0, 1)
+    SQ8_CASE(0, 2)
+    SQ8_CASE(1, 1)
+    SQ8_CASE(1, 2)
+#undef SQ8_CASE
+    return hipErrorInvalidValue;
 }
 
+hipError_t launch_group_0_0_1(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+hipError_t launch_group_0_0_2(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+hipError_t launch_group_0_1_1(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+hipError_t launch_group_0_1_2(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
 hipError_t launch_group_1_0_1(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
 hipError_t launch_group_1_0_2(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+hipError_t launch_group_2_0_1(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+hipError_t launch_group_2_0_2(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+hipError_t launch_group_2_1_1(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
+hipError_t launch_group_2_1_2(const GemmArgs &p, int shape, int epi, int out, hipStream_t stream);
 
-hipError_t launch_group_i8(const GemmArgs &p, int shape, int wl, int epi, int out, hipStream_t stream) {
-    return wl == W_NK ? launch_group_1_0_1(p, shape, epi, out, stream) : launch_group_1_0_2(p, shape, epi, out, stream);
+hipError_t launch_group(const GemmArgs &p, int math, int shape, int wt, int wl, int epi, int out, hipStream_t stream) {
+#define SQ8_CASE(M, T)                                                                                   \
+    if (math == M && wt == T)                                                                            \
+        return wl == W_NK ? launch_group_##M##_##T##_1(p, shape, epi, out, stream)                       \
+                          : launch_group_##M##_##T##_2(p, shape, epi, out, stream);
+    SQ8_CASE(0, 0)
+    SQ8_CASE(0, 1)
+    SQ8_CASE(1, 0)
+    SQ8_CASE(2, 0)
+    SQ8_CASE(2, 1)
+#undef SQ8_CASE
+    return hipErrorInvalidValue;
 }
 
-// The tile before the K-group tiles are considered.
-static int base_wd_tile(int M, int N, bool glu, int cus) {
-    // Tiles of 256 columns (four 64-column slabs; GLU: 32 output columns a slab), as tall as keeps
-    // at least 9/16 of the CUs' worth of them (144 on the 256 CUs of a whole MI355X) — the measured point
-    // below which a shorter tile fills the CUs better than the taller one loses (K = 3072: M = 1024 at
-    // N = 3072 runs 64-row tiles at one workgroup a CU in 28.5 µs against 42.8 in 128-row tiles; M = 512
-    // 32-row tiles in 22.7 against 42.9). Below that in 32-row tiles, the skinny kernel (K split over four
-    // waves): 32-row tiles to M = 128, 64-row above (M = 16: 8.3 µs against 20.2 for 32-row tiles of the
-    // main kernel); up to 16 rows on narrow weights, the short-M kernel. `cus`: the device's compute units (a compute-partitioned MI355X has fewer than 256),
-    // so a round is `cus` tiles of one workgroup a CU.
-    if (cus <= 0) cus = 256;
-    const long slabs = glu ? (N / 2 + 31) / 32 : (N + 63) / 64;
-    const long tn = (slabs + 3) / 4;
-    const long fill = (long)cus * 9 / 16;
-    auto tiles = [&](int bm) { return (long)((M + bm - 1) / bm) * tn; };
-    // 256 × 256 tiles (one workgroup a CU) once they occupy more than half the CUs: C1's
-    // up-projection, 768 tiles, 243.6 µs against 265.1 in 128-row tiles (one process, medians); C3's fp8
-    // gate-up (SiLU-GLU, 1280 tiles) 1353 against 1290 TFLOP/s; C1's down-projection, 192 tiles (one
-    // partial round), 1208–1228 against 1105. With fewer, the 128-row tiles spread over more CUs.
-    if (tiles(256) > cus / 2) {
-        // 224-row tiles where their rounds on the CUs cover fewer rows than the 256-row tiles' (the
-        // same work per row, one workgroup a CU): C1's down-projection (M = 4096, N = 3072) 228 tiles in
-        // one round against 192 in one; C4's and C2's fused QKV (M = 4608, N = 9216) 756 tiles in three
-        // rounds against 648 in three; never C1's up-projection (768 tiles, three full rounds).
-        auto rows = [&](int bm) { return (tiles(bm) + cus - 1) / cus * bm; };
-        return rows(224) < rows(256) ? WD_224 : WD_256;
-    }
-    if (tiles(128) >= fill) return WD_128;
-    if (tiles(64) >= fill) {
-        // 64 × 192 tiles of six one-block waves while they fit one round on the CUs (and not for the GLU
-        // epilogues): less activation and weight per workgroup for the same rows. Measured against the 64-row
-        // tiles at K = 3072 in one process: C0 (1024 × 3072) 29.7 against 30.9 µs, and 3–5 % faster on five
-        // other shapes of one round (768 × 3072, 192 and 256 × 12288, 256 × 9216); past one round (1280 × 3072,
-        // 384 × 9216) 1.6× slower, so not there.
-        const long tiles64x192 = (long)((M + 63) / 64) * ((N + 191) / 192);
-        return !glu && tiles64x192 <= cus ? WD_64x192 : WD_64;
-    }
-    if (tiles(32) >= fill) {
-        // 64 × 128 tiles, a 32-column block a wave (half the codes widened per MFMA), where they add no tiles
-        // to the 32-row ones (a ragged last row tile would): measured over 15 shapes at K = 3072 in one
-        // process, C2's text stream (512 × 3072) 20.5 against 23.3 µs, the shapes whose 32-row tiles number
-        // more than 256 (704 × 3072, 256 × 9216, 384 × 6144, 512 × 4608) 27.4–27.9 against 34.4–35.1 µs, the
-        // others within 0–5 % slower; not for the GLU epilogues.
-        const long tiles64n = (long)((M + 63) / 64) * ((N + 127) / 128);
-        return !glu && tiles64n <= tiles(32) ? WD_64N : WD_32;
-    }
-    // Up to 16 rows, the 16-column groups of the short-M kernel where they fit one round on the CUs (N ≤ 4096
-    // on 256 CUs; GLU: 2048 output columns): every K step's loads in flight, the activation read once per
-    // workgroup. Kernel traces at K = 3072, N = 3072 (int8 packed, bias): M = 1 4.10 µs against the skinny
-    // kernel's 7.44, M = 16 5.95 against 8.73; K = 12288, N = 3072: M = 1 10.1 against 19.4. Past one round
-    // (N = 9216, 12288) the skinny kernel's 64-column slabs stream better (M = 8: 8.3 against 11.6 µs).
-    // Without GLU also two groups a workgroup where one round holds them (N = 6144, M = 1: 7.4 against the
-    // skinny kernel's 9.7 µs; M = 16: 9.6 against 10.9), and three for a single row (N = 9216: 8.9 against
-    // 9.7; N = 12288: 10.6 against 11.4; at M = 16 the skinny kernel's 10.9 and 11.8 against 11.5 and 13.5).
-    const long gemv_groups = glu ? (N / 2 + 7) / 8 : (N + 15) / 16;
-    if (M <= 16 && gemv_groups <= cus) return WD_GEMV;
-    if (M <= 16 && !glu && (gemv_groups <= 2L * cus || (M == 1 && gemv_groups <= 3L * cus))) return WD_GEMV;
-    return M <= 128 ? WD_SKINNY32 : WD_SKINNY64;
-}
-
-int choose_wd_tile(int M, int N, bool glu, int cus, int kt) {
-    if (cus <= 0) cus = 256;
-    const int base = base_wd_tile(M, N, glu, cus);
-    // Below the 128-row tiles and not for the GLU epilogues: tiles of one-block waves whose K
-    // steps split over wave groups (each group its own activation stages; the CU holds two or four times
-    // the waves and the loads in flight of the same tile). The largest of them whose tiles number between
-    // 3/4 of the CUs and the CUs, else the one with the most tiles within one round. Measured against the
-    // kernel taken without them (one process, medians of 140 launches, HIP events), M × N at K = 3072:
-    // 64 × 3072 9.6 against 13.2 µs (32 × 32, four groups), 128 × 3072 11.4 against 13.6 (32 × 64), 256 ×
-    // 3072 14.7 against 19.3 (64 × 64), C2's text stream 512 × 3072 18.6 against 20.0 (64 × 128, two
-    // groups), C0 1024 × 3072 26.3 against 28.3 (64 × 192), 64 × 9216 14.4 against 20.8, 256 × 12288 26.3
-    // against 28.2; at K = 12288, N = 3072: M = 64 19.4 against 33.8, M = 256 36.2 against 56.8.
-    // Up to 16 rows only where the short-M kernel would read the activation from global memory (it does not
-    // fit its LDS): 16 × 6144 × 3072 11.2 against 13.4 µs, 16 × 12288 × 3072 16.8 against 21.1 (M = 4 at K =
-    // 12288 fits: 13.6 against 16.6 for the K-group tile). Past one round of 16-column groups the skinny kernel
-    // stays (M = 16, K = 12288, N = 12288: 26.7 against 27.8).
-    if (glu || base == WD_256 || base == WD_224 || base == WD_128) return base;
-    if (M <= 16 && (base != WD_GEMV || gemv_x_in_lds(M, kt))) return base;
-    // The short-M kernel's several groups a workgroup were measured with the activation in LDS only.
-    if (M <= 16 && (N + 15) / 16 > cus) return WD_SKINNY32;
-    struct Cand { int tile, bm, bn, groups; };
-    static const Cand cands[] = {{WD_K64x192, 64, 192, 2}, {WD_K64x128, 64, 128, 2}, {WD_K64x64, 64, 64, 4},
-                                 {WD_K32x64, 32, 64, 4}, {WD_K32x32, 32, 32, 4}};
-    auto count = [&](const Cand &c) { return (long)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn); };
-    for (const Cand &c : cands)
-        if (kt % c.groups == 0 && count(c) >= (long)cus * 3 / 4 && count(c) <= cus) return c.tile;
-    int best = base;
-    long most = 0;
-    for (const Cand &c : cands)
-        if (kt % c.groups == 0 && count(c) <= cus && count(c) > most) {
-            best = c.tile;
-            most = count(c);
-        }
-    return best;
+// Tiles of `rows` rows × `nb` of the weight's blocks; a count past 2^24 only rounds.
+static inline float tile_count(int M, int rows, int blocks, int nb) {
+    return (float)((M + rows - 1) / rows) * (float)((blocks + nb - 1) / nb);
 }
 
 // Microseconds of `tiles` workgroups, `cus` at a time, `round` each: a last, partly filled round is shorter (its
 // workgroups share the memory system with fewer others: half the CUs 0.83 of a full round).
-static float rounds_us(long tiles, int cus, float round) {
-    const long full = tiles / cus, rest = tiles % cus;
-    return round * ((float)full + (rest ? 0.66f + 0.34f * (float)rest / (float)cus : 0.0f));
+static float rounds_us(float tiles, int cus, float round) {
+    const float rounds = tiles / (float)cus, full = floorf(rounds), rest = rounds - full;
+    return round * (full + (rest > 0.0f ? 0.66f + 0.34f * rest : 0.0f));
+}
+
+// The same of a kernel of two workgroups a CU: `two` a round of them, `one` a last round of at most one a CU.
+static float pairs_us(float tiles, int cus, float two, float one) {
+    const float full = floorf(tiles / (2.0f * (float)cus)), rest = tiles - full * 2.0f * (float)cus;
+    return full * two + (rest > (float)cus ? two : rounds_us(rest, cus, one));
+}
+
+// Calls take(tile, µs) for every K-group shape that serves M rows × `blocks` 32-column blocks of weight and `steps` weight K
+// steps (unrolled: each shape's divisions are by constants; the rule runs on every call).
+template <int MATH, int I = 0, typename F>
+static inline void each_group(int M, int blocks, bool glu, int cus, int steps, F &&take) {
+    if constexpr (I < kGroupShapes) {
+        constexpr GroupShape g = group_shapes[I];
+        constexpr GroupCost c = g.cost[MATH];
+        constexpr int nw = g.cols / 32;
+        // bf16: four groups give the skinny kernel's bits at any K, two the 64 × 128 tiles' where the steps divide.
+        if (c.us_step > 0.0f && !(glu && nw % 2 != 0) && !(MATH == GM_BF16 && steps % 2 != 0 && g.groups == 2))
+            take(GROUP_TILE0 + I, rounds_us(tile_count(M, g.rows, blocks, nw), cus, c.us + c.us_step * (float)steps));
+        each_group<MATH, I + 1>(M, blocks, glu, cus, steps, take);
+    }
+}
+
+int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32, bool w256) {
+    if (cus <= 0) cus = 256;
+    const int kt = f32 ? 3 * steps : steps;  // the activation's K steps
+    // Up to 16 rows, the 16-column groups of the short-M kernel where they fit one round of one or two groups a
+    // workgroup on the CUs (N ≤ 8192 on 256 CUs), for a single row without GLU three (N ≤ 12288): every K step's loads
+    // in flight, the activation read once per workgroup. Kernel traces at K = 3072, N = 3072 (int8 packed, bias): M = 1
+    // 4.10 µs against the skinny kernel's 7.44, M = 16 5.95 against 8.73; two groups, SiLU-GLU: M = 3, N = 8192 5.8
+    // against 8.5, M = 16 7.3 against 9.4; three, M = 1: N = 9216 8.9 against 9.7, N = 12288 10.6 against 11.4. Past
+    // four rows only with the activation in its LDS (16 × 6144 × 3072 11.3 against 8.5 µs for a K-group tile).
+    const int groups16 = glu ? (N / 2 + 7) / 8 : (N + 15) / 16;
+    if (M <= 16 && (M <= 4 || gemv_x_in_lds(M, kt)) && (groups16 <= 2 * cus || (M == 1 && !glu && groups16 <= 3 * cus)))
+        return WD_GEMV;
+    // Up to 16 rows on a weight wider than 3/4 of the CUs' 64-column slabs, the skinny kernel (a slab a workgroup, four
+    // a CU): its many small workgroups stream the weight best (1 × 3072 × 18432 13.7 µs against 16.0 in 32 × 64 tiles, 8
+    // × 9216 7.9 against 7.2). The fp32 route's K-group tiles load the codes once for three parts (16 × 12288 17.8
+    // against 21.9).
+    const int blocks = glu ? 2 * ((N / 2 + 31) / 32) : (N + 31) / 32;  // 32-column blocks
+    if (M <= 16 && !f32 && (blocks + 1) / 2 >= cus * 3 / 4) return WD_SKINNY32;
+    // Else the tile of the least estimated time: µs a round of tiles, one a CU (128 × 256: two a CU, or one in a round
+    // of at most one a CU), measured at K = 1024, 3072 and 8192 as the K-group tiles' (GroupShape). Few tiles go to the
+    // K-group tiles: more CUs, and eight to sixteen waves a CU with their loads in flight whatever the tile; many to
+    // the 256- and 224-row tiles of one workgroup a CU (the least widening and operand traffic), the height whose
+    // rounds cover the fewest rows. Measured (µs, the thresholds of before → this): 512 × 3072 × 3072 16.5 → 14.6, 1531
+    // × 3072 × 3072 41.8 → 33.0, 200 × 3072 × 6144 16.4 → 14.0; SiLU-GLU 333 × 3840 × 20480 74.4 → 55.2, 77 × 3840 ×
+    // 20480 30.6 → 24.1, 20 × 3072 × 6144 10.0 → 7.0, 43 × 3424 × 10880 23.1 → 14.8; fp32 route 1531 × 3072 × 3072
+    // 141 → 87, 18 × 6592 × 64 36 → 20, 176 × 8512 × 64 117 → 34.
+    struct Round { float us, us_step; };
+    const Round two = f32 ? Round{21.5f, 5.07f} : Round{8.2f, 1.605f}, one = f32 ? Round{28.5f, 2.66f} : Round{7.0f, 0.905f};
+    const Round r224 = f32 ? Round{32.0f, 4.00f} : Round{7.9f, 1.28f}, r256 = f32 ? Round{35.0f, 4.56f} : Round{9.0f, 1.445f};
+    auto us = [&](const Round &r) { return r.us + r.us_step * (float)steps; };
+    auto tiles = [&](int bm) { return tile_count(M, bm, blocks, 8); };
+    float best = pairs_us(tiles(128), cus, us(two), us(one));
+    int tile = WD_128;
+    auto take = [&](int t, float time) {
+        if (time < best) {
+            best = time;
+            tile = t;
+        }
+    };
+    if (w256) {
+        take(WD_256, rounds_us(tiles(256), cus, us(r256)));
+        take(WD_224, rounds_us(tiles(224), cus, us(r224)));
+    }
+    if (f32)
+        each_group<GM_F32>(M, blocks, glu, cus, steps, take);
+    else
+        each_group<GM_BF16>(M, blocks, glu, cus, steps, take);
+    return tile;
 }
 
 int choose_i8_tile(int M, int N, bool glu, int cus, int kt) {
@@ -140,23 +152,15 @@ int choose_i8_tile(int M, int N, bool glu, int cus, int kt) {
     // against the rule's: 1 × 3072 20.8 → 4.9, 77 × 12288 22.6 → 12.9, 512 × 3072 23.0 → 10.8, 1021 × 3072 24.5 →
     // 17.0, 333 × 9216 25.0 → 20.0; K = 12288, 68 × 512 62.9 → 9.7.
     if (cus <= 0) cus = 256;
-    const long blocks = glu ? 2 * (((long)N / 2 + 31) / 32) : ((long)N + 31) / 32;  // 32-column blocks
-    const long big = (long)((M + 127) / 128) * ((blocks + 7) / 8), slots = 2L * cus;
-    const float two = 11.2f + 1.70f * (float)kt, one = 9.6f + 0.91f * (float)kt;
-    const long rest = big % slots;
-    float best = (float)(big / slots) * two + (rest > cus ? two : rounds_us(rest, cus, one));
+    const int blocks = glu ? 2 * ((N / 2 + 31) / 32) : (N + 31) / 32;  // 32-column blocks
+    float best = pairs_us(tile_count(M, 128, blocks, 8), cus, 11.2f + 1.70f * (float)kt, 9.6f + 0.91f * (float)kt);
     int tile = I8_128x256;
-    for (int i = 0; i < kGroupShapes; ++i) {
-        const GroupShape &g = group_shapes[i];
-        const int nw = g.cols / 32;
-        if (glu && nw % 2 != 0) continue;
-        const float us = rounds_us((long)((M + g.rows - 1) / g.rows) * ((blocks + nw - 1) / nw), cus,
-                                   g.us + g.us_step * (float)kt);
-        if (us < best) {
-            best = us;
-            tile = GROUP_TILE0 + i;
+    each_group<GM_I8>(M, blocks, glu, cus, kt, [&](int t, float time) {
+        if (time < best) {
+            best = time;
+            tile = t;
         }
-    }
+    });
     return tile;
 }
 
@@ -170,8 +174,8 @@ int choose_blocks_tile(int M, int N, bool glu, int cus, int kt) {
     // 396: one activation tile for twice the columns; level at two rounds).
     if (cus <= 0) cus = 256;
     const float steps = (float)kt;
-    const long slabs = glu ? ((long)N / 2 + 31) / 32 : ((long)N + 63) / 64;
-    auto a_cu = [&](int rows, long per) { return (float)(((long)((M + rows - 1) / rows) * ((slabs + per - 1) / per) + cus - 1) / cus); };
+    const int slabs = glu ? (N / 2 + 31) / 32 : (N + 63) / 64;
+    auto a_cu = [&](int rows, int per) { return ceilf(tile_count(M, rows, slabs, per) / (float)cus); };
     struct Narrow { int rows; float chain, work; };
     static const Narrow narrow[] = {{16, 0.175f, 0.13f}, {32, 0.208f, 0.15f}, {48, 0.26f, 0.195f}, {64, 0.3125f, 0.238f},
                                     {80, 0.375f, 0.294f}};

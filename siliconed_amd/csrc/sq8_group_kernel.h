@@ -3,9 +3,12 @@
 // stages), so one workgroup a CU holds eight waves and their loads in flight whatever its tile; the groups'
 // sums meet in LDS and are added in group order (deterministic; exact for int32).
 //
-// Two kinds of product (MATH):
+// Three kinds of product (MATH):
 //   GM_BF16 — bf16 activation × 8-bit codes widened to bf16 (sq8_wdirect_kernel.h's arithmetic, K steps of 64;
 //             every K-group count a family of bits of its own, the same over all tile shapes);
+//   GM_F32  — the same codes under an fp32 activation's three bf16 parts along K (the fp32 route): a weight step's
+//             codes are loaded and widened once and meet the three parts' activation steps in turn (as 3·K steps each
+//             code is loaded and widened three times); the steps split over the groups are the weight's;
 //   GM_I8   — int8 activation codes × int8 codes, int32 sums (sq8_i8_kernel.h's, K steps of 128): the same
 //             bits as every other W8A8 kernel whatever the split.
 // Both stage 128 bytes of every activation row per K step, so the rings, swizzles and direct loads are shared.
@@ -32,8 +35,6 @@ using wd::step_barrier;
 using wd::swz;
 using wd::wait_vmcnt;
 
-enum GroupMath { GM_BF16 = 0, GM_I8 = 1 };
-
 constexpr int PITCH = 144;           // bytes a row of 32 staged sums takes (16-byte aligned, banks spread)
 constexpr int SLOT = 32 * PITCH;     // one 32 × 32 block of sums
 
@@ -42,46 +43,72 @@ constexpr int lds_bytes(int bm, int nw, int ks, int nas) {
     return stages > sums ? stages : sums;
 }
 
-// Four output columns [col, col + 4) of row m, column values v (scaled, biased, activated), to the product's
-// output: the residual stream, or output tensor / head as out_index says; one store where aligned.
-__device__ __forceinline__ void store4(const GemmArgs &p, int m, int col, int n_out, const float (&v)[4]) {
+// Where four output columns [col, col + 4) go, rows 0: in the residual stream, or the output tensor and head out_index says;
+// `whole`: all four at at[0], aligned for one store. Worked out once a thread, before the row blocks: out_index divides
+// (by the split and the head), and its code in every row block's stores made kernels of up to 61 KB (now 46), which each
+// product reads past a cold instruction cache: 432 × 2048 × 8192 with GELU inside a block 27.1 → 25.5 µs. (A loop over the row
+// blocks, 33 KB, 26.3 there, but 0.5 µs more on every product alone.)
+struct Out4 {
+    uint8_t *at[4];
+    bool whole;
+};
+
+__device__ __forceinline__ Out4 out4(const GemmArgs &p, int col, int n_out) {
+    Out4 o;
     if (p.epi == EPI_RESIDUAL) {
-        float *xr = reinterpret_cast<float *>(p.c[0]) + (int64_t)m * p.ldc + col;
-        if (p.c_vec16 && col + 4 <= n_out) {
+        o.whole = p.c_vec16 && col + 4 <= n_out;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o.at[e] = reinterpret_cast<uint8_t *>(p.c[0]) + (int64_t)(col + e) * 4;
+        return o;
+    }
+    const int esz = p.out == OUT_F32 ? 4 : 2;
+    o.whole = p.c_vec && col + 4 <= n_out && (p.split % 4) == 0;  // the four in one output and head
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (e > 0 && o.whole) {
+            o.at[e] = o.at[0];
+        } else {
+            int which = 0;
+            const int64_t off = p.split > 0 || p.head_dim > 0 ? wd::out_index(p, 0, min(col + e, n_out - 1), which) : col + e;
+            o.at[e] = kern::out_base(p, which) + off * esz;
+        }
+    }
+    return o;
+}
+
+// Stores the values v (scaled, biased, activated) of columns [col, col + 4), `row` bytes past their rows 0.
+__device__ __forceinline__ void store4(const GemmArgs &p, const Out4 &o, int64_t row, int col, int n_out, const float (&v)[4]) {
+    if (p.epi == EPI_RESIDUAL) {
+        if (o.whole) {
+            float *xr = reinterpret_cast<float *>(o.at[0] + row);
             const f32x4 xv = *reinterpret_cast<const f32x4 *>(xr);
             const f32x4 gv = p.gate ? *reinterpret_cast<const f32x4 *>(p.gate + col) : f32x4{1.0f, 1.0f, 1.0f, 1.0f};
-            f32x4 o;
+            f32x4 y;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = __fadd_rn(xv[e], __fmul_rn(gv[e], v[e]));
-            *reinterpret_cast<f32x4 *>(xr) = o;
+            for (int e = 0; e < 4; ++e) y[e] = __fadd_rn(xv[e], __fmul_rn(gv[e], v[e]));
+            *reinterpret_cast<f32x4 *>(xr) = y;
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (col + e < n_out) xr[e] = __fadd_rn(xr[e], __fmul_rn(p.gate ? p.gate[col + e] : 1.0f, v[e]));
+                if (col + e < n_out) {
+                    float *xr = reinterpret_cast<float *>(o.at[e] + row);
+                    *xr = __fadd_rn(*xr, __fmul_rn(p.gate ? p.gate[col + e] : 1.0f, v[e]));
+                }
         }
-        return;
-    }
-    const bool whole = p.c_vec && col + 4 <= n_out && (p.split % 4) == 0;  // the four in one output and head
-    if (whole) {
-        int which = 0;
-        const int64_t off = p.split > 0 || p.head_dim > 0 ? wd::out_index(p, m, col, which) : (int64_t)m * p.ldc + col;
-        uint8_t *o = kern::out_base(p, which);
+    } else if (o.whole) {
         if (p.out == OUT_F32)
-            *reinterpret_cast<f32x4 *>(o + off * 4) = f32x4{v[0], v[1], v[2], v[3]};
+            *reinterpret_cast<f32x4 *>(o.at[0] + row) = f32x4{v[0], v[1], v[2], v[3]};
         else
-            *reinterpret_cast<u32x2 *>(o + off * 2) = u32x2{pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3])};
-        return;
-    }
+            *reinterpret_cast<u32x2 *>(o.at[0] + row) = u32x2{pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3])};
+    } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        if (col + e >= n_out) break;
-        int which;
-        const int64_t off = wd::out_index(p, m, col + e, which);
-        uint8_t *o = kern::out_base(p, which);
-        if (p.out == OUT_F32)
-            reinterpret_cast<float *>(o)[off] = v[e];
-        else
-            reinterpret_cast<uint16_t *>(o)[off] = (uint16_t)(pack_bf16_rne(v[e], 0.0f) & 0xFFFFu);
+        for (int e = 0; e < 4; ++e) {
+            if (col + e >= n_out) break;
+            if (p.out == OUT_F32)
+                *reinterpret_cast<float *>(o.at[e] + row) = v[e];
+            else
+                *reinterpret_cast<uint16_t *>(o.at[e] + row) = (uint16_t)(pack_bf16_rne(v[e], 0.0f) & 0xFFFFu);
+        }
     }
 }
 
@@ -123,7 +150,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * NW * KS, 64 * NW
                                amdgpu_waves_per_eu(NW *KS / 4, NW *KS / 4)))
 gemm_group_kernel(const GemmArgs p) {
     static_assert(NW * KS % 4 == 0, "the workgroup's waves spread evenly over the four SIMDs");
-    constexpr bool I8 = MATH == GM_I8;
+    constexpr bool I8 = MATH == GM_I8, F32 = MATH == GM_F32;
     constexpr int FM = BM / 32;
     constexpr int SA = BM * 128;                 // bytes per activation stage
     // 1 KB direct loads per wave per step; where the blocks do not split evenly over a group's waves the last loads
@@ -137,6 +164,8 @@ gemm_group_kernel(const GemmArgs p) {
     // Loads a wave may leave in flight at the end of step t, A(t+1) and W(t+1) landed.
     constexpr int STEP_WAIT = WLD + (NAS - 2) * (A_PER_WAVE + WLD);
     static_assert(STEP_WAIT < 64, "vmcnt budget");
+    static_assert(!F32 || NAS == 3, "the fp32 route's activation stages are its three parts");
+    constexpr int NWB = F32 ? 2 : NAS;           // code buffers
 
     __shared__ __attribute__((aligned(1024))) uint8_t lds[lds_bytes(BM, NW, KS, NAS)];
 
@@ -150,7 +179,7 @@ gemm_group_kernel(const GemmArgs p) {
     const bool glu = p.glu_half > 0;             // NW even only (the launcher's rule): a pair of blocks is one tile's
     const int slab = (tn * NW + wave) >> 1, b0 = (tn * NW + wave) & 1;  // the wave's block: b0 of slab
     const kern::gbytes Wg = (kern::gbytes)p.w;
-    const int KT = p.kt;
+    const int KT = F32 ? p.kt_w : p.kt;          // the weight's steps
 
     // ---- activation: wave block b = wave + NW·i of 8 rows, lane → row 8b + lane/8, chunk lane%8 ----
     uint32_t a_goff[A_PER_WAVE];
@@ -168,7 +197,9 @@ gemm_group_kernel(const GemmArgs p) {
     const wd::i32x4 a_rsrc = buffer_rsrc(p.a);
     auto issue_a = [&](int t, auto stage) {
         constexpr int S = decltype(stage)::value;
-        const int soff = __builtin_amdgcn_readfirstlane((int)((uint32_t)min(t * KS + group, KT - 1) * 128));
+        // Fp32 route: t counts activation steps, three (stages 0, 1, 2: the parts, KT · 128 bytes apart) a weight step.
+        const int soff = __builtin_amdgcn_readfirstlane(
+            (int)((uint32_t)min((F32 ? t / 3 : t) * KS + group, KT - 1) * 128 + (F32 ? (uint32_t)(S * KT) * 128 : 0u)));
 #pragma unroll
         for (int i = 0; i < A_PER_WAVE; ++i)
             raw_buffer_load_lds(a_rsrc, (lds_u32)(ldg + S * SA + a_blk[i] * 1024), 16, (int)a_goff[i], soff, 0, 0);
@@ -182,7 +213,7 @@ gemm_group_kernel(const GemmArgs p) {
         if constexpr (WL == W_PACKED) {
             const int slabs = glu ? (p.glu_half + 31) / 32 : (p.N + 63) / 64;
             const int s = slab < slabs ? slab : slabs - 1;
-            const int kt = p.kt_w > 0 ? p.kt_w : p.kt;
+            const int kt = I8 ? p.kt_w : KT;
             w_off[j] = (uint32_t)(((int64_t)s * kt * 4 + 2 * b0 + j) * 1024 + lane * 16);
         } else {
             const int hl = lane >> 5, nl = lane & 31;
@@ -191,7 +222,7 @@ gemm_group_kernel(const GemmArgs p) {
         }
     }
     constexpr uint32_t w_step = WL == W_PACKED ? 4096 : 64;
-    u32x4 raw[NAS][WLD];
+    u32x4 raw[NWB][WLD];
     auto issue_w = [&](int t, auto buf) {
         constexpr int B = decltype(buf)::value;
         const int tt = min(t * KS + group, KT - 1);
@@ -204,7 +235,7 @@ gemm_group_kernel(const GemmArgs p) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) raw[B][2 + j] = kern::gld<u32x4>(b1p, w_off[j]);
         } else {
-            const kern::gbytes base = Wg + (uint32_t)wd::weight_step(p, tt) * w_step;
+            const kern::gbytes base = Wg + (uint32_t)tt * w_step;
 #pragma unroll
             for (int j = 0; j < 2; ++j) raw[B][j] = kern::gld<u32x4>(base, w_off[j]);
         }
@@ -225,27 +256,52 @@ gemm_group_kernel(const GemmArgs p) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[bm][r] = 0;
 
-    // Prologue in the steps' issue order: A(0 .. NAS−2) and W(0 .. NAS−1); A(0) and W(0) landed.
-    static_for<0, NAS>([&](auto vc) {
-        constexpr int v = decltype(vc)::value;
-        if constexpr (v > 0) issue_a(v - 1, std::integral_constant<int, v - 1>{});
-        issue_w(v, vc);
-    });
-    wait_vmcnt<STEP_WAIT>();
+    // The prologue's loads in the order the waits count on (the compiler would move the codes' loads past the others).
+    auto ordered = [&](auto &&f) {
+        f();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (F32) {
+        // A(0), A(1) (parts 0 and 1 of the first weight step) and W(0), W(1): A(0) and W(0) landed.
+        using S0 = std::integral_constant<int, 0>;
+        using S1 = std::integral_constant<int, 1>;
+        ordered([&] { issue_w(0, S0{}); });
+        ordered([&] { issue_a(0, S0{}); });
+        ordered([&] { issue_w(1, S1{}); });
+        ordered([&] { issue_a(1, S1{}); });
+        wait_vmcnt<WLD + A_PER_WAVE>();
+    } else {
+        // The steps' issue order: A(0 .. NAS−2) and W(0 .. NAS−1); A(0) and W(0) landed.
+        static_for<0, NAS>([&](auto vc) {
+            constexpr int v = decltype(vc)::value;
+            if constexpr (v > 0) ordered([&] { issue_a(v - 1, std::integral_constant<int, v - 1>{}); });
+            ordered([&] { issue_w(v, vc); });
+        });
+        wait_vmcnt<STEP_WAIT>();
+    }
     step_barrier();
 
     using I0 = std::integral_constant<int, 0>;
-    auto step = [&](int t, auto uc) {
-        constexpr int U = decltype(uc)::value;  // stage and register buffer of step t
+    u32x4 wf[F32 ? 4 : 1];  // fp32 route: the weight step's widened codes, kept for its three parts
+    // Step t on stage U; its codes in buffer B (fp32 route: part U of the weight step in buffer B).
+    // TAIL: one of the last steps, whose code loads no later step uses and the compiler drops: the wait counts the
+    // activation's loads only (as if every code load had been dropped).
+    auto step = [&](int t, auto uc, auto bc, auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
+        constexpr int U = decltype(uc)::value, B = decltype(bc)::value;
         u32x4 wk[2];                            // the sub-step's codes (widened, or as they are)
         u32x4 xf[2][FM];
         auto codes = [&](auto sc) {
             constexpr int s = decltype(sc)::value;
             if constexpr (I8) {
-                wk[s & 1] = raw[U][s];
+                wk[s & 1] = raw[B][s];
+            } else if constexpr (F32 && U > 0) {
+                wk[s & 1] = wf[s];
             } else {
-                const u32x4 &r = raw[U][s >> 1];
+                const u32x4 &r = raw[B][s >> 1];
                 wk[s & 1] = __builtin_bit_cast(u32x4, wd::widen8<WT>(r[2 * (s & 1)], r[2 * (s & 1) + 1]));
+                if constexpr (F32) wf[s] = wk[s & 1];
             }
         };
         auto read_x = [&](auto sc) {
@@ -268,9 +324,9 @@ gemm_group_kernel(const GemmArgs p) {
             }
             // The buffer's last codes are read (bf16: widened) by sub-step 2; the A loads stay ahead of
             // these in issue order (the vmcnt counts rely on it).
-            if constexpr (!I8 && s == 2) {
+            if constexpr (!I8 && s == 2 && (!F32 || U == 0)) {
                 __builtin_amdgcn_sched_barrier(0);
-                issue_w(t + NAS, uc);
+                issue_w(F32 ? t / 3 + NWB : t + NAS, bc);
                 __builtin_amdgcn_sched_barrier(0);
             }
             static_for<0, FM>([&](auto bmc) {
@@ -294,10 +350,12 @@ gemm_group_kernel(const GemmArgs p) {
             __builtin_amdgcn_sched_barrier(0);
         });
         if constexpr (I8) {
-            issue_w(t + NAS, uc);
+            issue_w(t + NAS, bc);
             __builtin_amdgcn_sched_barrier(0);
         }
-        wait_vmcnt<STEP_WAIT>();
+        // Fp32 route: A(t + 1) landed; A(t + 2) may fly, and the codes issued in part 0 beside it.
+        if constexpr (F32) wait_vmcnt<A_PER_WAVE + (U < 2 && !TAIL ? WLD : 0)>();
+        else wait_vmcnt<TAIL ? (NAS - 2) * A_PER_WAVE : STEP_WAIT>();
         // A group of one wave shares no LDS within the K loop (it reads only the stages it loads itself).
         if constexpr (NW > 1) step_barrier();
         else asm volatile("" ::: "memory");
@@ -307,13 +365,22 @@ gemm_group_kernel(const GemmArgs p) {
     const int mine = group < KT ? (KT - group + KS - 1) / KS : 0;
     const int rounds = (KT + KS - 1) / KS;
     int t = 0;
-    for (; t + NAS <= mine; t += NAS) static_for<0, NAS>([&](auto uc) { step(t + decltype(uc)::value, uc); });
-    static_for<0, NAS>([&](auto uc) {
-        constexpr int u = decltype(uc)::value;
-        if (t + u < mine) step(t + u, uc);
-    });
+    if constexpr (F32) {
+        auto three = [&](int i, auto bc, auto tail) {
+            static_for<0, 3>([&](auto uc) { step(3 * i + decltype(uc)::value, uc, bc, tail); });
+        };
+        for (; t + 2 <= mine; t += 2)
+            static_for<0, 2>([&](auto bc) { three(t + decltype(bc)::value, bc, std::false_type{}); });
+        if (t < mine) three(t, I0{}, std::true_type{});
+    } else {
+        for (; t + NAS <= mine; t += NAS) static_for<0, NAS>([&](auto uc) { step(t + decltype(uc)::value, uc, uc, std::false_type{}); });
+        static_for<0, NAS>([&](auto uc) {
+            constexpr int u = decltype(uc)::value;
+            if (t + u < mine) step(t + u, uc, uc, std::true_type{});
+        });
+    }
     if constexpr (NW > 1) {
-        if (mine < rounds) step_barrier();
+        if (mine < rounds) static_for<0, F32 ? 3 : 1>([&](auto) { step_barrier(); });
     }
     wait_vmcnt<0>();
     __syncthreads();
@@ -327,11 +394,13 @@ gemm_group_kernel(const GemmArgs p) {
     const int chunk = tid & 7;
     float sc[IT][4], bi[IT][4], su[IT][4], bu[IT][4];
     int col[IT];
+    Out4 to[IT];
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
         const int it = tid + i * THREADS, blk = it >> 8;
         if (it < items) {
             col[i] = (glu ? tn * NW / 2 + blk : tn * NW + blk) * 32 + 4 * chunk;
+            to[i] = out4(p, min(col[i], n_out - 1), n_out);
             column4(p.scale, p.scale_per_col, p.sb_vec, col[i], n_out, 0, sc[i]);
             column4(p.bias, true, p.sb_vec, col[i], n_out, 0, bi[i]);
             if (glu) {
@@ -343,6 +412,7 @@ gemm_group_kernel(const GemmArgs p) {
         }
     }
     const bool has_bias = p.bias != nullptr;
+    const int64_t row_bytes = p.epi == EPI_RESIDUAL ? p.ldc * 4 : (p.head_dim > 0 ? p.head_dim : p.ldc) * (p.out == OUT_F32 ? 4 : 2);
     static_for<0, FM>([&](auto bmc) {
         constexpr int bm = decltype(bmc)::value;
         uint8_t *dst = lds + wave_all * SLOT + (lane & 31) * PITCH + 16 * h;
@@ -385,7 +455,7 @@ gemm_group_kernel(const GemmArgs p) {
                     }
                 }
                 activate4(p.epi, v, u);
-                store4(p, m, col[i], n_out, v);
+                store4(p, to[i], m * row_bytes, col[i], n_out, v);
             }
         }
         if constexpr (bm + 1 < FM) __syncthreads();

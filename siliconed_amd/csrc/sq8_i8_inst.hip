@@ -7,7 +7,7 @@
 namespace sq8 {
 
 hipError_t launch_i8gemm(const GemmArgs &p, int tile, int wl, int epi, int out, hipStream_t stream) {
-    if (tile >= GROUP_TILE0) return launch_group_i8(p, tile - GROUP_TILE0, wl, epi, out, stream);
+    if (tile >= GROUP_TILE0) return launch_group(p, GM_I8, tile - GROUP_TILE0, W_INT8, wl, epi, out, stream);
     // Three activation stages: C1 on the W8A8 route 2012 → 2025 TOP/s (three interleaved pairs).
     if (wl == W_PACKED) return wd::dispatch_i8<128, 4, W_PACKED, 3>(p, epi, out, stream);
     if (wl == W_NK) return wd::dispatch_i8<128, 4, W_NK, 3>(p, epi, out, stream);

@@ -216,7 +216,10 @@ gemm_w256_kernel(const GemmArgs p) {
     read_x(I0{}, I0{}, I0{});
     widen_ks(I0{}, I0{}, I0{});
 
-    auto step = [&](int s, auto uc) {
+    // TAIL: one of the last steps, whose code loads no later step uses and the compiler drops: the wait counts the
+    // activation's loads only (as if every code load had been dropped).
+    auto step = [&](int s, auto uc, auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
         constexpr int U = decltype(uc)::value;
         constexpr int N1 = (U + 1) % 4, N3 = (U + 3) % 4;
         using SU = std::integral_constant<int, U>;
@@ -241,19 +244,19 @@ gemm_w256_kernel(const GemmArgs p) {
             interleave(kc);
             __builtin_amdgcn_sched_barrier(0);
         });
-        wait_vmcnt<A_PER_WAVE + 4>();
+        wait_vmcnt<A_PER_WAVE + (TAIL ? 0 : 4)>();
         step_barrier();
     };
     int s = 0;
     for (; s + 4 <= KT; s += 4) {
-        step(s, I0{});
-        step(s + 1, I1{});
-        step(s + 2, I2{});
-        step(s + 3, I3{});
+        step(s, I0{}, std::false_type{});
+        step(s + 1, I1{}, std::false_type{});
+        step(s + 2, I2{}, std::false_type{});
+        step(s + 3, I3{}, std::false_type{});
     }
-    if (s < KT) step(s, I0{});
-    if (s + 1 < KT) step(s + 1, I1{});
-    if (s + 2 < KT) step(s + 2, I2{});
+    if (s < KT) step(s, I0{}, std::true_type{});
+    if (s + 1 < KT) step(s + 1, I1{}, std::true_type{});
+    if (s + 2 < KT) step(s + 2, I2{}, std::true_type{});
 
     // Every wave's last (clamped) loads have landed before any wave writes its region over the stages.
     wait_vmcnt<0>();
@@ -312,19 +315,6 @@ gemm_w256_kernel(const GemmArgs p) {
             }
         });
     }
-}
-
-// True when the 256 × 256 kernel runs this product: whole 64-column slabs (GLU: whole 32-column
-// slabs of each half) and 16-byte scale/bias loads; for the slab epilogue (bf16 out, no activation or
-// GELU) also slabs that each lie in one output (and one head) and 16-byte stores. The fp32 route's three
-// parts along K (kt_w > 0) face the weight's steps in turn (weight_step).
-inline bool w256_fits(const GemmArgs &p, int epi, int out) {
-    if (!p.sb_vec) return false;
-    if (p.glu_half > 0 ? p.glu_half % 32 != 0 : p.N % 64 != 0) return false;
-    if (epi == EPI_RESIDUAL && out != OUT_F32) return false;
-    if ((epi == EPI_NONE || epi == EPI_GELU) && out == OUT_BF16)
-        return p.split % 64 == 0 && p.head_dim % 64 == 0 && p.c_vec16;
-    return true;
 }
 
 template <int WT, int WL, int BM = 256>

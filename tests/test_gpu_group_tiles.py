@@ -108,3 +108,59 @@ def test_q8_tile_sums_in_k_order(gemm, q8_gemm, tile):
             z = q8_gemm["16"].product_blocks(a, w, bias=b, epilogue=epi, out_dtype=out, rounding=not exact)
             torch.cuda.synchronize()
             assert torch.equal(y, z)
+
+
+BF16_TILES = ["g32x32k4", "g32x64k4", "g64x64k4", "g64x96k4", "g64x128k4", "g64x128k2", "g64x192k2", "g96x96k4", "g96x128k4",
+              "g128x96k4", "g128x128k2", "g96x192k2", "g128x192k2"]
+F32_TILES = [t for t in BF16_TILES if t not in ("g96x128k4", "g128x96k4")]
+
+
+@pytest.mark.parametrize("route,tile", [("bf16", t) for t in BF16_TILES] + [("fp32", t) for t in F32_TILES])
+def test_group_tile_exact_sums_same_bits(tile_gemm, route, tile):
+    """The bf16 and fp32 routes on operands whose every partial sum is exact in fp32 (so any split and order of K gives
+    the same bits), against the 128-row tiles: int8 and fp8 codes, both layouts, every epilogue, output type and output
+    layout. fp32 route: values of two and of three non-zero bf16 parts (12 and 18 significant bits)."""
+    bm, bn = (int(v) for v in tile[1:].split("k")[0].split("x"))
+    got, want = tile_gemm(tile), tile_gemm("128")
+    cases = [(1, 64, bn, None, torch.float32, False, True), (bm + 1, 320, bn + 32, "gelu_tanh", torch.bfloat16, False, False),
+             (bm, 512, bn + 4, None, torch.bfloat16, True, False), (2 * bm - 1, 448, 2 * bn + 1, None, torch.float32, False, True),
+             (bm - 1, 200, bn - 3, "gelu_tanh", torch.float32, False, False)]
+    if bn % 64 == 0:
+        cases += [(bm + 3, 320, 2 * (bn // 2 + 5), "silu_glu", torch.bfloat16, False, False),
+                  (bm, 512, 2 * bn, "situ_glu", torch.float32, True, True)]
+
+    def operands(m, k, n, seed, fp8):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        q = torch.randint(-3, 4, (n, k), device=DEV, generator=g)
+        s = torch.rand(n, device=DEV, generator=g) * 1e-2 + 1e-3
+        if route == "bf16":
+            x = torch.randint(-5, 6, (m, k), device=DEV, generator=g).bfloat16()
+        elif k > 64:
+            x = torch.randint(-2047, 2048, (m, k), device=DEV, generator=g).float() / 1024     # |sum| < 2^24 / 1024
+        else:
+            x = torch.randint(-(2 ** 16), 2 ** 16 + 1, (m, k), device=DEV, generator=g).float() / 65536 * 1.0
+            x = x + torch.randint(-1, 2, (m, k), device=DEV, generator=g) / 65536 / 2           # 18 bits; |q| ≤ 1 below
+            q = q.clamp(-1, 1)
+        return x, q.to(torch.float8_e4m3fn if fp8 else torch.int8), s, torch.randn(n, device=DEV, generator=g)
+
+    for m, k, n, epi, out, nk, fp8 in cases:
+        print(f"{route} {tile}: {m} x {k} x {n} {epi} {out} {'nk' if nk else 'packed'} {'fp8' if fp8 else 'int8'}", flush=True)
+        x, q, s, b = operands(m, k, n, m + k + n, fp8)
+        w = q if nk else want.pack(q, layout="nk", glu=epi in ("silu_glu", "situ_glu"))
+        ys = [g.product(x, w, s, bias=b, epilogue=epi, out_dtype=out, rounding=route == "bf16") for g in (got, want)]
+        torch.cuda.synchronize()
+        assert torch.equal(*ys)
+    if route == "bf16":
+        m, k, d = bm + 2, 320, 128
+        x, q, s, b = operands(m, k, 3 * d, 7, False)
+        w = want.pack(q, layout="nk")
+        for head_dim in (0, 32):
+            parts = [g.product_qkv(x, w, s, bias=b, head_dim=head_dim) for g in (got, want)]
+            torch.cuda.synchronize()
+            assert all(torch.equal(u, v) for u, v in zip(*parts))
+        gate = torch.linspace(-1.0, 1.0, 3 * d, device=DEV)
+        streams = [torch.ones((m, 3 * d), device=DEV) for _ in range(2)]
+        for g, y in zip((got, want), streams):
+            g.product_residual(y, x, w, s, bias=b, gate=gate)
+        torch.cuda.synchronize()
+        assert torch.equal(*streams)
