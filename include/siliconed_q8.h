@@ -84,8 +84,8 @@ typedef struct sq8_ctx sq8_ctx;
  * device's null stream). Refuses (SQ8_ENODEVICE) a device that is not gfx950.
  * Three measurement knobs are read from the environment here, once per context: SQ8_TILE ("256",
  * "224", "128", "64", "32", "64n", "64x192", "s64", "s32", "gemv", "k32x32", "k32x64", "k64x64", "k64x128",
- * "k64x192": the weight-direct kernels' tile; "128" or "g<rows>x<columns>k<groups>", "g64x96k4" for one: the W8A8
- * product's),
+ * "k64x192": the weight-direct kernels' tile; "128": the W8A8 product's; "g<rows>x<columns>k<groups>", "g64x96k4" for
+ * one: the tile of either),
  * SQ8_Q8_TILE ("128x256", "128x128", or "16", "32", "48", "64", "80" rows of the narrow-wave kernel: the
  * block-scale product's tile) and SQ8_SPLITS (a
  * count ≥ 1: the skinny
@@ -121,11 +121,14 @@ int sq8_supports(const sq8_ctx *ctx, int a_dtype, int w_dtype, int w_layout, int
  * `gpu_seconds`: NULL → the launch is queued and the call returns at once (`settled`,
  * TensorGEMM.swift:261-263); non-NULL → the call waits and writes the kernel's GPU seconds
  * (TensorGEMM.swift:268-272, `Attention.verdict`). One exception to "at once": the context's
- * growable buffers — the bf16 copy (or, on the fp32 route, the three parts) of an fp32 A, the
- * repack of [K, N] codes read in place, and the fp32 partial sums of a short product whose K steps
+ * growable buffers — the bf16 copy (or, on the fp32 route, the three parts) of an fp32 A or of a bf16 one whose rows
+ * are ragged or not 16-byte aligned, the repack of [K, N] codes (and of [N, K] ones the same way ragged or unaligned)
+ * read in place, and the fp32 partial sums of a short product whose K steps
  * are split over several workgroups (added by a second launch) — are sized by the largest product so far; a call that needs
  * more first synchronizes the context's stream (queued work may still read the old buffer), frees
- * and allocates. A caller that must never block runs one product of its largest shape first.
+ * and allocates. A caller that must never block runs one product of its largest shape first. Under stream capture a
+ * buffer cannot grow, and ragged or unaligned operands run on the kernels that read them as they lie, several times
+ * slower.
  * Replaces: TensorGEMM.linear(a:int8:weightOffset:scales:scalesOffset:perColumn:block:rotation:
  * rounding:quantizing:prequantized:c:m:k:n:settled:) -> Double (TensorGEMM.swift:264-290) and
  * its encoders submit (:296-360) / submitRounded (TensorGEMMBF16.swift:208-264), with the bias

@@ -170,6 +170,13 @@ int reserve_scratch(sq8_ctx *ctx, size_t bytes) {
     return SQ8_OK;
 }
 
+// Whether the context's stream is being captured into a graph (the growable buffers may not grow then: that synchronizes
+// and allocates).
+bool capturing(const sq8_ctx *ctx) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+}
+
 struct Product {
     const void *a; int a_dtype; int64_t lda;
     const void *w; int w_dtype; int w_layout; int64_t ldw;
@@ -241,19 +248,42 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
     // K not a whole number of 64-wide steps on the step kernels (a packed weight, the fp32 route, the
     // residual epilogue): the operand is staged with its rows padded to kp (zeros past k) and the weight
     // packed (zero codes past k), so each sum is the one over k alone (TensorGEMM.swift:124-135 computes
-    // any K). The bf16 route on codes as they lie keeps the guarded kernel for such K.
+    // any K).
     const int kp = (q.k + 63) / 64 * 64;
-    const bool pad_k = q.k % 64 != 0 && (q.exact || q.residual || is_packed(q.w_layout));
+    bool pad_k = q.k % 64 != 0 && (q.exact || q.residual || is_packed(q.w_layout));
     // The kernels address A and W with 32-bit byte offsets from their bases.
     const int64_t a_row = q.exact ? 3 * (int64_t)kp : pad_k ? kp : q.a_dtype == SQ8_BF16 && q.group == 0 ? q.lda : q.k;
+    const int64_t w_packed = sq8::packed_bytes(q.k, q.n, is_glu(q.epilogue));
     if ((int64_t)q.m * a_row * 2 > (int64_t)UINT32_MAX ||
-        std::max<int64_t>(sq8::packed_bytes(q.k, q.n, is_glu(q.epilogue)),
-                          is_packed(q.w_layout) ? 0 : (int64_t)(q.w_layout == SQ8_KN ? q.k : q.n) * q.ldw) >
+        std::max<int64_t>(w_packed, is_packed(q.w_layout) ? 0 : (int64_t)(q.w_layout == SQ8_KN ? q.k : q.n) * q.ldw) >
             (int64_t)UINT32_MAX)
         return SQ8_EUNSUPPORTED;
 
     DeviceScope scope(ctx->device);
     if (scope.error != hipSuccess) return hip_status(scope.error);
+    // Codes as they lie and an operand the step kernels cannot read in place (a ragged K, or bf16 rows not aligned for
+    // 16-byte loads): staged the same way, rows padded to kp, the weight repacked below. On [K, N] codes 1 × 4672 × 11563
+    // takes 51 µs so and took 372 in the guarded kernel, 7 × 2152 × 1873 14 and 121, 512 × 1000 × 3072 17 and 69 ([N, K]
+    // the same within 2 µs).
+    // The guarded and LDS-transposing kernels (launch_gemm) keep what 32-bit offsets do not reach once padded, what
+    // there is no memory to stage, and what is captured into a graph: a buffer that a later product grows is freed, and
+    // the graph would go on reading it. (Whole [K, N] slabs are repacked in a graph too, where the buffer holds them.)
+    const bool plain = !is_packed(q.w_layout) && !q.exact && !q.residual && q.k > 0;
+    const bool w_aligned = aligned(q.w, 16) && q.ldw % 16 == 0;
+    bool stage = plain && (q.k % 64 != 0 || (q.a_dtype == SQ8_BF16 && q.group == 0 && !(aligned(q.a, 16) && q.lda % 8 == 0)));
+    bool repack = plain && (q.w_layout == SQ8_KN || !w_aligned || q.k % 64 != 0);
+    if ((stage || repack) && capturing(ctx)) {
+        repack = q.w_layout == SQ8_KN && w_aligned && q.k % 256 == 0 && q.n % 64 == 0 && ctx->wpack_bytes >= (size_t)w_packed;
+        stage = false;
+    } else if (stage || repack) {
+        const int64_t bytes = (int64_t)q.m * kp * 2;
+        if ((stage && (bytes > (int64_t)UINT32_MAX || reserve_scratch(ctx, (size_t)bytes) != SQ8_OK)) ||
+            (repack && reserve_buffer(ctx, &ctx->wpack, &ctx->wpack_bytes, (size_t)w_packed) != SQ8_OK)) {
+            (void)hipGetLastError();
+            stage = repack = false;
+        }
+    }
+    pad_k = pad_k || stage;
 
     sq8::GemmArgs p;
     memset(&p, 0, sizeof(p));
@@ -359,18 +389,14 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
     }
     p.cus = ctx->cus;
     hipError_t e;
-    // [K, N] codes in place: repacked per product into the context's buffer when the repack runs near
-    // the memory bandwidth (the reference's in-place route, Artifact.swift:443-459, at the speed of
-    // the staged one: 37.7 MB of C1 codes cost ~12 µs against ~230 µs saved).
-    // The fp32 route and the residual epilogue run on the weight-direct kernels only: they repack any
-    // [K, N] weight (the general pack where the fast one does not apply).
+    // Codes in place that the weight-direct kernels do not read as they lie — [K, N] ones, [N, K] ones not aligned for
+    // 16-byte loads, a padded K (the packed layout's zero codes past k) — are repacked per product into the context's
+    // buffer at the memory's speed (the reference's in-place route, Artifact.swift:443-459, at the speed of
+    // the staged one: 37.7 MB of C1 codes cost ~12 µs against ~230 µs saved). The fp32 route and the residual epilogue
+    // run on the weight-direct kernels only.
     int wl_run = q.w_layout;
-    // A padded K takes the packed layout (its zero codes past k) whatever the weight's own layout.
-    if (!is_packed(q.w_layout) && p.a_vec && k_steps &&
-        (pad_k || (q.w_layout == SQ8_KN && (q.exact || q.residual ||
-                                            sq8::pack_is_fast(p.w, sq8::W_KN, p.ldw, q.k, q.n, is_glu(q.epilogue)))))) {
-        const int64_t bytes = sq8::packed_bytes(q.k, q.n, is_glu(q.epilogue));
-        st = reserve_buffer(ctx, &ctx->wpack, &ctx->wpack_bytes, (size_t)bytes);
+    if (p.a_vec && k_steps && (plain ? repack : !is_packed(q.w_layout) && (q.k % 64 != 0 || q.w_layout == SQ8_KN))) {
+        st = reserve_buffer(ctx, &ctx->wpack, &ctx->wpack_bytes, (size_t)w_packed);
         if (st != SQ8_OK) return st;
         e = sq8::launch_pack(p.w, q.w_layout == SQ8_KN ? sq8::W_KN : sq8::W_NK, p.ldw, q.k, q.n, is_glu(q.epilogue),
                              static_cast<uint8_t *>(ctx->wpack), ctx->stream);
@@ -378,7 +404,7 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
         p.w = static_cast<const uint8_t *>(ctx->wpack);
         wl_run = is_glu(q.epilogue) ? SQ8_PACKED_GLU : SQ8_PACKED;
     }
-    if (is_packed(wl_run) || (q.w_layout == SQ8_NK && p.a_vec && p.w_vec && k_steps && cols_per_half >= 1)) {
+    if (is_packed(wl_run) || (q.w_layout == SQ8_NK && p.a_vec && p.w_vec && q.k > 0 && q.k % 64 == 0 && cols_per_half >= 1)) {
         // The weight-direct kernels: packed codes, or [N, K] rows read as they lie.
         if (!p.a_vec || !k_steps) return SQ8_EUNSUPPORTED;  // K = 0, or an activation not 16-byte aligned
         const int wl = is_packed(wl_run) ? sq8::W_PACKED : sq8::W_NK;
@@ -407,7 +433,7 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
     } else {
         const int wl = q.w_layout == SQ8_KN ? sq8::W_KN : sq8::W_NK;
         const int tile = sq8::choose_tile(q.m, n_out, is_glu(q.epilogue), ctx->cus);
-        const bool fast = p.a_vec && p.w_vec && k_steps && cols_per_half >= 4 &&
+        const bool fast = p.a_vec && p.w_vec && q.k > 0 && q.k % 64 == 0 && cols_per_half >= 4 &&
                           (q.w_layout == SQ8_NK || (cols_per_half % 4) == 0);
         e = sq8::launch_gemm(p, fast, tile, wt, wl, q.epilogue, out, ctx->stream);
     }

@@ -13,8 +13,8 @@ namespace sq8 {
 namespace {
 
 // Scale kinds, numbered as the C ABI's sq8_dtype.
-constexpr int S_BF16 = 1, S_F32 = 2, S_F16 = 5;
-constexpr int L_TENSOR = 0, L_COLUMNS = 1, L_BLOCKS = 2, L_ROWS = 3;
+constexpr int S_BF16 = 1, S_F16 = 5;  // 2, fp32, otherwise
+constexpr int L_TENSOR = 0, L_COLUMNS = 1, L_BLOCKS = 2;  // 3, rows, otherwise
 
 __device__ __forceinline__ float scale_at(const void *s, int kind, int64_t i) {
     if (kind == S_BF16) return __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(s)[i] << 16);
@@ -52,27 +52,80 @@ __global__ void __launch_bounds__(256) round_bf16_kernel(const float *__restrict
         y[i] = (uint16_t)round_bf16(x[i]);
 }
 
-// The same rounding of `rows` rows of k values read `ldx` apart, written kp ≥ k apart with columns
-// [k, kp) zero (a strided fp32 operand into the bf16 copy the products read, padded to whole K steps).
-__global__ void __launch_bounds__(256) round_bf16_rows_kernel(const float *__restrict__ x, int64_t ldx,
-                                                              uint16_t *__restrict__ y, int64_t rows, int k, int kp) {
-    const int64_t count = rows * kp;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = i / kp;
-        const int c = (int)(i - r * kp);
-        y[i] = c < k ? (uint16_t)round_bf16(x[r * ldx + c]) : (uint16_t)0;
-    }
-}
+// The passes that write the products' operands, `rows` rows of k values read `ldx` apart, four values a thread:
+//   ROUND  fp32 → bf16, rows kp ≥ k apart with columns [k, kp) zero;
+//   COPY   bf16 as they are, padded the same way (a K of no whole 64-wide steps, an operand not aligned for 16-byte loads);
+//   SPLIT3 fp32 → three bf16 parts along K: y[r, c] = hi, y[r, kp + c] = mid, y[r, 2kp + c] = lo (columns [k, kp) of each
+//          part zero), each part the top 16 bits of what the one before leaves (hi = x truncated to bf16, mid = (x − hi)
+//          truncated, lo = x − hi − mid): 24 significant bits in three parts of 8, every difference exact, no part
+//          rounded, so hi + mid + lo = x and every product of a part with a code is exact. Every part is a normal bf16 for
+//          |x| ≥ 2^−103; an infinity or NaN is its hi part alone.
+// Memory-bound: 2^lg threads a row (up to 1024 columns a workgroup, several short rows in one), 16- or 8-byte loads where
+// the rows are aligned for them (VEC) and 8-byte stores where kp and y are (`wide`). One value a thread and a 64-bit
+// division each took 12.6 µs for SPLIT3 of 1531 × 3072 values (47 MB); this takes 10.9.
+enum RowPass { ROUND = 0, COPY = 1, SPLIT3 = 2 };
 
-// bf16 rows copied as they are, k values read `ldx` apart, written kp ≥ k apart with columns [k, kp)
-// zero: a bf16 operand whose K is not a whole number of 64-wide steps, padded for the step kernels.
-__global__ void __launch_bounds__(256) pad_bf16_rows_kernel(const uint16_t *__restrict__ x, int64_t ldx,
-                                                            uint16_t *__restrict__ y, int64_t rows, int k, int kp) {
-    const int64_t count = rows * kp;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = i / kp;
-        const int c = (int)(i - r * kp);
-        y[i] = c < k ? x[r * ldx + c] : (uint16_t)0;
+template <int PASS, bool VEC>
+__global__ void __launch_bounds__(256) row_pass_kernel(const void *__restrict__ x, int64_t ldx, uint16_t *__restrict__ y,
+                                                       int64_t rows, int lg, int per_row, int k, int kp, int wide) {
+    const uint32_t part = blockIdx.x / (uint32_t)per_row;
+    const int64_t row = ((int64_t)part << (8 - lg)) + (threadIdx.x >> lg);
+    const int c = ((int)(blockIdx.x - part * (uint32_t)per_row) * 256 + (int)(threadIdx.x & ((1u << lg) - 1))) * 4;
+    if (c >= kp || row >= rows) return;
+    const int64_t at = row * ldx + c;
+    uint32_t hi[4] = {0, 0, 0, 0}, mid[4] = {0, 0, 0, 0}, lo[4] = {0, 0, 0, 0};
+    if constexpr (PASS == COPY) {
+        const uint16_t *src = static_cast<const uint16_t *>(x) + at;
+        if (VEC && wide && c + 4 <= k) {
+            *reinterpret_cast<u32x2 *>(y + row * kp + c) = *reinterpret_cast<const u32x2 *>(src);
+            return;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (c + e < k) hi[e] = src[e];
+    } else {
+        const float *src = static_cast<const float *>(x) + at;
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (VEC && c + 4 <= k) {
+            const f32x4 t = *reinterpret_cast<const f32x4 *>(src);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = t[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (c + e < k) v[e] = src[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (PASS == ROUND) {
+                hi[e] = round_bf16(v[e]);
+            } else {
+                const uint32_t u = __float_as_uint(v[e]);
+                hi[e] = u >> 16;
+                if ((u & 0x7f800000u) != 0x7f800000u) {
+                    const float r1 = v[e] - __uint_as_float(u & 0xffff0000u);  // the low 16 bits of x: exact
+                    mid[e] = __float_as_uint(r1) >> 16;
+                    lo[e] = __float_as_uint(r1 - __uint_as_float(mid[e] << 16)) >> 16;  // ≤ 8 bits left: a bf16 value
+                }
+            }
+        }
+    }
+    auto put = [&](uint16_t *dst, const uint32_t (&d)[4]) {
+        if (wide) {
+            *reinterpret_cast<u32x2 *>(dst) = u32x2{d[0] | d[1] << 16, d[2] | d[3] << 16};
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (c + e < kp) dst[e] = (uint16_t)d[e];
+        }
+    };
+    if constexpr (PASS == SPLIT3) {
+        uint16_t *dst = y + row * 3 * kp + c;
+        put(dst, hi);
+        put(dst + kp, mid);
+        put(dst + 2 * (int64_t)kp, lo);
+    } else {
+        put(y + row * kp + c, hi);
     }
 }
 
@@ -88,46 +141,36 @@ __global__ void __launch_bounds__(256) zero_tail_kernel(uint16_t *__restrict__ y
     }
 }
 
-// fp32 → three bf16 parts along K: y[r, c] = hi, y[r, kp + c] = mid, y[r, 2kp + c] = lo (kp ≥ k; columns
-// [k, kp) of each part zero, the padding to whole K steps), each part the top 16 bits of what the one
-// before leaves (hi = x truncated to bf16, mid = (x − hi) truncated, lo = x − hi − mid): 24 significant
-// bits in three parts of 8, every difference exact, no part rounded, so hi + mid + lo = x and every
-// product of a part with a code is exact. Every part is a normal bf16 for |x| ≥ 2^−103; an infinity or
-// NaN is its hi part alone. One thread per value of row r, column c.
-__global__ void __launch_bounds__(256) split3_kernel(const float *__restrict__ x, int64_t ldx, uint16_t *__restrict__ y,
-                                                     int64_t rows, int k, int kp) {
-    const int64_t count = rows * kp;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t r = i / kp;
-        const int c = (int)(i - r * kp);
-        uint32_t u = 0, m = 0, l = 0;
-        if (c < k) {
-            const float v = x[r * ldx + c];
-            u = __float_as_uint(v);
-            if ((u & 0x7f800000u) != 0x7f800000u) {
-                const float r1 = v - __uint_as_float(u & 0xffff0000u);  // the low 16 bits of x: exact
-                m = __float_as_uint(r1) >> 16;
-                l = __float_as_uint(r1 - __uint_as_float(m << 16)) >> 16;  // ≤ 8 bits left: a bf16 value
-            }
-        }
-        uint16_t *row = y + r * 3 * (int64_t)kp;
-        row[c] = (uint16_t)(u >> 16);
-        row[kp + c] = (uint16_t)m;
-        row[2 * kp + c] = (uint16_t)l;
-    }
-}
-
 int grid_for(int64_t count) {
     const int64_t blocks = (count + 255) / 256;
     return (int)(blocks < 8192 ? (blocks > 0 ? blocks : 1) : 8192);
 }
 
-// One thread per 16-byte chunk of the packed layout: chunk c = ((slab·kt + t)·4 + j)·64 + lane holds
+// One row pass: `size` the input's bytes a value.
+template <int PASS>
+hipError_t row_pass(const void *x, int64_t ldx, int size, uint16_t *y, int64_t rows, int k, int kp, hipStream_t stream) {
+    if (rows == 0 || kp == 0) return hipSuccess;
+    int lg = 0;
+    while (lg < 8 && (4 << lg) < kp) ++lg;
+    const int64_t per_row = (kp + 1023) / 1024, blocks = ((rows + (256 >> lg) - 1) >> (8 - lg)) * per_row;
+    if (blocks > INT32_MAX) return hipErrorInvalidValue;
+    const int wide = kp % 4 == 0 && (reinterpret_cast<uintptr_t>(y) % 8) == 0;
+    const bool vec = ldx % 4 == 0 && (reinterpret_cast<uintptr_t>(x) % (4 * size)) == 0;
+    if (vec)
+        hipLaunchKernelGGL((row_pass_kernel<PASS, true>), dim3((unsigned)blocks), dim3(256), 0, stream, x, ldx, y, rows,
+                           lg, (int)per_row, k, kp, wide);
+    else
+        hipLaunchKernelGGL((row_pass_kernel<PASS, false>), dim3((unsigned)blocks), dim3(256), 0, stream, x, ldx, y, rows,
+                           lg, (int)per_row, k, kp, wide);
+    return hipGetLastError();
+}
+
+// [N, K] codes, one thread per 16-byte chunk of the packed layout: chunk c = ((slab·kt + t)·4 + j)·64 + lane holds
 // codes k ∈ [64t + 32h + 16(j&1), +16) of virtual column 32·(j>>1) + (lane & 31) of the slab
 // (h = lane >> 5); virtual columns are the weight's own, or for GLU the slab's 32 output columns of
 // the first half then the same of the second. Zeros past K and past the columns.
-__global__ void __launch_bounds__(256) pack_kernel(const uint8_t *__restrict__ w, int wl, int64_t ldw, int k, int n,
-                                                   int glu, int kt, int64_t chunks, uint8_t *__restrict__ out) {
+__global__ void __launch_bounds__(256) pack_kernel(const uint8_t *__restrict__ w, int64_t ldw, int k, int n, int glu, int kt,
+                                                   int64_t chunks, uint8_t *__restrict__ out) {
     for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < chunks; c += (int64_t)gridDim.x * blockDim.x) {
         const int lane = (int)(c & 63), j = (int)((c >> 6) & 3);
         const int64_t st = c >> 8;
@@ -145,47 +188,64 @@ __global__ void __launch_bounds__(256) pack_kernel(const uint8_t *__restrict__ w
         }
         const int k0 = 64 * t + 32 * h + 16 * (j & 1);
         u32x4 v = {0, 0, 0, 0};
-        if (valid && wl == W_NK && k0 + 16 <= k && (ldw & 15) == 0 && ((uintptr_t)w & 15) == 0) {
-            // [N, K]: the chunk is 16 contiguous codes of row `col`.
-            v = *reinterpret_cast<const u32x4 *>(w + (int64_t)col * ldw + k0);
+        if (valid && k0 + 16 <= k) {
+            // The chunk is 16 contiguous codes of row `col` (at any byte address).
+            __builtin_memcpy(&v, w + (int64_t)col * ldw + k0, 16);
         } else {
             uint32_t d[4] = {0, 0, 0, 0};
-            for (int e = 0; e < 16; ++e) {
-                const int kk = k0 + e;
-                uint32_t x = 0;
-                if (valid && kk < k) x = wl == W_KN ? w[(int64_t)kk * ldw + col] : w[(int64_t)col * ldw + kk];
-                d[e >> 2] |= x << (8 * (e & 3));
-            }
+            for (int e = 0; e < 16; ++e)
+                if (valid && k0 + e < k) d[e >> 2] |= (uint32_t)w[(int64_t)col * ldw + k0 + e] << (8 * (e & 3));
             v = u32x4{d[0], d[1], d[2], d[3]};
         }
         *reinterpret_cast<u32x4 *>(out + c * 16) = v;
     }
 }
 
-// [K, N] codes, full tiles: one workgroup per (slab, 4 K steps) — 256 rows of K × the slab's 64
+// [K, N] codes: one workgroup per (slab, 4 K steps) — 256 rows of K × the slab's 64
 // (virtual) columns. Each thread loads 4 consecutive rows × 16 columns (four 16-byte loads),
 // transposes the 4 × 16 bytes in registers into 16 words of 4 consecutive K of one column, and
 // writes them to an LDS tile [column][K]; the packed chunks (16 consecutive K of one column) are then
-// 16-byte LDS reads. Requires k % 256 == 0, whole slabs (n % 64 == 0, GLU: half % 32 == 0), ldw %
-// 16 == 0 and a 16-byte aligned base.
+// 16-byte LDS reads. WHOLE: k % 256 == 0, whole slabs (n % 64 == 0, GLU: half % 32 == 0), ldw %
+// 16 == 0 and a 16-byte aligned base; else any k, n, row stride and base: 16-byte loads at any byte address where a
+// row holds the 16 columns, single codes at the edges, zeros past them (4672 × 11563 codes 38.1 µs, 40.6 by a gather of
+// single bytes; 3072 × 12288, whole, 17.8).
 constexpr int PK_KSTEPS = 4;
 constexpr int PK_PITCH = 64 * PK_KSTEPS + 16;  // bytes per LDS column row (16-byte aligned, bank spread)
 
 __device__ __forceinline__ uint32_t byte_of(const u32x4 &v, int e) { return (v[e >> 2] >> (8 * (e & 3))) & 0xFF; }
 
-__global__ void __launch_bounds__(256) pack_kn_kernel(const uint8_t *__restrict__ w, int64_t ldw, int n, int glu, int kt,
+template <bool WHOLE>
+__global__ void __launch_bounds__(256) pack_kn_kernel(const uint8_t *__restrict__ w, int64_t ldw, int k, int n, int glu, int kt,
                                                       uint8_t *__restrict__ out) {
     __shared__ __attribute__((aligned(16))) uint8_t tile[64 * PK_PITCH];
-    const int groups = kt / PK_KSTEPS;
+    const int groups = (kt + PK_KSTEPS - 1) / PK_KSTEPS;
     const int slab = blockIdx.x / groups, tq = blockIdx.x - slab * groups;
     const int tid = threadIdx.x;
     const int seg = tid & 3, kq = tid >> 2;  // columns [16·seg, +16) of the slab, rows 4·kq .. 4·kq + 3
     const int vc0 = 16 * seg, b = vc0 >> 5;
-    const int col0 = glu ? slab * 32 + (vc0 & 31) + b * (n / 2) : slab * 64 + vc0;
-    const uint8_t *src = w + (int64_t)(tq * 64 * PK_KSTEPS + 4 * kq) * ldw + col0;
+    const int oc0 = glu ? slab * 32 + (vc0 & 31) : slab * 64 + vc0;
+    const int left = (glu ? n / 2 : n) - oc0;  // columns of this half from oc0 on
+    const int col0 = glu ? oc0 + b * (n / 2) : oc0;
+    const int row0 = tq * 64 * PK_KSTEPS + 4 * kq;
     u32x4 r[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = *reinterpret_cast<const u32x4 *>(src + i * ldw);
+    for (int i = 0; i < 4; ++i) {
+        const uint8_t *src = w + (int64_t)(row0 + i) * ldw + col0;
+        if constexpr (WHOLE) {
+            r[i] = *reinterpret_cast<const u32x4 *>(src);
+        } else {
+            r[i] = u32x4{0, 0, 0, 0};
+            if (row0 + i < k) {
+                if (left >= 16) {
+                    __builtin_memcpy(&r[i], src, 16);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        if (e < left) r[i][e >> 2] |= (uint32_t)src[e] << (8 * (e & 3));
+                }
+            }
+        }
+    }
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
         const uint32_t word = byte_of(r[0], e) | byte_of(r[1], e) << 8 | byte_of(r[2], e) << 16 | byte_of(r[3], e) << 24;
@@ -201,7 +261,7 @@ __global__ void __launch_bounds__(256) pack_kn_kernel(const uint8_t *__restrict_
         const int kr = 64 * ts + 32 * (lane >> 5) + 16 * (j & 1);
         const u32x4 v = *reinterpret_cast<const u32x4 *>(tile + vc * PK_PITCH + kr);
         const int t = tq * PK_KSTEPS + ts;
-        *reinterpret_cast<u32x4 *>(out + (((int64_t)slab * kt + t) * 4 + j) * 1024 + lane * 16) = v;
+        if (WHOLE || t < kt) *reinterpret_cast<u32x4 *>(out + (((int64_t)slab * kt + t) * 4 + j) * 1024 + lane * 16) = v;
     }
 }
 
@@ -213,24 +273,22 @@ int64_t packed_bytes(int k, int n, bool glu) {
     return slabs * kt * 4096;
 }
 
-bool pack_is_fast(const uint8_t *w, int wl, int64_t ldw, int k, int n, bool glu) {
-    const bool whole_slabs = glu ? (n % 2 == 0 && (n / 2) % 32 == 0) : n % 64 == 0;
-    return wl == W_KN && k > 0 && k % (64 * PK_KSTEPS) == 0 && n > 0 && whole_slabs && ldw % 16 == 0 &&
-           ((uintptr_t)w & 15) == 0;
-}
-
 hipError_t launch_pack(const uint8_t *w, int wl, int64_t ldw, int k, int n, bool glu, uint8_t *out, hipStream_t stream) {
     const int kt = (k + 63) / 64;
     const int64_t chunks = packed_bytes(k, n, glu) / 16;
     if (chunks == 0) return hipSuccess;
-    if (pack_is_fast(w, wl, ldw, k, n, glu)) {
-        const int64_t slabs = glu ? (n / 2) / 32 : n / 64;
-        hipLaunchKernelGGL(pack_kn_kernel, dim3((unsigned)(slabs * (kt / PK_KSTEPS))), dim3(256), 0, stream, w, ldw, n,
-                           glu ? 1 : 0, kt, out);
+    if (wl == W_KN) {
+        const bool whole = k % (64 * PK_KSTEPS) == 0 && (glu ? (n / 2) % 32 == 0 : n % 64 == 0) && ldw % 16 == 0 &&
+                           ((uintptr_t)w & 15) == 0;
+        const int64_t slabs = packed_bytes(k, n, glu) / ((int64_t)kt * 4096);
+        const dim3 grid((unsigned)(slabs * ((kt + PK_KSTEPS - 1) / PK_KSTEPS)));
+        if (whole)
+            hipLaunchKernelGGL(pack_kn_kernel<true>, grid, dim3(256), 0, stream, w, ldw, k, n, glu ? 1 : 0, kt, out);
+        else
+            hipLaunchKernelGGL(pack_kn_kernel<false>, grid, dim3(256), 0, stream, w, ldw, k, n, glu ? 1 : 0, kt, out);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(pack_kernel, dim3(grid_for(chunks)), dim3(256), 0, stream, w, wl, ldw, k, n, glu ? 1 : 0, kt,
-                       chunks, out);
+    hipLaunchKernelGGL(pack_kernel, dim3(grid_for(chunks)), dim3(256), 0, stream, w, ldw, k, n, glu ? 1 : 0, kt, chunks, out);
     return hipGetLastError();
 }
 
@@ -249,10 +307,7 @@ hipError_t launch_dequantize(const uint8_t *codes, int wt, int64_t rows, int64_t
 }
 
 hipError_t launch_split3(const float *x, int64_t ldx, uint16_t *y, int64_t rows, int k, int kp, hipStream_t stream) {
-    const int64_t count = rows * kp;
-    if (count == 0) return hipSuccess;
-    hipLaunchKernelGGL(split3_kernel, dim3(grid_for(count)), dim3(256), 0, stream, x, ldx, y, rows, k, kp);
-    return hipGetLastError();
+    return row_pass<SPLIT3>(x, ldx, 4, y, rows, k, kp, stream);
 }
 
 hipError_t launch_round_bf16(const float *x, uint16_t *y, int64_t count, hipStream_t stream) {
@@ -263,17 +318,12 @@ hipError_t launch_round_bf16(const float *x, uint16_t *y, int64_t count, hipStre
 
 hipError_t launch_round_bf16_rows(const float *x, int64_t ldx, uint16_t *y, int64_t rows, int k, int kp,
                                   hipStream_t stream) {
-    if (rows == 0 || kp == 0) return hipSuccess;
-    if (ldx == k && kp == k) return launch_round_bf16(x, y, rows * k, stream);
-    hipLaunchKernelGGL(round_bf16_rows_kernel, dim3(grid_for(rows * kp)), dim3(256), 0, stream, x, ldx, y, rows, k, kp);
-    return hipGetLastError();
+    return row_pass<ROUND>(x, ldx, 4, y, rows, k, kp, stream);
 }
 
 hipError_t launch_pad_bf16_rows(const uint16_t *x, int64_t ldx, uint16_t *y, int64_t rows, int k, int kp,
                                 hipStream_t stream) {
-    if (rows == 0 || kp == 0) return hipSuccess;
-    hipLaunchKernelGGL(pad_bf16_rows_kernel, dim3(grid_for(rows * kp)), dim3(256), 0, stream, x, ldx, y, rows, k, kp);
-    return hipGetLastError();
+    return row_pass<COPY>(x, ldx, 2, y, rows, k, kp, stream);
 }
 
 hipError_t launch_zero_tail(uint16_t *y, int64_t ld, int64_t rows, int k, int kp, hipStream_t stream) {
