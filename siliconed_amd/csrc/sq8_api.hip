@@ -581,7 +581,7 @@ int run_w8a8(sq8_ctx *ctx, const W8A8 &q, double *gpu_seconds) {
         p.w = static_cast<const uint8_t *>(ctx->wpack);
         p.kt_w = (q.k + 63) / 64;
     }
-    int tile = ctx->i8_tile >= 0 ? ctx->i8_tile : sq8::choose_i8_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, p.kt);
+    int tile = ctx->i8_tile >= 0 ? ctx->i8_tile : sq8::choose_i8_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, p.kt, q.residual);
     if (tile >= sq8::GROUP_TILE0 && !group_serves(tile, sq8::GM_I8, is_glu(q.epilogue))) tile = sq8::I8_128x256;
     e = sq8::launch_i8gemm(p, tile, wl, q.residual ? sq8::EPI_RESIDUAL : q.epilogue,
                            q.c_dtype == SQ8_F32 ? sq8::OUT_F32 : sq8::OUT_BF16, ctx->stream);

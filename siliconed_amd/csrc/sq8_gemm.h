@@ -183,7 +183,7 @@ hipError_t launch_pad_codes(const int8_t *src, int64_t ld_src, int8_t *dst, int6
                             hipStream_t stream);
 // `tile`: choose_i8_tile's: I8_128x256 (128 × 256, two workgroups a CU) or a K-group tile's id. kt: K steps of 128.
 constexpr int I8_128x256 = 0;
-int choose_i8_tile(int M, int N, bool glu, int cus, int kt);
+int choose_i8_tile(int M, int N, bool glu, int cus, int kt, bool residual);
 hipError_t launch_i8gemm(const GemmArgs &p, int tile, int wl, int epi, int out, hipStream_t stream);
 
 // The DiT block's elementwise passes (sq8_block.hip).

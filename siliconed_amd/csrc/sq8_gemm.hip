@@ -79,17 +79,18 @@ static float pairs_us(float tiles, int cus, float two, float one) {
 }
 
 // Calls take(tile, µs) for every K-group shape that serves M rows × `blocks` 32-column blocks of weight and `steps` weight K
-// steps (unrolled: each shape's divisions are by constants; the rule runs on every call).
+// steps (unrolled: each shape's divisions are by constants; the rule runs on every call); `value_us`: further µs a value of
+// the tile.
 template <int MATH, int I = 0, typename F>
-static inline void each_group(int M, int blocks, bool glu, int cus, int steps, F &&take) {
+static inline void each_group(int M, int blocks, bool glu, int cus, int steps, float value_us, F &&take) {
     if constexpr (I < kGroupShapes) {
         constexpr GroupShape g = group_shapes[I];
         constexpr GroupCost c = g.cost[MATH];
         constexpr int nw = g.cols / 32;
         // bf16: four groups give the skinny kernel's bits at any K, two the 64 × 128 tiles' where the steps divide.
         if (c.us_step > 0.0f && !(glu && nw % 2 != 0) && !(MATH == GM_BF16 && steps % 2 != 0 && g.groups == 2))
-            take(GROUP_TILE0 + I, rounds_us(tile_count(M, g.rows, blocks, nw), cus, c.us + c.us_step * (float)steps));
-        each_group<MATH, I + 1>(M, blocks, glu, cus, steps, take);
+            take(GROUP_TILE0 + I, rounds_us(tile_count(M, g.rows, blocks, nw), cus, c.us + c.us_step * (float)steps + value_us * (float)(g.rows * g.cols)));
+        each_group<MATH, I + 1>(M, blocks, glu, cus, steps, value_us, take);
     }
 }
 
@@ -137,25 +138,29 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32, bool w2
         take(WD_224, rounds_us(tiles(224), cus, us(r224)));
     }
     if (f32)
-        each_group<GM_F32>(M, blocks, glu, cus, steps, take);
+        each_group<GM_F32>(M, blocks, glu, cus, steps, 0.0f, take);
     else
-        each_group<GM_BF16>(M, blocks, glu, cus, steps, take);
+        each_group<GM_BF16>(M, blocks, glu, cus, steps, 0.0f, take);
     return tile;
 }
 
-int choose_i8_tile(int M, int N, bool glu, int cus, int kt) {
+int choose_i8_tile(int M, int N, bool glu, int cus, int kt, bool residual) {
     // The tile of the least estimated time. Every tile gives the same bits (int32 sums), so only time decides; the
     // 128 × 256 kernel's rounds (two workgroups a CU: 11.2 + 1.70 µs a K step; one: 9.6 + 0.91) are measured as the
     // K-group tiles' (GroupShape). It has the least operand traffic per output and wins where its tiles fill the
     // chip (K = 3072: 4096 × 12288 150 µs against 203 in 128 × 192); with fewer the K-group tiles spread the work
     // over more CUs and hold more loads in flight a CU. Measured, K = 3072, product alone, µs, 128 × 256 tiles
     // against the rule's: 1 × 3072 20.8 → 4.9, 77 × 12288 22.6 → 12.9, 512 × 3072 23.0 → 10.8, 1021 × 3072 24.5 →
-    // 17.0, 333 × 9216 25.0 → 20.0; K = 12288, 68 × 512 62.9 → 9.7.
+    // 17.0, 333 × 9216 25.0 → 20.0; K = 12288, 68 × 512 62.9 → 9.7. The residual epilogue reads and writes 8 bytes a value
+    // past the sums, a round's at the CU's share of the memory's rate (0.4 ns a value) where one workgroup fills the CU,
+    // half of that under the other's K steps where two do: 3742 × 3072 × 3072 62.9 µs in 128 × 256 and 71.3 in 128 × 192
+    // tiles, at K = 12288 163 and 159.
     if (cus <= 0) cus = 256;
     const int blocks = glu ? 2 * ((N / 2 + 31) / 32) : (N + 31) / 32;  // 32-column blocks
-    float best = pairs_us(tile_count(M, 128, blocks, 8), cus, 11.2f + 1.70f * (float)kt, 9.6f + 0.91f * (float)kt);
+    const float two = residual ? 22.2f : 11.2f, one = residual ? 15.6f : 9.6f;
+    float best = pairs_us(tile_count(M, 128, blocks, 8), cus, two + 1.70f * (float)kt, one + 0.91f * (float)kt);
     int tile = I8_128x256;
-    each_group<GM_I8>(M, blocks, glu, cus, kt, [&](int t, float time) {
+    each_group<GM_I8>(M, blocks, glu, cus, kt, residual ? 4e-4f : 0.0f, [&](int t, float time) {
         if (time < best) {
             best = time;
             tile = t;
