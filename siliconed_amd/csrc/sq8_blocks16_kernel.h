@@ -217,7 +217,7 @@ gemm_blocks16_kernel(const GemmArgs p) {
             for (int e = 0; e < 4; ++e) u[e] = has_bias ? __fadd_rn(y[e], bu[e]) : y[e];
         }
         grp::activate4(p.epi, v, u);
-        grp::store4(p, m, col, n_out, v);
+        grp::store4(p, grp::out4(p, col, n_out), m * grp::row_bytes(p), col, n_out, v);
     }
 }
 

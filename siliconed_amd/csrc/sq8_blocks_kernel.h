@@ -245,6 +245,8 @@ gemm_blocks_kernel(const GemmArgs p) {
     const int chunk = tid % per_row;
     const int col = tn * cols + 4 * chunk, blk = chunk >> 3;   // blk: the 32-column output block
     const bool has_bias = p.bias != nullptr;
+    const grp::Out4 to = grp::out4(p, min(col, n_out - 1), n_out);
+    const int64_t row_bytes = grp::row_bytes(p);
     float bi[4], bu[4];
     if (col < n_out) {
         grp::column4(p.bias, true, p.sb_vec, col, n_out, 0, bi);
@@ -272,7 +274,7 @@ gemm_blocks_kernel(const GemmArgs p) {
                     for (int e = 0; e < 4; ++e) u[e] = has_bias ? __fadd_rn(y[e], bu[e]) : y[e];
                 }
                 grp::activate4(p.epi, v, u);
-                grp::store4(p, m, col, n_out, v);
+                grp::store4(p, to, m * row_bytes, col, n_out, v);
             }
         }
         if constexpr (bm + 1 < FM) __syncthreads();

@@ -76,6 +76,11 @@ __device__ __forceinline__ Out4 out4(const GemmArgs &p, int col, int n_out) {
     return o;
 }
 
+// Bytes from one output row to the next.
+__device__ __forceinline__ int64_t row_bytes(const GemmArgs &p) {
+    return p.epi == EPI_RESIDUAL ? p.ldc * 4 : (p.head_dim > 0 ? p.head_dim : p.ldc) * (p.out == OUT_F32 ? 4 : 2);
+}
+
 // Stores the values v (scaled, biased, activated) of columns [col, col + 4), `row` bytes past their rows 0.
 __device__ __forceinline__ void store4(const GemmArgs &p, const Out4 &o, int64_t row, int col, int n_out, const float (&v)[4]) {
     if (p.epi == EPI_RESIDUAL) {
@@ -412,7 +417,7 @@ gemm_group_kernel(const GemmArgs p) {
         }
     }
     const bool has_bias = p.bias != nullptr;
-    const int64_t row_bytes = p.epi == EPI_RESIDUAL ? p.ldc * 4 : (p.head_dim > 0 ? p.head_dim : p.ldc) * (p.out == OUT_F32 ? 4 : 2);
+    const int64_t row_stride = row_bytes(p);
     static_for<0, FM>([&](auto bmc) {
         constexpr int bm = decltype(bmc)::value;
         uint8_t *dst = lds + wave_all * SLOT + (lane & 31) * PITCH + 16 * h;
@@ -455,7 +460,7 @@ gemm_group_kernel(const GemmArgs p) {
                     }
                 }
                 activate4(p.epi, v, u);
-                store4(p, to[i], m * row_bytes, col[i], n_out, v);
+                store4(p, to[i], m * row_stride, col[i], n_out, v);
             }
         }
         if constexpr (bm + 1 < FM) __syncthreads();
