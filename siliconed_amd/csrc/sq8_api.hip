@@ -410,8 +410,7 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
         const int wl = is_packed(wl_run) ? sq8::W_PACKED : sq8::W_NK;
         const int steps = q.exact ? p.kt_w : p.kt;
         const int tile = ctx->wd_tile >= 0 ? wd_knob_tile(ctx->wd_tile, is_glu(q.epilogue), steps, q.exact)
-                                           : sq8::choose_wd_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, steps, q.exact,
-                                                                 sq8::w256_fits(p, epi, out));
+                                           : sq8::choose_wd_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, steps, q.exact);
         if ((tile == sq8::WD_SKINNY32 || tile == sq8::WD_SKINNY64) && ctx->splits > 1) {
             // Short M with the SQ8_SPLITS knob: the K steps split over several workgroups per tile, partial
             // sums in the context's buffer, added in split order by a second launch. Not the default: the

@@ -59,20 +59,8 @@ hipError_t launch_gemm(const GemmArgs &p, bool fast, int tile, int wt, int wl, i
 enum WdTile { WD_256 = 0, WD_128 = 1, WD_SKINNY64 = 2, WD_SKINNY32 = 3, WD_64 = 4, WD_32 = 5, WD_224 = 6, WD_64N = 7, WD_64x192 = 8,
               WD_GEMV = 9 };
 // The tile for an M × N product (GLU: N = 2h) of `steps` weight K steps of 64, `f32` on the fp32 route (three parts of
-// an fp32 activation), `w256`: the 256-row kernel serves it (w256_fits).
-int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32, bool w256);
-// True when the 256- and 224-row kernel runs this product: whole 64-column slabs (GLU: whole 32-column
-// slabs of each half) and 16-byte scale/bias loads; for the slab epilogue (bf16 out, no activation or
-// GELU) also slabs that each lie in one output (and one head) and 16-byte stores. The fp32 route's three
-// parts along K (kt_w > 0) face the weight's steps in turn (weight_step).
-inline bool w256_fits(const GemmArgs &p, int epi, int out) {
-    if (!p.sb_vec) return false;
-    if (p.glu_half > 0 ? p.glu_half % 32 != 0 : p.N % 64 != 0) return false;
-    if (epi == EPI_RESIDUAL && out != OUT_F32) return false;
-    if ((epi == EPI_NONE || epi == EPI_GELU) && out == OUT_BF16)
-        return p.split % 64 == 0 && p.head_dim % 64 == 0 && p.c_vec16;
-    return true;
-}
+// an fp32 activation): by the shape alone, so that a call's bits depend on nothing else.
+int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32);
 // The short-M kernel (sq8_gemv_kernel.h): the activation staged in LDS (M rows of K' = kt · 64 bf16, rows
 // gemv_xpitch bytes apart: 16 more than a row, so the 16 rows a fragment read touches start on different banks)
 // when it fits GEMV_XLDS bytes and each row is whole 1 KB runs (K' a multiple of 512), the unit of a direct load.

@@ -94,7 +94,7 @@ static inline void each_group(int M, int blocks, bool glu, int cus, int steps, f
     }
 }
 
-int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32, bool w256) {
+int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
     if (cus <= 0) cus = 256;
     const int kt = f32 ? 3 * steps : steps;  // the activation's K steps
     // Up to 16 rows, the 16-column groups of the short-M kernel where they fit one round of one or two groups a
@@ -133,10 +133,17 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32, bool w2
             tile = t;
         }
     };
-    if (w256) {
+    // By the shape alone: the 256- and 224-row kernel also wants its scales and outputs aligned, but a choice by alignment
+    // or output type would give one call two sets of bits (launch_wdirect takes 128-row tiles, the same sums, where that
+    // kernel cannot serve the product).
+    if (glu ? N / 2 % 32 == 0 : N % 64 == 0) {
         take(WD_256, rounds_us(tiles(256), cus, us(r256)));
         take(WD_224, rounds_us(tiles(224), cus, us(r224)));
     }
+    // From 4096 rows on and past 1024 columns no K groups: the tall tiles sum each output's K in one sequence, so a host that
+    // chunks its rows by that many gets the bits of one call. What it costs where 128 × 192 tiles of two groups would fill
+    // the rounds better (µs): 5760 × 3072 × 3072 115.9 → 119.9, with the residual 124.6 → 141.8, fp32 route 309 → 375.
+    if (M >= 4096 && N > 1024) return tile;
     if (f32)
         each_group<GM_F32>(M, blocks, glu, cus, steps, 0.0f, take);
     else

@@ -317,6 +317,19 @@ gemm_w256_kernel(const GemmArgs p) {
     }
 }
 
+// True when the 256- and 224-row kernel runs this product: whole 64-column slabs (GLU: whole 32-column
+// slabs of each half) and 16-byte scale/bias loads; for the slab epilogue (bf16 out, no activation or
+// GELU) also slabs that each lie in one output (and one head) and 16-byte stores. The fp32 route's three
+// parts along K (kt_w > 0) face the weight's steps in turn (weight_step).
+inline bool w256_fits(const GemmArgs &p, int epi, int out) {
+    if (!p.sb_vec) return false;
+    if (p.glu_half > 0 ? p.glu_half % 32 != 0 : p.N % 64 != 0) return false;
+    if (epi == EPI_RESIDUAL && out != OUT_F32) return false;
+    if ((epi == EPI_NONE || epi == EPI_GELU) && out == OUT_BF16)
+        return p.split % 64 == 0 && p.head_dim % 64 == 0 && p.c_vec16;
+    return true;
+}
+
 template <int WT, int WL, int BM = 256>
 hipError_t launch_w256(const GemmArgs &args, int epi, int out, hipStream_t stream) {
     GemmArgs p = args;

@@ -16,7 +16,7 @@ hipError_t SQ8_CAT(launch_wdirect_, SQ8_CAT(SQ8_WT, SQ8_CAT(_, SQ8_WL)))(const G
     // 256 × 256 or 224 × 256 tiles where their kernel serves the product (whole slabs, aligned scales and
     // biases); else the two-workgroup 128-row tiles.
     if (tile == WD_256 || tile == WD_224) {
-        if (w256_fits(p, epi, out))
+        if (wd::w256_fits(p, epi, out))
             return tile == WD_256 ? wd::launch_w256<SQ8_WT, SQ8_WL, 256>(p, epi, out, stream)
                                   : wd::launch_w256<SQ8_WT, SQ8_WL, 224>(p, epi, out, stream);
         tile = WD_128;

@@ -55,3 +55,44 @@ def test_default_tile_matches_a_fixed_tile(gemm, orc, tile_gemm, i):
     assert any(bitwise_equal(ys["default"], ys[t]) == 0 for t in ("128", "s32", "gemv", "k32x32", "k64x128"))
     if m >= 31:
         judge(orc, ys["default"], x, q, fp8, s, b, epi, out, rows=orc.sample_rows(m, 32))
+
+
+def _random_operands(m, k, n, f32, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn((m, k), device="cuda", generator=g)
+    q = torch.randint(-127, 128, (n, k), device="cuda", generator=g, dtype=torch.int8)
+    s = torch.rand(n, device="cuda", generator=g) * 1e-2 + 1e-3
+    return x if f32 else x.bfloat16(), q, s, torch.randn(n, device="cuda", generator=g)
+
+
+@pytest.mark.parametrize("route,k,n,chunks", [
+    ("bf16", 1024, 3840, (4608, 4608)), ("bf16", 3072, 3072, (5760, 4096)), ("bf16", 320, 1088, (4100, 5377)),
+    ("fp32", 1024, 3072, (4096, 7168))])
+def test_chunks_of_4096_rows_have_one_calls_bits(gemm, route, k, n, chunks):
+    """A host's row chunks of 4096 or more give the bits of the one call over all rows (past 1024 columns)."""
+    x, q, s, b = _random_operands(sum(chunks), k, n, route == "fp32", n + k)
+    w = gemm.pack(q, layout="nk")
+    run = lambda rows: gemm.product(rows, w, s, bias=b, out_dtype=torch.float32, rounding=route == "bf16")
+    whole = run(x)
+    parts = torch.cat([run(rows) for rows in x.split(chunks)])
+    torch.cuda.synchronize()
+    assert torch.equal(whole, parts)
+
+
+@pytest.mark.parametrize("route,m,k,n", [("bf16", 2737, 3072, 3072), ("bf16", 1088, 3072, 9216), ("bf16", 333, 1024, 3072),
+                                         ("fp32", 1282, 3072, 9216)])
+def test_bits_do_not_depend_on_alignment_or_output_type(gemm, route, m, k, n):
+    """The order of sums is the shape's alone: outputs, scales and biases off the 16-byte grid, and a bf16 output, round
+    the same sums."""
+    x, q, s, b = _random_operands(m, k, n, route == "fp32", n + k)
+    w = gemm.pack(q, layout="nk")
+    off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+    run = lambda s, b, out: gemm.product(x, w, s, bias=b, out=out, rounding=route == "bf16")
+    want = run(s, b, torch.empty((m, n), device="cuda"))
+    plain = run(s, b, torch.empty((m, n), device="cuda", dtype=torch.bfloat16))
+    for dtype in (torch.float32, torch.bfloat16):
+        for ss, bb in ((s, b), (off(s), off(b))):
+            y = run(ss, bb, off(torch.zeros((m, n), device="cuda", dtype=dtype)))
+            torch.cuda.synchronize()
+            assert torch.equal(y, want if dtype == torch.float32 else plain)
+    assert torch.equal(want.bfloat16(), plain)
