@@ -127,8 +127,11 @@ int sq8_supports(const sq8_ctx *ctx, int a_dtype, int w_dtype, int w_layout, int
  * are split over several workgroups (added by a second launch) — are sized by the largest product so far; a call that needs
  * more first synchronizes the context's stream (queued work may still read the old buffer), frees
  * and allocates. A caller that must never block runs one product of its largest shape first. Under stream capture a
- * buffer cannot grow, and ragged or unaligned operands run on the kernels that read them as they lie, several times
- * slower.
+ * buffer cannot grow: a captured call needs it as large before (one eager call of its shape), except that ragged or
+ * unaligned operands in place then run on the kernels that read them as they lie, several times slower and with K
+ * summed in their own order. Memory that a captured call used is kept when its buffer grows later, and freed by
+ * sq8_destroy, which no such graph may outlive; its replays use the context's buffers as a call does, so the caller
+ * orders them with the context's other work.
  * Replaces: TensorGEMM.linear(a:int8:weightOffset:scales:scalesOffset:perColumn:block:rotation:
  * rounding:quantizing:prequantized:c:m:k:n:settled:) -> Double (TensorGEMM.swift:264-290) and
  * its encoders submit (:296-360) / submitRounded (TensorGEMMBF16.swift:208-264), with the bias

@@ -14,6 +14,7 @@
 #include <mutex>
 #include <new>
 
+#include "sq8_buffers.h"
 #include "sq8_gemm.h"
 
 // The allocation-free entry point's device memory (sq8_linear_quantized_static): one array per GPU,
@@ -26,12 +27,10 @@ struct sq8_ctx {
     int device;
     hipStream_t stream;
     hipEvent_t begin, end;
-    void *scratch;          // bf16 copy of an fp32 activation (the reference's rounding scratch)
-    size_t scratch_bytes;
-    void *wpack;            // [K, N] codes repacked for the weight-direct kernels, per product
-    size_t wpack_bytes;
-    void *part;             // the skinny kernel's partial sums of a K split
-    size_t part_bytes;
+    sq8::Buffer scratch;    // bf16 copy of an fp32 activation (the reference's rounding scratch)
+    sq8::Buffer wpack;      // [K, N] codes repacked for the weight-direct kernels, per product
+    sq8::Buffer part;       // the skinny kernel's partial sums of a K split
+    sq8::SetAside *aside;   // what these outgrew while a captured graph may use it
     rocblas_handle blas;    // the bf16-weight product's library GEMM (created on its first call)
     int wd_tile;            // measurement knobs, read once at sq8_create (SQ8_TILE, SQ8_Q8_TILE, SQ8_SPLITS): a
     int q8_tile;            // forced weight-direct / block-scale tile, or -1 (the product's own choice); the
@@ -136,45 +135,9 @@ int check_config(int a_dtype, int w_dtype, int w_layout, int scale_layout, int c
     return SQ8_OK;
 }
 
-// Grows the rounding scratch to `bytes` (never shrinks; freed with the context).
-// Grows a context buffer (after the stream has finished with the old one).
-int reserve_buffer(sq8_ctx *ctx, void **buf, size_t *have, size_t bytes) {
-    if (*have >= bytes) return SQ8_OK;
-    hipError_t e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) return hip_status(e);
-    if (*buf) (void)hipFree(*buf);
-    *buf = nullptr;
-    *have = 0;
-    e = hipMalloc(buf, bytes);
-    if (e != hipSuccess) { *buf = nullptr; return hip_status(e); }
-    *have = bytes;
-    return SQ8_OK;
-}
-
-int reserve_scratch(sq8_ctx *ctx, size_t bytes) {
-    if (ctx->scratch_bytes >= bytes) return SQ8_OK;
-    if (ctx->scratch) {
-        hipError_t e = hipStreamSynchronize(ctx->stream);
-        if (e != hipSuccess) return hip_status(e);
-        e = hipFree(ctx->scratch);
-        ctx->scratch = nullptr;
-        ctx->scratch_bytes = 0;
-        if (e != hipSuccess) return hip_status(e);
-    }
-    hipError_t e = hipMalloc(&ctx->scratch, bytes);
-    if (e != hipSuccess) {
-        ctx->scratch = nullptr;
-        return hip_status(e);
-    }
-    ctx->scratch_bytes = bytes;
-    return SQ8_OK;
-}
-
-// Whether the context's stream is being captured into a graph (the growable buffers may not grow then: that synchronizes
-// and allocates).
-bool capturing(const sq8_ctx *ctx) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(ctx->stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
+// Grows one of the context's buffers to `bytes` (never shrinks; freed with the context).
+int reserve(sq8_ctx *ctx, sq8::Buffer &b, size_t bytes) {
+    return hip_status(sq8::reserve(b, bytes, ctx->stream, ctx->aside));
 }
 
 struct Product {
@@ -196,14 +159,14 @@ int stage_parts(sq8_ctx *ctx, const float *a, int64_t lda, int group, int m, int
     const size_t mk = (size_t)m * (size_t)k;
     const size_t parts = (size_t)m * (size_t)kp * 6;
     const size_t bytes = parts + (group != 0 ? mk * 4 : 0);
-    int st = reserve_scratch(ctx, bytes > 0 ? bytes : 2);
+    int st = reserve(ctx, ctx->scratch, bytes > 0 ? bytes : 2);
     if (st != SQ8_OK) return st;
-    uint16_t *y = static_cast<uint16_t *>(ctx->scratch);
+    uint16_t *y = static_cast<uint16_t *>(ctx->scratch.at);
     const float *src = a;
     int64_t lds = lda;
     if (group != 0) {
         // m·kp·6 bytes in: a multiple of 4 as kp is even.
-        float *r = reinterpret_cast<float *>(static_cast<uint8_t *>(ctx->scratch) + parts);
+        float *r = reinterpret_cast<float *>(static_cast<uint8_t *>(ctx->scratch.at) + parts);
         hipError_t e = sq8::launch_rotate_groups(a, false, lda, r, false, k, m, k, group, ctx->stream);
         if (e != hipSuccess) return hip_status(e);
         src = r;
@@ -220,9 +183,9 @@ int stage_parts(sq8_ctx *ctx, const float *a, int64_t lda, int group, int m, int
 // weight's zero codes past K: every sum as over k alone).
 int stage_padded_bf16(sq8_ctx *ctx, const uint16_t *a, int64_t lda, int m, int k, int kp, const uint16_t **out) {
     const size_t bytes = (size_t)m * (size_t)kp * 2;
-    int st = reserve_scratch(ctx, bytes > 0 ? bytes : 2);
+    int st = reserve(ctx, ctx->scratch, bytes > 0 ? bytes : 2);
     if (st != SQ8_OK) return st;
-    uint16_t *y = static_cast<uint16_t *>(ctx->scratch);
+    uint16_t *y = static_cast<uint16_t *>(ctx->scratch.at);
     hipError_t e = sq8::launch_pad_bf16_rows(a, lda, y, m, k, kp, ctx->stream);
     if (e != hipSuccess) return hip_status(e);
     *out = y;
@@ -266,19 +229,20 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
     // takes 51 µs so and took 372 in the guarded kernel, 7 × 2152 × 1873 14 and 121, 512 × 1000 × 3072 17 and 69 ([N, K]
     // the same within 2 µs).
     // The guarded and LDS-transposing kernels (launch_gemm) keep what 32-bit offsets do not reach once padded, what
-    // there is no memory to stage, and what is captured into a graph: a buffer that a later product grows is freed, and
-    // the graph would go on reading it. (Whole [K, N] slabs are repacked in a graph too, where the buffer holds them.)
+    // there is no memory to stage, and what is captured into a graph: the buffers may not grow then, and a replay on
+    // another stream that used them would race with the context's eager products. (Whole [K, N] slabs are repacked in a
+    // graph too, where the buffer holds them: the caller orders those replays.)
     const bool plain = !is_packed(q.w_layout) && !q.exact && !q.residual && q.k > 0;
     const bool w_aligned = aligned(q.w, 16) && q.ldw % 16 == 0;
     bool stage = plain && (q.k % 64 != 0 || (q.a_dtype == SQ8_BF16 && q.group == 0 && !(aligned(q.a, 16) && q.lda % 8 == 0)));
     bool repack = plain && (q.w_layout == SQ8_KN || !w_aligned || q.k % 64 != 0);
-    if ((stage || repack) && capturing(ctx)) {
-        repack = q.w_layout == SQ8_KN && w_aligned && q.k % 256 == 0 && q.n % 64 == 0 && ctx->wpack_bytes >= (size_t)w_packed;
+    if ((stage || repack) && sq8::capturing(ctx->stream)) {
+        repack = q.w_layout == SQ8_KN && w_aligned && q.k % 256 == 0 && q.n % 64 == 0 && ctx->wpack.bytes >= (size_t)w_packed;
         stage = false;
     } else if (stage || repack) {
         const int64_t bytes = (int64_t)q.m * kp * 2;
-        if ((stage && (bytes > (int64_t)UINT32_MAX || reserve_scratch(ctx, (size_t)bytes) != SQ8_OK)) ||
-            (repack && reserve_buffer(ctx, &ctx->wpack, &ctx->wpack_bytes, (size_t)w_packed) != SQ8_OK)) {
+        if ((stage && (bytes > (int64_t)UINT32_MAX || reserve(ctx, ctx->scratch, (size_t)bytes) != SQ8_OK)) ||
+            (repack && reserve(ctx, ctx->wpack, (size_t)w_packed) != SQ8_OK)) {
             (void)hipGetLastError();
             stage = repack = false;
         }
@@ -307,9 +271,9 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
         // with zero columns past k when K is padded.
         const int ky = pad_k ? kp : q.k;
         const size_t bytes = (size_t)q.m * (size_t)ky * 2;
-        st = reserve_scratch(ctx, bytes > 0 ? bytes : 2);
+        st = reserve(ctx, ctx->scratch, bytes > 0 ? bytes : 2);
         if (st != SQ8_OK) return st;
-        uint16_t *y = static_cast<uint16_t *>(ctx->scratch);
+        uint16_t *y = static_cast<uint16_t *>(ctx->scratch.at);
         hipError_t e = sq8::launch_rotate_groups(q.a, q.a_dtype == SQ8_BF16, q.lda, y, true, ky, q.m, q.k, q.group,
                                                  ctx->stream);
         if (e == hipSuccess) e = sq8::launch_zero_tail(y, ky, q.m, q.k, ky, ctx->stream);
@@ -320,10 +284,10 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
         // The operand rounded to bf16 once, into the context's scratch (TensorGEMMBF16.swift:208-264).
         const int ky = pad_k ? kp : q.k;
         const size_t bytes = (size_t)q.m * (size_t)ky * 2;
-        st = reserve_scratch(ctx, bytes > 0 ? bytes : 2);
+        st = reserve(ctx, ctx->scratch, bytes > 0 ? bytes : 2);
         if (st != SQ8_OK) return st;
         const float *x = static_cast<const float *>(q.a);
-        uint16_t *y = static_cast<uint16_t *>(ctx->scratch);
+        uint16_t *y = static_cast<uint16_t *>(ctx->scratch.at);
         hipError_t e = sq8::launch_round_bf16_rows(x, q.lda, y, q.m, q.k, ky, ctx->stream);
         if (e != hipSuccess) return hip_status(e);
         p.a = y;
@@ -396,12 +360,12 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
     // run on the weight-direct kernels only.
     int wl_run = q.w_layout;
     if (p.a_vec && k_steps && (plain ? repack : !is_packed(q.w_layout) && (q.k % 64 != 0 || q.w_layout == SQ8_KN))) {
-        st = reserve_buffer(ctx, &ctx->wpack, &ctx->wpack_bytes, (size_t)w_packed);
+        st = reserve(ctx, ctx->wpack, (size_t)w_packed);
         if (st != SQ8_OK) return st;
         e = sq8::launch_pack(p.w, q.w_layout == SQ8_KN ? sq8::W_KN : sq8::W_NK, p.ldw, q.k, q.n, is_glu(q.epilogue),
-                             static_cast<uint8_t *>(ctx->wpack), ctx->stream);
+                             static_cast<uint8_t *>(ctx->wpack.at), ctx->stream);
         if (e != hipSuccess) return hip_status(e);
-        p.w = static_cast<const uint8_t *>(ctx->wpack);
+        p.w = static_cast<const uint8_t *>(ctx->wpack.at);
         wl_run = is_glu(q.epilogue) ? SQ8_PACKED_GLU : SQ8_PACKED;
     }
     if (is_packed(wl_run) || (q.w_layout == SQ8_NK && p.a_vec && p.w_vec && q.k > 0 && q.k % 64 == 0 && cols_per_half >= 1)) {
@@ -420,9 +384,9 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
             if (splits > 1) {
                 const int64_t bytes = sq8::skinny_part_bytes(q.m, q.n, is_glu(q.epilogue),
                                                              tile == sq8::WD_SKINNY32 ? 32 : 64, splits);
-                st = reserve_buffer(ctx, &ctx->part, &ctx->part_bytes, (size_t)bytes);
+                st = reserve(ctx, ctx->part, (size_t)bytes);
                 if (st != SQ8_OK) return st;
-                p.part = static_cast<float *>(ctx->part);
+                p.part = static_cast<float *>(ctx->part.at);
                 p.splits = splits;
             }
         }
@@ -506,9 +470,9 @@ int run_w8a8(sq8_ctx *ctx, const W8A8 &q, double *gpu_seconds) {
         const hipError_t e = static_scratch_of(ctx->device, &scr);
         if (e != hipSuccess) return hip_status(e);
     } else if (bytes > 0) {
-        st = reserve_scratch(ctx, bytes);
+        st = reserve(ctx, ctx->scratch, bytes);
         if (st != SQ8_OK) return st;
-        scr = static_cast<uint8_t *>(ctx->scratch);
+        scr = static_cast<uint8_t *>(ctx->scratch.at);
     }
     int8_t *codes = own_codes ? reinterpret_cast<int8_t *>(scr) : const_cast<int8_t *>(q.codes);
     const float *sx = q.a ? reinterpret_cast<float *>(scr + code_bytes) : q.sx;
@@ -572,12 +536,12 @@ int run_w8a8(sq8_ctx *ctx, const W8A8 &q, double *gpu_seconds) {
         p.kt_w = q.k / 64;
     } else {
         const int64_t wbytes = sq8::packed_bytes(q.k, q.n, is_glu(q.epilogue));
-        st = reserve_buffer(ctx, &ctx->wpack, &ctx->wpack_bytes, (size_t)wbytes);
+        st = reserve(ctx, ctx->wpack, (size_t)wbytes);
         if (st != SQ8_OK) return st;
         e = sq8::launch_pack(static_cast<const uint8_t *>(q.w), q.w_layout == SQ8_KN ? sq8::W_KN : sq8::W_NK, q.ldw, q.k,
-                             q.n, is_glu(q.epilogue), static_cast<uint8_t *>(ctx->wpack), ctx->stream);
+                             q.n, is_glu(q.epilogue), static_cast<uint8_t *>(ctx->wpack.at), ctx->stream);
         if (e != hipSuccess) return hip_status(e);
-        p.w = static_cast<const uint8_t *>(ctx->wpack);
+        p.w = static_cast<const uint8_t *>(ctx->wpack.at);
         p.kt_w = (q.k + 63) / 64;
     }
     int tile = ctx->i8_tile >= 0 ? ctx->i8_tile : sq8::choose_i8_tile(q.m, q.n, is_glu(q.epilogue), ctx->cus, p.kt, q.residual);
@@ -662,10 +626,10 @@ int run_blocks(sq8_ctx *ctx, const Blocks &q, double *gpu_seconds) {
     } else if (q.a_dtype == SQ8_F32) {
         // The operand rounded to bf16 once, into the context's scratch (TensorGEMMBF16.swift:208-264).
         const size_t bytes = (size_t)q.m * (size_t)kp * 2;
-        int st = reserve_scratch(ctx, bytes > 0 ? bytes : 2);
+        int st = reserve(ctx, ctx->scratch, bytes > 0 ? bytes : 2);
         if (st != SQ8_OK) return st;
         const float *x = static_cast<const float *>(q.a);
-        uint16_t *y = static_cast<uint16_t *>(ctx->scratch);
+        uint16_t *y = static_cast<uint16_t *>(ctx->scratch.at);
         hipError_t e = sq8::launch_round_bf16_rows(x, q.lda, y, q.m, q.k, kp, ctx->stream);
         if (e != hipSuccess) return hip_status(e);
         p.a = y;
@@ -683,13 +647,13 @@ int run_blocks(sq8_ctx *ctx, const Blocks &q, double *gpu_seconds) {
         // The codes and their scales packed per product into the context's buffer (the reference
         // reads the map's [K, N] codes and [K/B, N] scales in place, TensorGEMM.swift:307-318).
         const int64_t bytes = sq8::packed_blocks_bytes(q.k, q.n, is_glu(q.epilogue));
-        int st = reserve_buffer(ctx, &ctx->wpack, &ctx->wpack_bytes, (size_t)bytes);
+        int st = reserve(ctx, ctx->wpack, (size_t)bytes);
         if (st != SQ8_OK) return st;
         hipError_t e = sq8::launch_pack_blocks(p.w, q.w_layout == SQ8_KN ? sq8::W_KN : sq8::W_NK, q.ldw, q.scale,
                                                q.scale_dtype, q.block, q.k, q.n, is_glu(q.epilogue),
-                                               static_cast<uint8_t *>(ctx->wpack), ctx->stream);
+                                               static_cast<uint8_t *>(ctx->wpack.at), ctx->stream);
         if (e != hipSuccess) return hip_status(e);
-        p.w = static_cast<const uint8_t *>(ctx->wpack);
+        p.w = static_cast<const uint8_t *>(ctx->wpack.at);
     }
     p.bias = q.bias;
     p.c[0] = q.c;
@@ -866,9 +830,10 @@ int sq8_destroy(sq8_ctx *ctx) {
     int st = SQ8_OK;
     hipError_t e = hipStreamSynchronize(ctx->stream);
     if (e != hipSuccess) st = hip_status(e);
-    if (ctx->scratch) (void)hipFree(ctx->scratch);
-    if (ctx->wpack) (void)hipFree(ctx->wpack);
-    if (ctx->part) (void)hipFree(ctx->part);
+    sq8::release(ctx->scratch);
+    sq8::release(ctx->wpack);
+    sq8::release(ctx->part);
+    sq8::release(ctx->aside);
     if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
     (void)hipEventDestroy(ctx->begin);
     (void)hipEventDestroy(ctx->end);

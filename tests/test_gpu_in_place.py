@@ -90,3 +90,47 @@ def test_in_place_under_capture(layout, m, k, n, before):
                                   layout=layout, bias=b if layout == "kn" else b.repeat(i + 2), out_dtype=torch.float32)
             torch.cuda.synchronize()
             assert torch.allclose(got[:m, :n], want, rtol=2e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("kind", ["kn_slabs", "fp32_rounded", "fp32_route", "rotated", "padded_k", "w8a8", "w8a8_kn", "q8_kn"])
+def test_graph_buffers_outlive_growth(kind):
+    """A captured product that uses the context's buffers, replayed after larger products have outgrown them: the same bits as
+    before the capture, and the larger products' own as on another context."""
+    import siliconed_amd as sq
+    k = 200 if kind == "padded_k" else 512
+    x, q, s, b = _operands(40, k, 192, 11)
+    a = x.float() if kind in ("fp32_rounded", "fp32_route", "w8a8", "w8a8_kn") else x
+    d = torch.rand((k // 32, 192), device=DEV) * 0.02 + 1e-3
+
+    def product(ctx, a, y):
+        if kind in ("w8a8", "w8a8_kn"):
+            return ctx.product_quantized(a, w, s, group=64, bias=b, out=y, layout="kn" if kind == "w8a8_kn" else "nk")
+        if kind == "q8_kn":
+            return ctx.product_blocks(a, w, d, 32, layout="kn", bias=b, out=y)
+        return ctx.product(a, w, s, bias=b, out=y, layout="kn" if kind == "kn_slabs" else "nk", rounding=kind != "fp32_route",
+                           rotation=64 if kind == "rotated" else 0)
+
+    stream = torch.cuda.Stream()
+    ctx, other = sq.TensorGEMM.make(0, stream), sq.TensorGEMM.make(0, stream)
+    w = q.t().contiguous() if kind in ("kn_slabs", "w8a8_kn", "q8_kn") else ctx.pack(q, layout="nk") if kind == "padded_k" else q
+    big = [a.repeat(8 << i, 1) for i in range(3)]  # each needs a larger scratch
+    wide = [_operands(40, 512, 256 << i, i) for i in range(3)]  # and each a larger packing buffer
+    y, want = torch.zeros((40, 192), device=DEV), torch.zeros((40, 192), device=DEV)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        product(ctx, a, want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        product(ctx, a, y)
+    for rows, (xw, qw, sw, bw) in zip(big, wide):
+        y.zero_()
+        with torch.cuda.stream(stream):
+            outs = [product(c, rows, torch.zeros((rows.shape[0], 192), device=DEV)) for c in (ctx, other)]
+            outs += [c.product(xw, qw.t().contiguous(), sw, layout="kn", bias=bw) for c in (ctx, other)]
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[3])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+    torch.cuda.synchronize()
