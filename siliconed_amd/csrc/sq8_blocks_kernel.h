@@ -70,6 +70,7 @@ gemm_blocks_kernel(const GemmArgs p) {
     constexpr int A_PER_WAVE = BM / 8 / NW;
     static_assert(BM / 8 % NW == 0, "the activation blocks split evenly over the waves");
     constexpr int GROUPS = FM;                // groups a step: two K blocks × FM/2 pairs of row blocks
+    static_assert(A_PER_WAVE <= GROUPS, "a group issues one activation load, the one before the last a second");
     constexpr int WLOADS = 3;                 // two code loads and a scale load per step
     constexpr int LDS_BYTES = NAS * SA > NW * grp::SLOT ? NAS * SA : NW * grp::SLOT;
 
@@ -201,8 +202,11 @@ gemm_blocks_kernel(const GemmArgs p) {
                 if constexpr (kb == 0) widen(SU{}, I1{}, KS{});
                 else widen(S1{}, I0{}, KS{});
             }
-            // Into the stage and buffer last read during step t − 1 (its barrier saw every wave's reads).
-            if constexpr (g < A_PER_WAVE) issue_a1(t + 3, S3{}, gc);
+            // Into the stage and buffer last read during step t − 1 (its barrier saw every wave's reads): the activation's loads
+            // in the groups before the last, the code loads in the last, so that the step's wait counts them in this order
+            // (within a group the compiler orders loads as it likes).
+            if constexpr (g < A_PER_WAVE && g < GROUPS - 1) issue_a1(t + 3, S3{}, gc);
+            if constexpr (g == GROUPS - 2 && A_PER_WAVE == GROUPS) issue_a1(t + 3, S3{}, std::integral_constant<int, GROUPS - 1>{});
             if constexpr (g == GROUPS - 1) issue_w(t + 3, S3{});
             static_for<0, 2>([&](auto kc) {
                 constexpr int ks = decltype(kc)::value;
