@@ -164,3 +164,95 @@ def test_group_tile_exact_sums_same_bits(tile_gemm, route, tile):
             g.product_residual(y, x, w, s, bias=b, gate=gate)
         torch.cuda.synchronize()
         assert torch.equal(*streams)
+
+
+def _same(x, y):
+    """The same values, NaN in the same places."""
+    return torch.equal(x.isnan(), y.isnan()) and torch.equal(x.nan_to_num(), y.nan_to_num())
+
+
+@pytest.mark.parametrize("route,tile", [("bf16", "g32x64k4"), ("bf16", "g128x192k2"), ("fp32", "g64x96k4"), ("fp32", "g96x192k2")])
+def test_group_tile_infinities_and_nan(tile_gemm, route, tile):
+    """NaN and infinite activations reach their own rows only, NaN fp8 codes their own columns, through the split of K
+    (a K of 200 padded to whole steps; 7 steps over the groups), as in the 128-row tiles."""
+    got, want = tile_gemm(tile), tile_gemm("128")
+    for m, k, n, fp8, epi in [(40, 448, 200, False, None), (131, 200, 96, True, "gelu_tanh"), (33, 512, 128, True, "silu_glu")]:
+        g = torch.Generator(device=DEV).manual_seed(m)
+        q = torch.randint(-3, 4, (n, k), device=DEV, generator=g).to(torch.float8_e4m3fn if fp8 else torch.int8)
+        if fp8:
+            q.view(torch.uint8)[17, k - 1] = 0x7F
+        x = torch.randint(-5, 6, (m, k), device=DEV, generator=g).float()
+        x[5, 7], x[9, 3], x[12, k - 1], x[31, 64] = float("nan"), float("inf"), float("-inf"), float("inf")
+        x = x if route == "fp32" else x.bfloat16()
+        s, b = torch.rand(n, device=DEV, generator=g) * 1e-2 + 1e-3, torch.randn(n, device=DEV, generator=g)
+        s[3] = float("inf")
+        w = want.pack(q, layout="nk", glu=epi == "silu_glu")
+        ys = [c.product(x, w, s, bias=b, epilogue=epi, out_dtype=torch.float32, rounding=route == "bf16") for c in (got, want)]
+        torch.cuda.synchronize()
+        assert _same(*ys)
+        assert ys[0][5].isnan().all() and (ys[0].isnan().sum(1) < n // 4).sum() >= m - 5
+
+
+@pytest.mark.parametrize("tile", Q8_TILES)
+def test_q8_tile_infinities_and_nan(q8_gemm, tile):
+    """The same through the block scales: an infinite scale meets one block of one column; the padded half step's zero
+    codes and scales (a K of 32·odd) stay out of every sum."""
+    m, k, n = 37, 352, 136
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randint(-5, 6, (m, k), device=DEV, generator=g).float()
+    x[5, 7], x[9, 3], x[12, k - 1] = float("nan"), float("inf"), float("-inf")
+    q = torch.randint(-127, 128, (n, k), device=DEV, generator=g, dtype=torch.int8)
+    d = (torch.rand((n, k // 32), device=DEV, generator=g) * 0.02 + 1e-3).half()
+    d[20, 4] = float("inf")
+    ctx = q8_gemm[tile]
+    y = ctx.product_blocks(x.bfloat16(), ctx.pack_blocks(q, d, 32, layout="nk"), out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    acc = torch.zeros((m, n), dtype=torch.float64)
+    xs, qs, ds = x.double().cpu(), q.double().cpu(), d.double().cpu()
+    for i in range(k // 32):
+        part = (xs[:, None, 32 * i:32 * i + 32] * qs[None, :, 32 * i:32 * i + 32]).sum(-1)
+        acc = (part * ds[:, i] + acc).float().double()
+    assert _same(y.cpu(), acc.float())
+    assert torch.isfinite(y).sum() == (m - 3) * (n - 1)
+
+
+@pytest.mark.parametrize("kind,tile", [("bf16", "g64x96k4"), ("bf16", "g96x192k2"), ("w8a8", "g32x64k8"), ("w8a8", "g128x96k4")])
+def test_group_tile_outputs_off_the_four_column_grid(tile_gemm, kind, tile):
+    """Stores one column at a time: three outputs off the 16-byte grid, rows and heads that end inside a wave's columns; a
+    residual stream of an odd width, off the grid, with and without a gate; a plain output one element in. Bit for bit the
+    128-row tiles'."""
+    got, want = tile_gemm(tile), tile_gemm("128")
+    m, k = 75, 384
+    off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+
+    def operands(n, seed):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        q = torch.randint(-3, 4, (n, k), device=DEV, generator=g).to(torch.int8)
+        x = torch.randint(-5, 6, (m, k), device=DEV, generator=g)
+        s, b = torch.rand(n, device=DEV, generator=g) * 1e-2 + 1e-3, torch.randn(n, device=DEV, generator=g)
+        sx = torch.rand(m, device=DEV, generator=g) + 0.5
+        return ((x.bfloat16(),) if kind == "bf16" else (x.to(torch.int8), sx)), want.pack(q, layout="nk"), s, b
+
+    for d, head_dim in ((100, 0), (100, 20), (96, 12), (36, 4)):
+        x, w, s, b = operands(3 * d, d + head_dim)
+        shape = (m, d) if head_dim == 0 else (d // head_dim, m, head_dim)
+        for dtype in (torch.bfloat16, torch.float32):
+            outs = [tuple(f(torch.zeros(shape, device=DEV, dtype=dtype)) for f in (off, off, torch.clone)) for _ in range(2)]
+            for ctx, out in zip((got, want), outs):
+                (ctx.product_qkv if kind == "bf16" else ctx.product_w8a8_qkv)(*x, w, s, bias=b, head_dim=head_dim, out=out,
+                                                                             out_dtype=dtype)
+            torch.cuda.synchronize()
+            assert all(torch.equal(u, v) for u, v in zip(*outs)) and all(u.any() for u in outs[0])
+    for n in (385, 384):
+        x, w, s, b = operands(n, n)
+        for gate in (None, off(torch.linspace(-1.0, 1.0, n, device=DEV))):
+            streams = [off(torch.ones((m, n), device=DEV)) for _ in range(2)]
+            for ctx, y in zip((got, want), streams):
+                (ctx.product_residual if kind == "bf16" else ctx.product_w8a8_residual)(y, *x, w, s, bias=b, gate=gate)
+            torch.cuda.synchronize()
+            assert torch.equal(*streams) and not torch.equal(streams[0], torch.ones_like(streams[0]))
+        outs = [off(torch.zeros((m, n), device=DEV, dtype=torch.bfloat16)) for _ in range(2)]
+        for ctx, y in zip((got, want), outs):
+            (ctx.product if kind == "bf16" else ctx.product_w8a8)(*x, w, s, bias=b, out=y)
+        torch.cuda.synchronize()
+        assert torch.equal(*outs)
