@@ -101,10 +101,14 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
     // workgroup on the CUs (N ≤ 8192 on 256 CUs), for a single row without GLU three (N ≤ 12288): every K step's loads
     // in flight, the activation read once per workgroup. Kernel traces at K = 3072, N = 3072 (int8 packed, bias): M = 1
     // 4.10 µs against the skinny kernel's 7.44, M = 16 5.95 against 8.73; two groups, SiLU-GLU: M = 3, N = 8192 5.8
-    // against 8.5, M = 16 7.3 against 9.4; three, M = 1: N = 9216 8.9 against 9.7, N = 12288 10.6 against 11.4. Past
-    // four rows only with the activation in its LDS (16 × 6144 × 3072 11.3 against 8.5 µs for a K-group tile).
+    // against 8.5, M = 16 7.3 against 9.4; three, M = 1: N = 9216 8.9 against 9.7, N = 12288 10.6 against 11.4. With the
+    // activation not in its LDS, to four rows of up to two groups (16 × 6144 × 3072 11.3 against 8.5 µs for a K-group
+    // tile; one row of three, 1 × 7808 × 10944, 23.5 against 18.8), and one group of GLU columns
+    // (SiLU-GLU 10 × 3840 × 3072 7.2 against 9.1 for a K-group tile, 5 × 1152 × 3200 4.8 against 5.9).
     const int groups16 = glu ? (N / 2 + 7) / 8 : (N + 15) / 16;
-    if (M <= 16 && (M <= 4 || gemv_x_in_lds(M, kt)) && (groups16 <= 2 * cus || (M == 1 && !glu && groups16 <= 3 * cus)))
+    const bool staged = gemv_x_in_lds(M, kt);
+    if (M <= 16 && ((groups16 <= 2 * cus && (M <= 4 || staged)) || (glu && groups16 <= cus) ||
+                    (M == 1 && !glu && staged && groups16 <= 3 * cus)))
         return WD_GEMV;
     // Up to 16 rows on a weight wider than 3/4 of the CUs' 64-column slabs, the skinny kernel (a slab a workgroup, four
     // a CU): its many small workgroups stream the weight best (1 × 3072 × 18432 13.7 µs against 16.0 in 32 × 64 tiles, 8

@@ -14,20 +14,33 @@ PROBE = r"""
 #include "sq8_gemm.hip"
 #include <stdio.h>
 int main() {
-    int m, n, glu, cus, steps, f32;
-    while (scanf("%d %d %d %d %d %d", &m, &n, &glu, &cus, &steps, &f32) == 6) {
-        const int tile = sq8::choose_wd_tile(m, n, glu != 0, cus, steps, f32 != 0);
-        const int groups = tile >= sq8::GROUP_TILE0 ? sq8::group_shapes[tile - sq8::GROUP_TILE0].groups : 0;
-        const bool one = tile == sq8::WD_128 || tile == sq8::WD_224 || tile == sq8::WD_256;
-        printf("%s\n", one ? "one" : groups == 2 ? "two" : groups == 4 ? "four" : "short");
+    char route[8];
+    int m, n, glu, cus, steps, residual;
+    while (scanf("%7s %d %d %d %d %d %d", route, &m, &n, &glu, &cus, &steps, &residual) == 7) {
+        if (route[0] == 'q') {
+            const int tile = sq8::choose_blocks_tile(m, n, glu != 0, cus, steps);
+            if (tile > sq8::BLOCKS16_ROWS) printf("short %d\n", tile - sq8::BLOCKS16_ROWS);
+            else printf("one %s\n", tile == sq8::BL_128x128 ? "128x128" : "128x256");
+            continue;
+        }
+        const int tile = route[0] == 'w' ? sq8::choose_i8_tile(m, n, glu != 0, cus, steps, residual != 0)
+                                         : sq8::choose_wd_tile(m, n, glu != 0, cus, steps, route[0] == 'f');
+        if (tile >= sq8::GROUP_TILE0) {
+            const sq8::GroupShape &g = sq8::group_shapes[tile - sq8::GROUP_TILE0];
+            printf("%s %s\n", g.groups == 2 ? "two" : g.groups == 4 ? "four" : "eight", g.name);
+        } else if (route[0] == 'w' || tile == sq8::WD_128 || tile == sq8::WD_224 || tile == sq8::WD_256) {
+            printf("one %s\n", route[0] == 'w' || tile == sq8::WD_128 ? "128" : tile == sq8::WD_224 ? "224" : "256");
+        } else {
+            printf("short %s\n", tile == sq8::WD_GEMV ? "gemv" : "skinny");
+        }
     }
 }
 """
 
 
 @pytest.fixture(scope="module")
-def families(tmp_path_factory):
-    """[(m, n, glu, cus, steps, f32), …] → each product's order of sums by the rule."""
+def rule(tmp_path_factory):
+    """[(route, m, n, glu, cus, steps, residual), …] → each product's (order of sums, tile) by the rule."""
     from siliconed_amd.build import HIPCC
     d = tmp_path_factory.mktemp("tile_rule")
     src, exe = str(d / "probe.hip"), str(d / "probe")
@@ -38,24 +51,35 @@ def families(tmp_path_factory):
     assert r.returncode == 0, r.stderr
 
     def run(cases):
-        text = "".join(" ".join(str(int(v)) for v in c) + "\n" for c in cases)
+        text = "".join(" ".join(str(v if isinstance(v, str) else int(v)) for v in c) + "\n" for c in cases)
         out = subprocess.run([exe], input=text, capture_output=True, text=True)
         assert out.returncode == 0, out.stderr
-        return out.stdout.split()
+        return [tuple(line.split()) for line in out.stdout.splitlines()]
 
     return run
 
 
-@pytest.mark.parametrize("f32", [False, True], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("route", ["bf16", "fp32"])
 @pytest.mark.parametrize("n", [1025, 2048, 3072, 3840, 4608, 5120, 9217, 12288, 20480])
-def test_tall_products_sum_in_one_sequence(families, n, f32):
+def test_tall_products_sum_in_one_sequence(rule, n, route):
     """From 4096 rows on and past 1024 columns a product's rows have the same bits however they are chunked."""
-    cases = [(m, n, glu, 256, steps, f32) for m in [*range(4096, 12289, 61), 4352, 4608, 5376, 6144, 8192, 20000, 100000]
+    cases = [(route, m, n, glu, 256, steps, 0) for m in [*range(4096, 12289, 61), 4352, 4608, 5376, 6144, 8192, 20000, 100000]
              for glu in (False, True) if n % 2 == 0 or not glu for steps in (1, 16, 48, 60, 192)]
-    assert set(families(cases)) == {"one"}
+    assert {order for order, _ in rule(cases)} == {"one"}
 
 
-def test_short_products_split_k(families):
+def test_short_products_split_k(rule):
     """The rule still splits K where tiles are few."""
-    assert families([(77, 3072, 0, 256, 48, 0), (1531, 3072, 0, 256, 48, 1), (1, 3072, 0, 256, 48, 0), (4096, 128, 0, 256, 48, 0)]) == [
-        "four", "two", "short", "four"]
+    assert [order for order, _ in rule([("bf16", 77, 3072, 0, 256, 48, 0), ("fp32", 1531, 3072, 0, 256, 48, 0),
+                                        ("bf16", 1, 3072, 0, 256, 48, 0), ("bf16", 4096, 128, 0, 256, 48, 0),
+                                        ("w8a8", 77, 3072, 0, 256, 24, 0)])] == ["four", "two", "short", "four", "eight"]
+
+
+@pytest.mark.parametrize("case,tile", [
+    # Up to 16 rows of one group of GLU columns, the activation not in the short-M kernel's LDS; one row of three groups.
+    (("bf16", 10, 3072, 1, 256, 60, 0), "gemv"), (("bf16", 5, 3200, 1, 256, 18, 0), "gemv"), (("bf16", 11, 256, 1, 256, 26, 0), "gemv"),
+    (("bf16", 1, 10944, 0, 256, 122, 0), "g32x64k4"), (("bf16", 1, 9216, 0, 256, 48, 0), "gemv"), (("bf16", 16, 3072, 0, 256, 96, 0), "g32x32k4"),
+], ids=str)
+def test_measured_choices(rule, case, tile):
+    """Shapes on which another tile measured 10 % slower or more."""
+    assert rule([case])[0][1] == tile
