@@ -72,25 +72,30 @@ static float rounds_us(float tiles, int cus, float round) {
     return round * (full + (rest > 0.0f ? 0.66f + 0.34f * rest : 0.0f));
 }
 
-// The same of a kernel of two workgroups a CU: `two` a round of them, `one` a last round of at most one a CU.
+// The same of a kernel of two workgroups a CU: `two` a round of them, `one` a last round of at most one a CU; a last round
+// with two on some CUs and one on the others is shorter (384 of 512: 0.88 to 0.96 of `two` on the three routes).
 static float pairs_us(float tiles, int cus, float two, float one) {
     const float full = floorf(tiles / (2.0f * (float)cus)), rest = tiles - full * 2.0f * (float)cus;
-    return full * two + (rest > (float)cus ? two : rounds_us(rest, cus, one));
+    if (rest > (float)cus) return two * (full + 0.86f + 0.14f * (rest / (float)cus - 1.0f));
+    return full * two + rounds_us(rest, cus, one);
 }
 
 // Calls take(tile, µs) for every K-group shape that serves M rows × `blocks` 32-column blocks of weight and `steps` weight K
 // steps (unrolled: each shape's divisions are by constants; the rule runs on every call); `value_us`: further µs a value of
-// the tile.
+// the tile, `round_us`: a round past the first.
 template <int MATH, int I = 0, typename F>
-static inline void each_group(int M, int blocks, bool glu, int cus, int steps, float value_us, F &&take) {
+static inline void each_group(int M, int blocks, bool glu, int cus, int steps, float value_us, float round_us, F &&take) {
     if constexpr (I < kGroupShapes) {
         constexpr GroupShape g = group_shapes[I];
         constexpr GroupCost c = g.cost[MATH];
         constexpr int nw = g.cols / 32;
         // bf16: four groups give the skinny kernel's bits at any K, two the 64 × 128 tiles' where the steps divide.
-        if (c.us_step > 0.0f && !(glu && nw % 2 != 0) && !(MATH == GM_BF16 && steps % 2 != 0 && g.groups == 2))
-            take(GROUP_TILE0 + I, rounds_us(tile_count(M, g.rows, blocks, nw), cus, c.us + c.us_step * (float)steps + value_us * (float)(g.rows * g.cols)));
-        each_group<MATH, I + 1>(M, blocks, glu, cus, steps, value_us, take);
+        if (c.us_step > 0.0f && !(glu && nw % 2 != 0) && !(MATH == GM_BF16 && steps % 2 != 0 && g.groups == 2)) {
+            const float tiles = tile_count(M, g.rows, blocks, nw);
+            take(GROUP_TILE0 + I, rounds_us(tiles, cus, c.us + c.us_step * (float)steps + value_us * (float)(g.rows * g.cols)) +
+                                      round_us * floorf((tiles - 1.0f) / (float)cus));
+        }
+        each_group<MATH, I + 1>(M, blocks, glu, cus, steps, value_us, round_us, take);
     }
 }
 
@@ -149,9 +154,9 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
     // the rounds better (µs): 5760 × 3072 × 3072 115.9 → 119.9, with the residual 124.6 → 141.8, fp32 route 309 → 375.
     if (M >= 4096 && N > 1024) return tile;
     if (f32)
-        each_group<GM_F32>(M, blocks, glu, cus, steps, 0.0f, take);
+        each_group<GM_F32>(M, blocks, glu, cus, steps, 0.0f, 0.0f, take);
     else
-        each_group<GM_BF16>(M, blocks, glu, cus, steps, 0.0f, take);
+        each_group<GM_BF16>(M, blocks, glu, cus, steps, 0.0f, 0.0f, take);
     return tile;
 }
 
@@ -165,13 +170,15 @@ int choose_i8_tile(int M, int N, bool glu, int cus, int kt, bool residual) {
     // 17.0, 333 × 9216 25.0 → 20.0; K = 12288, 68 × 512 62.9 → 9.7. The residual epilogue reads and writes 8 bytes a value
     // past the sums, a round's at the CU's share of the memory's rate (0.4 ns a value) where one workgroup fills the CU,
     // half of that under the other's K steps where two do: 3742 × 3072 × 3072 62.9 µs in 128 × 256 and 71.3 in 128 × 192
-    // tiles, at K = 12288 163 and 159.
+    // tiles, at K = 12288 163 and 159. Rounds of K-group tiles past the first cost about 1 µs more than it (their loads wait
+    // for an epilogue): 3277 × 1024 × 1024 with SiLU-GLU 14.8 µs in 1.6 rounds of 64 × 128, 11.0 in one of 128 × 128; 1975
+    // × 3072 × 6144 57.1 in 128 × 192, 49.4 in 128 × 256.
     if (cus <= 0) cus = 256;
     const int blocks = glu ? 2 * ((N / 2 + 31) / 32) : (N + 31) / 32;  // 32-column blocks
     const float two = residual ? 22.2f : 11.2f, one = residual ? 15.6f : 9.6f;
     float best = pairs_us(tile_count(M, 128, blocks, 8), cus, two + 1.70f * (float)kt, one + 0.91f * (float)kt);
     int tile = I8_128x256;
-    each_group<GM_I8>(M, blocks, glu, cus, kt, residual ? 4e-4f : 0.0f, [&](int t, float time) {
+    each_group<GM_I8>(M, blocks, glu, cus, kt, residual ? 4e-4f : 0.0f, 1.0f, [&](int t, float time) {
         if (time < best) {
             best = time;
             tile = t;

@@ -79,6 +79,10 @@ def test_short_products_split_k(rule):
     # Up to 16 rows of one group of GLU columns, the activation not in the short-M kernel's LDS; one row of three groups.
     (("bf16", 10, 3072, 1, 256, 60, 0), "gemv"), (("bf16", 5, 3200, 1, 256, 18, 0), "gemv"), (("bf16", 11, 256, 1, 256, 26, 0), "gemv"),
     (("bf16", 1, 10944, 0, 256, 122, 0), "g32x64k4"), (("bf16", 1, 9216, 0, 256, 48, 0), "gemv"), (("bf16", 16, 3072, 0, 256, 96, 0), "g32x32k4"),
+    # W8A8: a round of more than one and fewer than two workgroups a CU; rounds of K-group tiles past the first.
+    (("w8a8", 3912, 3072, 0, 256, 24, 0), "128"), (("w8a8", 1975, 6144, 0, 256, 24, 0), "128"),
+    (("w8a8", 3277, 1024, 1, 256, 8, 0), "g128x128k2"), (("w8a8", 239, 16000, 0, 256, 8, 0), "g128x128k2"),
+    (("w8a8", 498, 18752, 0, 256, 7, 0), "128"), (("w8a8", 512, 3072, 0, 256, 24, 0), "g64x96k4"), (("w8a8", 1531, 3072, 0, 256, 24, 0), "g96x192k2"),
 ], ids=str)
 def test_measured_choices(rule, case, tile):
     """Shapes on which another tile measured 10 % slower or more."""
