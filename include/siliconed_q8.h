@@ -86,7 +86,7 @@ typedef struct sq8_ctx sq8_ctx;
  * "224", "128", "64", "32", "64n", "64x192", "s64", "s32", "gemv", "k32x32", "k32x64", "k64x64", "k64x128",
  * "k64x192": the weight-direct kernels' tile; "128": the W8A8 product's; "g<rows>x<columns>k<groups>", "g64x96k4" for
  * one: the tile of either),
- * SQ8_Q8_TILE ("128x256", "128x128", or "16", "32", "48", "64", "80" rows of the narrow-wave kernel: the
+ * SQ8_Q8_TILE ("128x256", "64x256", "128x128", or "16", "32", "48", "64", "80" rows of the narrow-wave kernel: the
  * block-scale product's tile) and SQ8_SPLITS (a
  * count ≥ 1: the skinny
  * kernel's K split over workgroups, added by a second launch; 1, the default, none; at most the

@@ -805,7 +805,7 @@ int sq8_create(int device, void *stream, sq8_ctx **out) {
         {"gemv", sq8::WD_GEMV}, {"k32x32", KNOB_K + 0}, {"k32x64", KNOB_K + 1}, {"k64x64", KNOB_K + 2},
         {"k64x128", KNOB_K + 3}, {"k64x192", KNOB_K + 4}}));
     ctx->i8_tile = group_knob(getenv("SQ8_TILE"), knob(getenv("SQ8_TILE"), {{"128", sq8::I8_128x256}}));
-    ctx->q8_tile = knob(getenv("SQ8_Q8_TILE"), {{"128x256", sq8::BL_128x256}, {"128x128", sq8::BL_128x128},
+    ctx->q8_tile = knob(getenv("SQ8_Q8_TILE"), {{"128x256", sq8::BL_128x256}, {"128x128", sq8::BL_128x128}, {"64x256", sq8::BL_64x256},
                                                 {"16", sq8::BLOCKS16_ROWS + 16}, {"32", sq8::BLOCKS16_ROWS + 32},
                                                 {"48", sq8::BLOCKS16_ROWS + 48}, {"64", sq8::BLOCKS16_ROWS + 64},
                                                 {"80", sq8::BLOCKS16_ROWS + 80}});

@@ -98,6 +98,7 @@ hipError_t launch_pack_blocks(const uint8_t *w, int wl, int64_t ldw, const void 
 
 hipError_t launch_blocks_product(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream) {
     if (tile > BLOCKS16_ROWS) return launch_blocks16(p, tile - BLOCKS16_ROWS, epi, out, stream);
+    if (tile == BL_64x256) return blk::launch_blocks_product<64, 8>(p, epi, out, stream);
     if (tile == BL_128x128) return blk::launch_blocks_product<128, 4>(p, epi, out, stream);
     return blk::launch_blocks_product<128, 8>(p, epi, out, stream);
 }

@@ -32,6 +32,9 @@
 // 33.6 in 128 × 128; 1021 × 3072 × 3072 54.9 → 40.3 (128 × 128, two workgroups a CU: one's epilogue under the other's
 // MFMAs). On a full chip the clock follows the power (4096 × 3072 × 12288, the same 780 k cycles: 403 µs, with every
 // activation zero 349, with every code zero 321), so there the cycles saved come back as 2.5 % (400 → 391 µs).
+// 64 × 256 tiles (two row blocks a wave: two groups a step, each widening a whole K block) serve products that leave a
+// round of the taller ones part empty: SiLU-GLU 575 × 1024 × 7040 17.5 µs (28 tiles of 128 × 256 a row 23.5), 1065 ×
+// 1536 × 7488 42.2 (128 × 128 51.5).
 // Measured and not kept: eight activation stages with a barrier every two steps (402 against 406 µs, two registers
 // spilled).
 //
@@ -196,12 +199,13 @@ gemm_blocks_kernel(const GemmArgs p) {
                 read_x(SU{}, std::integral_constant<int, g + 1>{}, std::integral_constant<int, (g + 1) & 1>{});
             else
                 read_x(S1{}, I0{}, I0{});  // the next step's first
-            // The next K block's codes: one sub-step each in the K block's last two groups.
-            if constexpr (pair >= FM / 2 - 2) {
-                using KS = std::integral_constant<int, pair - (FM / 2 - 2)>;
-                if constexpr (kb == 0) widen(SU{}, I1{}, KS{});
-                else widen(S1{}, I0{}, KS{});
-            }
+            // The next K block's codes: one sub-step each in the K block's last two groups (both where it has one).
+            static_for<0, 2>([&](auto ks) {
+                if constexpr (FM == 2 || pair == FM / 2 - 2 + decltype(ks)::value) {
+                    if constexpr (kb == 0) widen(SU{}, I1{}, ks);
+                    else widen(S1{}, I0{}, ks);
+                }
+            });
             // Into the stage and buffer last read during step t − 1 (its barrier saw every wave's reads): the activation's loads
             // in the groups before the last, the code loads in the last, so that the step's wait counts them in this order
             // (within a group the compiler orders loads as it likes).
@@ -222,9 +226,9 @@ gemm_blocks_kernel(const GemmArgs p) {
             sp = sraw[U][kb];
             static_for<0, 4>([&](auto) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, FM == 2 ? 8 : 6, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, FM == 2 ? 6 : 5, 0);
                 __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
             });
             __builtin_amdgcn_sched_barrier(0);

@@ -117,10 +117,11 @@ hipError_t launch_pack(const uint8_t *w, int wl, int64_t ldw, int k, int n, bool
 // Codes with a scale per block of rows and column (GGUF Q8_0; sq8_blocks.hip): the packed Q8 layout
 // (codes in block-aligned K order, then fp32 scales per step and column) and its product, int8
 // codes, K a multiple of 64, A aligned for 16-byte loads. `tile`: choose_blocks_tile's: BL_128x256 (eight waves of one
-// 32-column block each, one workgroup per CU), BL_128x128 (four, two per CU), or BLOCKS16_ROWS + rows (below). Scales
+// 32-column block each, one workgroup per CU), BL_64x256 (the same waves on half the rows), BL_128x128 (four, two per
+// CU), or BLOCKS16_ROWS + rows (below). Scales
 // [K/B, N] for W_KN codes, [N, K/B] for W_NK; B a multiple of 32 dividing K; scale dtype numbered as the C ABI's
 // (fp32, bf16, fp16).
-enum BlocksTile { BL_128x256 = 0, BL_128x128 = 1 };
+enum BlocksTile { BL_128x256 = 0, BL_128x128 = 1, BL_64x256 = 2 };
 int64_t packed_blocks_bytes(int k, int n, bool glu);
 hipError_t launch_pack_blocks(const uint8_t *w, int wl, int64_t ldw, const void *scale, int scale_dtype, int block,
                               int k, int n, bool glu, uint8_t *out, hipStream_t stream);

@@ -188,28 +188,36 @@ int choose_i8_tile(int M, int N, bool glu, int cus, int kt, bool residual) {
 }
 
 int choose_blocks_tile(int M, int N, bool glu, int cus, int kt) {
-    // Every tile gives the same bits (each sum in K order), so only time decides: the least estimate of a workgroup's
-    // chain of K steps (µs a step, one workgroup a CU) against the CU's throughput (µs a step and workgroup), both
-    // measured at K = 3072 on full and nearly empty chips. Narrow waves (16 … 80 rows × 64 columns) where the wide
-    // kernel's tiles are few; measured against it (old → rule, µs, K = 3072): 77 × 12288 54 → 22, 512 × 3072 54 → 25,
-    // 16 × 128 (K = 2816) 48 → 11; K = 9728, 148 × 960 152 → 31. Wide: 128 × 128, two workgroups a CU (1021 × 3072
-    // 54.9 → 40.3, 333 × 9216 55 → 39.6), and 128 × 256 from four rounds of them on (GELU, 4096 × 12288 385 against
-    // 396: one activation tile for twice the columns; level at two rounds).
+    // Every tile gives the same bits (each sum in K order), so only time decides: the least estimate for the CU that holds
+    // the most workgroups, `at_once` of them side by side (registers): µs of a launch, of a workgroup (`group`), and of a K
+    // step, a workgroup's chain alone or the CU's work for each of several. Fitted to 270 to 370 shapes of 1 to 5000 rows, K
+    // 768 to 12288, plain and GLU, weights in and out of the caches (each tile's estimate within 4 % in the median; the
+    // choice 0.1 % past the best tile in the mean, 8 % at most). Narrow waves (16 … 80 rows × 64 columns) where tiles are
+    // few; measured against 128 × 256 tiles (µs, K = 3072): 77 × 12288 54 → 22, 512 × 3072 54 → 25, 16 × 128 (K = 2816) 48 →
+    // 11; K = 9728, 148 × 960 152 → 31. 64 × 256 where it fits a round that the taller tiles leave part empty or exceed
+    // (before it → with it: SiLU-GLU 575 × 1024 × 7040 23.5 → 17.5, 1065 × 1536 × 7488 51.5 → 42.2; GELU 300 × 3456 × 10944
+    // 54.1 → 40.3). 128 × 128, two a CU, past that (1021 × 3072 54.9 → 40.3), and 128 × 256 on a full chip and many steps
+    // (GELU, 4096 × 12288 385 against 396: one activation tile for twice the columns).
     if (cus <= 0) cus = 256;
     const float steps = (float)kt;
     const int slabs = glu ? (N / 2 + 31) / 32 : (N + 63) / 64;
-    auto a_cu = [&](int rows, int per) { return ceilf(tile_count(M, rows, slabs, per) / (float)cus); };
-    struct Narrow { int rows; float chain, work; };
-    static const Narrow narrow[] = {{16, 0.175f, 0.13f}, {32, 0.208f, 0.15f}, {48, 0.26f, 0.195f}, {64, 0.3125f, 0.238f},
-                                    {80, 0.375f, 0.294f}};
-    if (a_cu(128, 4) >= 4.0f) return BL_128x256;
-    float best = fmaxf(6.0f + 0.66f * steps, 4.0f + a_cu(128, 2) * 0.655f * steps);
-    int tile = BL_128x128;
-    for (const Narrow &w : narrow) {
-        const float us = steps * fmaxf(w.chain, a_cu(w.rows, 1) * w.work);
+    struct Tile { int tile, rows, slabs, at_once; float launch, group, chain, work; };
+    static const Tile tiles[] = {
+        {BLOCKS16_ROWS + 16, 16, 1, 4, 3.9f, 0.45f, 0.172f, 0.131f}, {BLOCKS16_ROWS + 32, 32, 1, 4, 4.1f, 0.65f, 0.195f, 0.142f},
+        {BLOCKS16_ROWS + 48, 48, 1, 3, 4.1f, 0.92f, 0.255f, 0.180f}, {BLOCKS16_ROWS + 64, 64, 1, 2, 3.3f, 1.78f, 0.309f, 0.206f},
+        {BLOCKS16_ROWS + 80, 80, 1, 2, 3.6f, 1.99f, 0.358f, 0.250f}, {BL_128x128, 128, 2, 2, 6.3f, 2.47f, 0.434f, 0.548f},
+        {BL_128x256, 128, 4, 1, 2.0f, 7.70f, 0.814f, 0.992f},        {BL_64x256, 64, 4, 1, 2.0f, 5.00f, 0.524f, 0.608f}};
+    float best = INFINITY;
+    int tile = BL_128x256;
+    for (const Tile &t : tiles) {
+        const float n = ceilf(tile_count(M, t.rows, slabs, t.slabs) / (float)cus), at_once = (float)t.at_once;
+        auto together = [&](float j) { return j > 0.0f ? j * t.group + steps * fmaxf(t.chain, j * t.work) : 0.0f; };
+        const float full = floorf(n / at_once);
+        const float us = t.launch + (t.at_once == 1 ? n * (t.group + steps * (n > 1.0f ? t.work : t.chain))
+                                                    : full * together(at_once) + together(n - full * at_once));
         if (us < best) {
             best = us;
-            tile = BLOCKS16_ROWS + w.rows;
+            tile = t.tile;
         }
     }
     return tile;

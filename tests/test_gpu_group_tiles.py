@@ -56,7 +56,7 @@ def test_w8a8_group_tile_same_bits(tile_gemm, tile):
 
 
 Q8_TILES = {"16": (16, 64), "32": (32, 64), "48": (48, 64), "64": (64, 64), "80": (80, 64), "128x128": (128, 128),
-            "128x256": (128, 256)}
+            "128x256": (128, 256), "64x256": (64, 256)}
 
 
 @pytest.fixture(scope="module")

@@ -13,7 +13,7 @@ SOURCE = os.path.join(ROOT, "siliconed_amd", "csrc", "sq8_blocks.hip")
 
 @pytest.fixture(scope="module")
 def steps(tmp_path_factory):
-    """Waves of the instance → its loads between barriers, A an activation load into LDS, W one into registers."""
+    """(rows, waves) of the instance → its loads between barriers, A an activation load into LDS, W one into registers."""
     from siliconed_amd.build import FLAGS, HIPCC
     out = str(tmp_path_factory.mktemp("asm") / "blocks.s")
     r = subprocess.run([HIPCC, *FLAGS, "--cuda-device-only", "-S", SOURCE, "-o", out], capture_output=True, text=True)
@@ -25,12 +25,12 @@ def steps(tmp_path_factory):
         lines = [line.strip() for line in body.split("\n")]
         loads = ["A" if line.startswith("buffer_load") and line.endswith("lds") else "W" if line.startswith("global_load") else
                  "|" if line.startswith("s_barrier") else "" for line in lines]
-        found[int(re.search(r"ILi128ELi(\d+)E", name).group(1))] = "".join(loads).split("|")
+        found[tuple(int(v) for v in re.search(r"ILi(\d+)ELi(\d+)E", name).groups())] = "".join(loads).split("|")
     return found
 
 
-@pytest.mark.parametrize("waves", [4, 8])
-def test_a_steps_activation_loads_come_before_its_code_loads(steps, waves):
-    loop = [s for s in steps[waves][1:] if "A" in s and "W" in s]  # after the prologue, which drains all its loads
-    assert len(loop) >= 4, steps[waves]
-    assert all(re.fullmatch("A{%d}W{3}" % (16 // waves), s) for s in loop), loop
+@pytest.mark.parametrize("rows,waves", [(128, 4), (128, 8), (64, 8)])
+def test_a_steps_activation_loads_come_before_its_code_loads(steps, rows, waves):
+    loop = [s for s in steps[rows, waves][1:] if "A" in s and "W" in s]  # after the prologue, which drains all its loads
+    assert len(loop) >= 4, steps[rows, waves]
+    assert all(re.fullmatch("A{%d}W{3}" % (rows // 8 // waves), s) for s in loop), loop

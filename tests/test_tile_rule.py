@@ -20,7 +20,7 @@ int main() {
         if (route[0] == 'q') {
             const int tile = sq8::choose_blocks_tile(m, n, glu != 0, cus, steps);
             if (tile > sq8::BLOCKS16_ROWS) printf("short %d\n", tile - sq8::BLOCKS16_ROWS);
-            else printf("one %s\n", tile == sq8::BL_128x128 ? "128x128" : "128x256");
+            else printf("one %s\n", tile == sq8::BL_128x128 ? "128x128" : tile == sq8::BL_64x256 ? "64x256" : "128x256");
             continue;
         }
         const int tile = route[0] == 'w' ? sq8::choose_i8_tile(m, n, glu != 0, cus, steps, residual != 0)
@@ -83,6 +83,11 @@ def test_short_products_split_k(rule):
     (("w8a8", 3912, 3072, 0, 256, 24, 0), "128"), (("w8a8", 1975, 6144, 0, 256, 24, 0), "128"),
     (("w8a8", 3277, 1024, 1, 256, 8, 0), "g128x128k2"), (("w8a8", 239, 16000, 0, 256, 8, 0), "g128x128k2"),
     (("w8a8", 498, 18752, 0, 256, 7, 0), "128"), (("w8a8", 512, 3072, 0, 256, 24, 0), "g64x96k4"), (("w8a8", 1531, 3072, 0, 256, 24, 0), "g96x192k2"),
+    # Q8_0: half-height tiles where they fit a round; few K steps; a full chip.
+    (("q8", 575, 7040, 1, 256, 16, 0), "64x256"), (("q8", 1065, 7488, 1, 256, 24, 0), "64x256"), (("q8", 486, 5696, 1, 256, 186, 0), "64x256"),
+    (("q8", 300, 10944, 0, 256, 54, 0), "64x256"), (("q8", 664, 8384, 0, 256, 14, 0), "128x256"),
+    (("q8", 3913, 8960, 0, 256, 18, 0), "128x128"),
+    (("q8", 4096, 12288, 0, 256, 48, 0), "128x256"), (("q8", 77, 12288, 0, 256, 48, 0), "80"), (("q8", 1, 3072, 0, 256, 48, 0), "16"),
 ], ids=str)
 def test_measured_choices(rule, case, tile):
     """Shapes on which another tile measured 10 % slower or more."""
