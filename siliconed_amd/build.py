@@ -30,10 +30,8 @@ SOURCES = [
     ("sq8_short_inst.hip", "sq8_short_f8_packed", ["-DSQ8_WT=1", "-DSQ8_WL=2"]),
     ("sq8_gemm.hip", "sq8_gemm", []),
     ("sq8_gemm_general.hip", "sq8_gemm_general", []),
-    ("sq8_gemm_inst.hip", "sq8_gemm_i8_kn", ["-DSQ8_WT=0", "-DSQ8_WL=0"]),
-    ("sq8_gemm_inst.hip", "sq8_gemm_i8_nk", ["-DSQ8_WT=0", "-DSQ8_WL=1"]),
-    ("sq8_gemm_inst.hip", "sq8_gemm_f8_kn", ["-DSQ8_WT=1", "-DSQ8_WL=0"]),
-    ("sq8_gemm_inst.hip", "sq8_gemm_f8_nk", ["-DSQ8_WT=1", "-DSQ8_WL=1"]),
+    ("sq8_gemm_inst.hip", "sq8_gemm_i8_kn", ["-DSQ8_WT=0"]),
+    ("sq8_gemm_inst.hip", "sq8_gemm_f8_kn", ["-DSQ8_WT=1"]),
     ("sq8_aux.hip", "sq8_aux", []),
     ("sq8_block.hip", "sq8_block", []),
     ("sq8_convrot.hip", "sq8_convrot", []),

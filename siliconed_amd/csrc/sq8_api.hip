@@ -396,8 +396,8 @@ int run_product(sq8_ctx *ctx, const Product &q, double *gpu_seconds) {
     } else {
         const int wl = q.w_layout == SQ8_KN ? sq8::W_KN : sq8::W_NK;
         const int tile = sq8::choose_tile(q.m, n_out, is_glu(q.epilogue), ctx->cus);
-        const bool fast = p.a_vec && p.w_vec && q.k > 0 && q.k % 64 == 0 && cols_per_half >= 4 &&
-                          (q.w_layout == SQ8_NK || (cols_per_half % 4) == 0);
+        // ([N, K] codes that could be read so took the branch above.)
+        const bool fast = wl == sq8::W_KN && p.a_vec && p.w_vec && q.k > 0 && q.k % 64 == 0 && cols_per_half % 4 == 0;
         e = sq8::launch_gemm(p, fast, tile, wt, wl, q.epilogue, out, ctx->stream);
     }
     if (e != hipSuccess) return hip_status(e);

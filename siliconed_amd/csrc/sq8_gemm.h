@@ -43,9 +43,8 @@ struct GemmArgs {
 enum Tile { TILE_256x256 = 0, TILE_128x128 = 1 };
 
 int choose_tile(int M, int N_out, bool glu, int cus);
-// `fast`: the branch-free kernels, valid when A rows and W rows/columns can be read with vector
-// loads (alignment), K is a positive multiple of 64, and there are at least 4 weight columns (per
-// GLU half) with a [K, N] weight's column count a multiple of 4.
+// `fast`: the branch-free kernels on [K, N] codes, valid when A rows and W columns can be read with vector loads
+// (alignment), K is a positive multiple of 64, and the weight columns (per GLU half) are a positive multiple of 4.
 hipError_t launch_gemm(const GemmArgs &p, bool fast, int tile, int wt, int wl, int epi, int out, hipStream_t stream);
 
 // The weight-direct kernels (sq8_wdirect_inst.hip): [N, K] or packed weights, K a multiple of 64,

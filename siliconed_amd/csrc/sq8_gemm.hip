@@ -6,10 +6,8 @@
 
 namespace sq8 {
 
-hipError_t launch_fast_0_0(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
-hipError_t launch_fast_0_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
-hipError_t launch_fast_1_0(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
-hipError_t launch_fast_1_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
+hipError_t launch_fast_0(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
+hipError_t launch_fast_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 hipError_t launch_general(const GemmArgs &p, int wt, int wl, int epi, int out, hipStream_t stream);
 hipError_t launch_short_0_1(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
 hipError_t launch_short_0_2(const GemmArgs &p, int tile, int epi, int out, hipStream_t stream);
@@ -239,11 +237,8 @@ int choose_tile(int M, int N_out, bool glu, int cus) {
 
 hipError_t launch_gemm(const GemmArgs &p, bool fast, int tile, int wt, int wl, int epi, int out, hipStream_t stream) {
     if (!fast) return launch_general(p, wt, wl, epi, out, stream);
-    if (wt == W_INT8 && wl == W_KN) return launch_fast_0_0(p, tile, epi, out, stream);
-    if (wt == W_INT8 && wl == W_NK) return launch_fast_0_1(p, tile, epi, out, stream);
-    if (wt == W_FP8 && wl == W_KN) return launch_fast_1_0(p, tile, epi, out, stream);
-    if (wt == W_FP8 && wl == W_NK) return launch_fast_1_1(p, tile, epi, out, stream);
-    return hipErrorInvalidValue;
+    if (wl != W_KN) return hipErrorInvalidValue;
+    return wt == W_INT8 ? launch_fast_0(p, tile, epi, out, stream) : launch_fast_1(p, tile, epi, out, stream);
 }
 
 }  // namespace sq8

@@ -192,6 +192,7 @@ gemm_q8_kernel(const GemmArgs p) {
     constexpr int SA = BM * 128, SB = BN * 128; // bytes of one stage of A, of W
     constexpr int B0 = 2 * SA;                // W stages follow the two A stages
     static_assert(BN % 128 == 0 || WL == W_NK, "the [K,N] loader takes 128-column slabs");
+    static_assert(!FAST || WL == W_KN, "[N,K] codes of whole, aligned rows go to the weight-direct kernels");
     static_assert(!GLU || (FN % 2 == 0), "GLU pairs blocks inside a wave");
 
     // LDS: [A stage 0][A stage 1][W stage 0][W stage 1], each row 64 bf16 of K.
@@ -280,19 +281,15 @@ gemm_q8_kernel(const GemmArgs p) {
 #pragma unroll
         for (int j = 0; j < W_ITEMS; ++j) {
             if constexpr (WL == W_NK) {
-                if constexpr (FAST) {
-                    rw_nk[j] = gld<u32x4>(Wg, w_goff[j] + (uint32_t)k0);
-                } else {
-                    const int k = k0 + (tid & 3) * 16;
-                    uint32_t d[4] = {0, 0, 0, 0};
+                const int k = k0 + (tid & 3) * 16;
+                uint32_t d[4] = {0, 0, 0, 0};
 #pragma unroll
-                    for (int x = 0; x < 16; ++x) {
-                        const uint32_t b =
-                            (w_col[j] >= 0 && k + x < p.K) ? gld<uint8_t>(Wg, w_goff[j] + (uint32_t)(k0 + x)) : 0u;
-                        d[x >> 2] |= b << (8 * (x & 3));
-                    }
-                    rw_nk[j] = u32x4{d[0], d[1], d[2], d[3]};
+                for (int x = 0; x < 16; ++x) {
+                    const uint32_t b =
+                        (w_col[j] >= 0 && k + x < p.K) ? gld<uint8_t>(Wg, w_goff[j] + (uint32_t)(k0 + x)) : 0u;
+                    d[x >> 2] |= b << (8 * (x & 3));
                 }
+                rw_nk[j] = u32x4{d[0], d[1], d[2], d[3]};
             } else {
                 const uint32_t base = w_goff[j] + (uint32_t)k0 * (uint32_t)p.ldw;
                 if constexpr (FAST) {

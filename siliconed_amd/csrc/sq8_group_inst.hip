@@ -18,10 +18,13 @@ hipError_t SQ8_CAT(launch_group_, SQ8_CAT(SQ8_MATH, SQ8_CAT(_, SQ8_CAT(SQ8_WT, S
     // built for it), as many as fit the LDS beside the groups'.
 #define SQ8_SHAPE(I, BM, NW, KS, BF16, I8, F32)                                                                       \
     case I: {                                                                                                         \
-        constexpr int NAS = MATH == GM_I8 ? I8 : MATH == GM_F32 ? F32 : BF16;                               \
+        constexpr int NAS = MATH == GM_I8 ? I8 : MATH == GM_F32 ? F32 : BF16;                                         \
+        static_assert(group_shapes[I].rows == BM && group_shapes[I].cols == 32 * NW && group_shapes[I].groups == KS); \
+        static_assert((NAS > 0) == (group_shapes[I].cost[MATH].us_step > 0.0f), "priced where it is built");          \
         if constexpr (NAS > 0) return grp::launch_group<MATH, WT, WL, BM, NW, KS, NAS>(p, epi, out, stream);          \
         break;                                                                                                        \
     }
+    static_assert(kGroupShapes == 15, "a case for each");
     switch (shape) {
         SQ8_SHAPE(0, 32, 1, 8, 0, 4, 0)
         SQ8_SHAPE(1, 32, 2, 8, 0, 2, 0)
