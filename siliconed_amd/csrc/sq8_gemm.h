@@ -51,10 +51,9 @@ hipError_t launch_gemm(const GemmArgs &p, bool fast, int tile, int wt, int wl, i
 // A aligned for 16-byte loads. `tile`: WD_256 (256 × 256, one workgroup per CU), WD_224 (224 × 256, the
 // same kernel), WD_128 (128 × 256, two workgroups per CU), WD_GEMV (M ≤ 16 in 16-column groups on 16 × 16 MFMAs, every
 // K step's loads issued far ahead), the skinny-M kernel with 64- or 32-row tiles of one 64-column slab and the K steps
-// split over four waves (WD_SKINNY64, WD_SKINNY32), or a K-group tile's id (below). By the SQ8_TILE knob only: WD_64
-// (64 × 256, one per CU), WD_32 (32 × 256, two per CU), WD_64N (64 × 128, a 32-column block a wave, two per CU; not
-// GLU), WD_64x192 (64 × 192, six waves of one 32-column block; not GLU): the K-group tiles' shapes without groups, in
-// WD_128's order of sums.
+// split over four waves (WD_SKINNY64, WD_SKINNY32), a K-group tile's id (below), or 64 rows without groups in WD_128's order of sums: WD_64
+// (64 × 256, one per CU), WD_64N (64 × 128, a 32-column block a wave, two per CU; not GLU). By the SQ8_TILE knob only:
+// WD_32 (32 × 256, two per CU), WD_64x192 (64 × 192, six waves of one 32-column block; not GLU), WD_SKINNY64.
 enum WdTile { WD_256 = 0, WD_128 = 1, WD_SKINNY64 = 2, WD_SKINNY32 = 3, WD_64 = 4, WD_32 = 5, WD_224 = 6, WD_64N = 7, WD_64x192 = 8,
               WD_GEMV = 9 };
 // The tile for an M × N product (GLU: N = 2h) of `steps` weight K steps of 64, `f32` on the fp32 route (three parts of
@@ -74,8 +73,10 @@ hipError_t launch_wdirect(const GemmArgs &p, int tile, int wt, int wl, int epi, 
 
 // The K-group kernels (sq8_group_kernel.h): `rows` × `cols` tiles (cols: weight columns) whose K steps split over
 // `groups` wave groups; GLU products take those of an even number of 32-column blocks. What a round of tiles on
-// the CUs, one a CU, takes by kind of product: us + us_step · (weight K steps) microseconds, fitted to 256 and 512
-// tiles at K = 1024, 3072 and 8192 (graph launches, the launch's own 2.5 µs taken off); us_step 0: not built for it.
+// the CUs, one a CU, takes by kind of product: us + us_step · (weight K steps) microseconds, the launch's own 2.5 µs (and
+// the fp32 route's split pass) taken off; us_step 0: not built for it. W8A8: fitted to 256 and 512 tiles at K = 1024, 3072
+// and 8192; the others to 857 and 596 shapes of 17 to 5000 rows, K 256 to 12288, plain and GLU, weights in and out of
+// the caches (each within 4 to 7 %).
 enum GroupMath { GM_BF16 = 0, GM_I8 = 1, GM_F32 = 2 };
 struct GroupCost {
     float us, us_step;
@@ -89,19 +90,19 @@ constexpr int GROUP_TILE0 = 100;  // tile ids of the K-group kernels: GROUP_TILE
 constexpr GroupShape group_shapes[] = {
     {32, 32, 8, "g32x32k8", {{}, {0.65f, 0.104f}, {}}},
     {32, 64, 8, "g32x64k8", {{}, {0.55f, 0.165f}, {}}},
-    {32, 32, 4, "g32x32k4", {{1.16f, 0.064f}, {}, {2.20f, 0.277f}}},
-    {32, 64, 4, "g32x64k4", {{1.74f, 0.089f}, {}, {2.11f, 0.352f}}},
-    {64, 64, 4, "g64x64k4", {{2.64f, 0.151f}, {1.60f, 0.204f}, {5.15f, 0.511f}}},
-    {64, 96, 4, "g64x96k4", {{3.42f, 0.212f}, {2.65f, 0.243f}, {6.26f, 0.620f}}},
-    {64, 128, 4, "g64x128k4", {{2.81f, 0.284f}, {2.30f, 0.325f}, {7.01f, 0.746f}}},
-    {64, 128, 2, "g64x128k2", {{2.56f, 0.290f}, {}, {6.77f, 0.752f}}},
-    {64, 192, 2, "g64x192k2", {{3.79f, 0.407f}, {}, {8.56f, 1.032f}}},
-    {96, 96, 4, "g96x96k4", {{3.88f, 0.299f}, {3.60f, 0.312f}, {9.95f, 0.822f}}},
-    {96, 128, 4, "g96x128k4", {{4.23f, 0.371f}, {4.40f, 0.408f}, {}}},
-    {128, 96, 4, "g128x96k4", {{4.59f, 0.382f}, {4.70f, 0.402f}, {}}},
-    {128, 128, 2, "g128x128k2", {{5.61f, 0.482f}, {6.30f, 0.493f}, {14.93f, 1.284f}}},
-    {96, 192, 2, "g96x192k2", {{6.10f, 0.520f}, {6.30f, 0.560f}, {11.95f, 1.425f}}},
-    {128, 192, 2, "g128x192k2", {{7.80f, 0.656f}, {8.70f, 0.694f}, {13.96f, 1.848f}}},
+    {32, 32, 4, "g32x32k4", {{1.85f, 0.077f}, {}, {1.09f, 0.198f}}},
+    {32, 64, 4, "g32x64k4", {{2.55f, 0.107f}, {}, {1.40f, 0.280f}}},
+    {64, 64, 4, "g64x64k4", {{3.55f, 0.161f}, {1.60f, 0.204f}, {2.81f, 0.366f}}},
+    {64, 96, 4, "g64x96k4", {{3.87f, 0.210f}, {2.65f, 0.243f}, {3.73f, 0.472f}}},
+    {64, 128, 4, "g64x128k4", {{4.28f, 0.277f}, {2.30f, 0.325f}, {4.38f, 0.591f}}},
+    {64, 128, 2, "g64x128k2", {{4.04f, 0.263f}, {}, {3.81f, 0.628f}}},
+    {64, 192, 2, "g64x192k2", {{5.11f, 0.390f}, {}, {5.18f, 0.893f}}},
+    {96, 96, 4, "g96x96k4", {{5.08f, 0.273f}, {3.60f, 0.312f}, {5.12f, 0.666f}}},
+    {96, 128, 4, "g96x128k4", {{5.61f, 0.357f}, {4.40f, 0.408f}, {}}},
+    {128, 96, 4, "g128x96k4", {{5.72f, 0.375f}, {4.70f, 0.402f}, {}}},
+    {128, 128, 2, "g128x128k2", {{6.22f, 0.443f}, {6.30f, 0.493f}, {6.75f, 1.131f}}},
+    {96, 192, 2, "g96x192k2", {{6.59f, 0.482f}, {6.30f, 0.560f}, {7.02f, 1.207f}}},
+    {128, 192, 2, "g128x192k2", {{8.00f, 0.606f}, {8.70f, 0.694f}, {8.85f, 1.553f}}},
 };
 constexpr int kGroupShapes = (int)(sizeof(group_shapes) / sizeof(group_shapes[0]));
 hipError_t launch_group(const GemmArgs &p, int math, int shape, int wt, int wl, int epi, int out, hipStream_t stream);

@@ -105,34 +105,34 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
     // in flight, the activation read once per workgroup. Kernel traces at K = 3072, N = 3072 (int8 packed, bias): M = 1
     // 4.10 µs against the skinny kernel's 7.44, M = 16 5.95 against 8.73; two groups, SiLU-GLU: M = 3, N = 8192 5.8
     // against 8.5, M = 16 7.3 against 9.4; three, M = 1: N = 9216 8.9 against 9.7, N = 12288 10.6 against 11.4. With the
-    // activation not in its LDS, to four rows of up to two groups (16 × 6144 × 3072 11.3 against 8.5 µs for a K-group
-    // tile; one row of three, 1 × 7808 × 10944, 23.5 against 18.8), and one group of GLU columns
-    // (SiLU-GLU 10 × 3840 × 3072 7.2 against 9.1 for a K-group tile, 5 × 1152 × 3200 4.8 against 5.9).
+    // activation not in its LDS, to four rows of up to two groups; one row of three to 32 steps (1 × 832 × 8447 4.7 against
+    // 6.0 for a K-group tile, 1 × 7808 × 10944 23.5 against 18.8); ten rows (the fp32 route, with three times the activation,
+    // six past ten steps: 10 × 576 × 1152 6.6 against 7.2) of one group (6 × 12160 × 166 11.3 against 14.2, 5 × 1472 × 2944 4.7 against 5.4; by 11 rows level, 16 × 6144 ×
+    // 3072 11.3 against 8.5); one group of GLU columns (SiLU-GLU 10 × 3840 × 3072 7.2 against 9.1, 5 × 1152 × 3200 4.8 against
+    // 5.9).
     const int groups16 = glu ? (N / 2 + 7) / 8 : (N + 15) / 16;
     const bool staged = gemv_x_in_lds(M, kt);
-    if (M <= 16 && ((groups16 <= 2 * cus && (M <= 4 || staged)) || (glu && groups16 <= cus) ||
-                    (M == 1 && !glu && staged && groups16 <= 3 * cus)))
+    if (M <= 16 && ((groups16 <= 2 * cus && (M <= 4 || staged)) || (groups16 <= cus && (glu || M <= (f32 && steps > 10 ? 6 : 10))) ||
+                    (M == 1 && !glu && (staged || kt <= 32) && groups16 <= 3 * cus)))
         return WD_GEMV;
     // Up to 16 rows on a weight wider than 3/4 of the CUs' 64-column slabs, the skinny kernel (a slab a workgroup, four
     // a CU): its many small workgroups stream the weight best (1 × 3072 × 18432 13.7 µs against 16.0 in 32 × 64 tiles, 8
-    // × 9216 7.9 against 7.2). The fp32 route's K-group tiles load the codes once for three parts (16 × 12288 17.8
+    // × 9216 7.9 against 7.2), and on short K than half of them (12 × 640 × 11968 5.4 against 5.8; 10 × 6912 × 9216 15.1
+    // against 14.2), unless its rows are stored value by value (below). The fp32 route's K-group tiles load the codes once for three parts (16 × 12288 17.8
     // against 21.9).
     const int blocks = glu ? 2 * ((N / 2 + 31) / 32) : (N + 31) / 32;  // 32-column blocks
-    if (M <= 16 && !f32 && (blocks + 1) / 2 >= cus * 3 / 4) return WD_SKINNY32;
-    // Else the tile of the least estimated time: µs a round of tiles, one a CU (128 × 256: two a CU, or one in a round
-    // of at most one a CU), measured at K = 1024, 3072 and 8192 as the K-group tiles' (GroupShape). Few tiles go to the
-    // K-group tiles: more CUs, and eight to sixteen waves a CU with their loads in flight whatever the tile; many to
-    // the 256- and 224-row tiles of one workgroup a CU (the least widening and operand traffic), the height whose
-    // rounds cover the fewest rows. Measured (µs, the thresholds of before → this): 512 × 3072 × 3072 16.5 → 14.6, 1531
-    // × 3072 × 3072 41.8 → 33.0, 200 × 3072 × 6144 16.4 → 14.0; SiLU-GLU 333 × 3840 × 20480 74.4 → 55.2, 77 × 3840 ×
-    // 20480 30.6 → 24.1, 20 × 3072 × 6144 10.0 → 7.0, 43 × 3424 × 10880 23.1 → 14.8; fp32 route 1531 × 3072 × 3072
-    // 141 → 87, 18 × 6592 × 64 36 → 20, 176 × 8512 × 64 117 → 34.
-    struct Round { float us, us_step; };
-    const Round two = f32 ? Round{21.5f, 5.07f} : Round{8.2f, 1.605f}, one = f32 ? Round{28.5f, 2.66f} : Round{7.0f, 0.905f};
-    const Round r224 = f32 ? Round{32.0f, 4.00f} : Round{7.9f, 1.28f}, r256 = f32 ? Round{35.0f, 4.56f} : Round{9.0f, 1.445f};
-    auto us = [&](const Round &r) { return r.us + r.us_step * (float)steps; };
-    auto tiles = [&](int bm) { return tile_count(M, bm, blocks, 8); };
-    float best = pairs_us(tiles(128), cus, us(two), us(one));
+    const int slabs = (blocks + 1) / 2;
+    const bool ragged = (glu ? N / 2 : N) % 8 != 0;
+    if (M <= 16 && !f32 && (slabs >= cus * 3 / 4 || (!glu && !ragged && slabs > cus / 2 && steps <= 40))) return WD_SKINNY32;
+    // Else the tile of the least estimated time: µs a round of tiles, one a CU (128 × 256 and 64 × 128: two a CU, or one in a
+    // round of at most one a CU), fitted as the K-group tiles' (GroupShape). Few tiles go to the K-group tiles: more CUs, and
+    // eight to sixteen waves a CU with their loads in flight whatever the tile; many to the 256- and 224-row tiles of one
+    // workgroup a CU (the least widening and operand traffic), the height whose rounds cover the fewest rows. Measured
+    // (µs, thresholds on tile counts → estimates): 512 × 3072 × 3072 16.5 → 14.6, 1531 × 3072 × 3072 41.8 → 33.0, 200 × 3072 ×
+    // 6144 16.4 → 14.0; SiLU-GLU 333 × 3840 × 20480 62.6 → 55.2, 77 × 3840 × 20480 30.6 → 24.1, 20 × 3072 × 6144 10.0 → 7.0, 43
+    // × 3424 × 10880 23.1 → 14.8; fp32 route 1531 × 3072 × 3072 130 → 87, 18 × 6592 × 64 36 → 20, 176 × 8512 × 64 117 → 34.
+    auto tiles = [&](int rows, int nb) { return tile_count(M, rows, blocks, nb); };
+    float best = INFINITY;
     int tile = WD_128;
     auto take = [&](int t, float time) {
         if (time < best) {
@@ -140,21 +140,54 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
             tile = t;
         }
     };
+    struct One {  // a round of a tile of one workgroup a CU; `later`: more, past the first
+        float us, us_step, later;
+        float of(float n, int cus, int steps) const {
+            return rounds_us(n, cus, us + us_step * (float)steps) + later * floorf((n - 1.0f) / (float)cus);
+        }
+    };
+    struct Two {
+        float two, two_step, one, one_step;
+        float of(float n, int cus, int steps, float ragged_two, float ragged_one) const {
+            return pairs_us(n, cus, two + two_step * (float)steps + ragged_two, one + one_step * (float)steps + ragged_one);
+        }
+    };
     // By the shape alone: the 256- and 224-row kernel also wants its scales and outputs aligned, but a choice by alignment
     // or output type would give one call two sets of bits (launch_wdirect takes 128-row tiles, the same sums, where that
     // kernel cannot serve the product).
-    if (glu ? N / 2 % 32 == 0 : N % 64 == 0) {
-        take(WD_256, rounds_us(tiles(256), cus, us(r256)));
-        take(WD_224, rounds_us(tiles(224), cus, us(r224)));
-    }
+    const bool whole = glu ? N / 2 % 32 == 0 : N % 64 == 0;
     // From 4096 rows on and past 1024 columns no K groups: the tall tiles sum each output's K in one sequence, so a host that
     // chunks its rows by that many gets the bits of one call. What it costs where 128 × 192 tiles of two groups would fill
-    // the rounds better (µs): 5760 × 3072 × 3072 115.9 → 119.9, with the residual 124.6 → 141.8, fp32 route 309 → 375.
-    if (M >= 4096 && N > 1024) return tile;
-    if (f32)
-        each_group<GM_F32>(M, blocks, glu, cus, steps, 0.0f, 0.0f, take);
-    else
-        each_group<GM_BF16>(M, blocks, glu, cus, steps, 0.0f, 0.0f, take);
+    // the rounds better (µs): 5760 × 3072 × 3072 115.9 → 119.9, with the residual 124.6 → 141.8, fp32 route 309 → 375. Priced
+    // at the clock of long runs of such products.
+    if (M >= 4096 && N > 1024) {
+        const Two t128 = f32 ? Two{21.5f, 5.07f, 28.5f, 2.66f} : Two{8.2f, 1.605f, 7.0f, 0.905f};
+        take(WD_128, t128.of(tiles(128, 8), cus, steps, 0.0f, 0.0f));
+        if (whole) {
+            take(WD_256, (f32 ? One{35.0f, 4.56f, 0.0f} : One{9.0f, 1.445f, 0.0f}).of(tiles(256, 8), cus, steps));
+            take(WD_224, (f32 ? One{32.0f, 4.00f, 0.0f} : One{7.9f, 1.28f, 0.0f}).of(tiles(224, 8), cus, steps));
+        }
+        return tile;
+    }
+    // Output rows that are not whole 16 bytes of bf16 are stored value by value in these kernels, not in the K-group ones
+    // (1032 × 512 × 6559 33.4 µs in 128 × 256 and 25.5 in 96 × 192 tiles).
+    const Two t128 = f32 ? Two{9.5f, 4.48f, 7.1f, 2.53f} : Two{8.7f, 1.464f, 5.8f, 0.921f};
+    take(WD_128, t128.of(tiles(128, 8), cus, steps, ragged ? 20.0f : 0.0f, ragged ? 14.0f : 0.0f));
+    if (whole) {
+        take(WD_256, (f32 ? One{12.8f, 3.67f, 1.0f} : One{10.7f, 1.271f, 5.2f}).of(tiles(256, 8), cus, steps));
+        take(WD_224, (f32 ? One{11.2f, 3.28f, 2.3f} : One{9.5f, 1.151f, 4.7f}).of(tiles(224, 8), cus, steps));
+    }
+    // A K-group round past the first costs 0.8 µs more.
+    if (f32) {
+        each_group<GM_F32>(M, blocks, glu, cus, steps, 0.0f, 0.8f, take);
+    } else {
+        each_group<GM_BF16>(M, blocks, glu, cus, steps, 0.0f, 0.8f, take);
+        // 64 rows without groups: 64 × 128 of one-block waves, two a CU, and for the GLU epilogues (and wide plain ones) 64 × 256.
+        // They win on few K steps (139 × 384 × 17856 8.2 µs against 12.6 in 64 × 128 of two groups; SiLU-GLU 652 × 3776 ×
+        // 5120 33.1 against 40.1) and where an odd count of steps leaves only the tiles of four groups (2199 × 12096 × 1728).
+        if (!glu) take(WD_64N, Two{3.5f, 0.500f, 2.8f, 0.348f}.of(tiles(64, 4), cus, steps, ragged ? 5.4f : 0.0f, ragged ? 4.6f : 0.0f));
+        take(WD_64, One{ragged ? 12.2f : 4.3f, 0.540f, -0.8f}.of(tiles(64, 8), cus, steps));
+    }
     return tile;
 }
 

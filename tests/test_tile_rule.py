@@ -30,6 +30,8 @@ int main() {
             printf("%s %s\n", g.groups == 2 ? "two" : g.groups == 4 ? "four" : "eight", g.name);
         } else if (route[0] == 'w' || tile == sq8::WD_128 || tile == sq8::WD_224 || tile == sq8::WD_256) {
             printf("one %s\n", route[0] == 'w' || tile == sq8::WD_128 ? "128" : tile == sq8::WD_224 ? "224" : "256");
+        } else if (tile == sq8::WD_64 || tile == sq8::WD_64N) {
+            printf("one %s\n", tile == sq8::WD_64 ? "64" : "64n");
         } else {
             printf("short %s\n", tile == sq8::WD_GEMV ? "gemv" : "skinny");
         }
@@ -79,6 +81,16 @@ def test_short_products_split_k(rule):
     # Up to 16 rows of one group of GLU columns, the activation not in the short-M kernel's LDS; one row of three groups.
     (("bf16", 10, 3072, 1, 256, 60, 0), "gemv"), (("bf16", 5, 3200, 1, 256, 18, 0), "gemv"), (("bf16", 11, 256, 1, 256, 26, 0), "gemv"),
     (("bf16", 1, 10944, 0, 256, 122, 0), "g32x64k4"), (("bf16", 1, 9216, 0, 256, 48, 0), "gemv"), (("bf16", 16, 3072, 0, 256, 96, 0), "g32x32k4"),
+    # The same of one group of plain columns, to ten rows (fp32 route: six).
+    (("bf16", 6, 4043, 0, 256, 59, 0), "gemv"), (("bf16", 5, 64, 0, 256, 53, 0), "gemv"), (("fp32", 6, 2295, 0, 256, 129, 0), "gemv"),
+    (("bf16", 16, 2880, 0, 256, 60, 0), "g32x32k4"), (("fp32", 13, 2295, 0, 256, 145, 0), "g32x32k4"),
+    # One row of three groups on short K; the skinny kernel's slabs past half the CUs.
+    (("bf16", 1, 8447, 0, 256, 13, 0), "gemv"), (("bf16", 6, 8352, 0, 256, 11, 0), "skinny"), (("bf16", 10, 9216, 0, 256, 108, 0), "g32x64k4"),
+    # 64 rows without groups: few K steps, odd counts of them; output rows of odd values; a second round of small tiles.
+    (("bf16", 2840, 1152, 0, 256, 7, 0), "64n"), (("bf16", 139, 17856, 0, 256, 6, 0), "64n"), (("bf16", 652, 5120, 1, 256, 59, 0), "64"),
+    (("bf16", 1119, 2944, 0, 256, 9, 0), "64n"), (("bf16", 1032, 6559, 0, 256, 8, 0), "g128x128k2"),
+    (("bf16", 21, 16576, 0, 256, 46, 0), "g64x96k4"), (("bf16", 441, 12800, 1, 256, 24, 0), "128"),
+    (("fp32", 855, 8064, 0, 256, 12, 0), "128"), (("fp32", 188, 4640, 0, 256, 4, 0), "g64x64k4"),
     # W8A8: a round of more than one and fewer than two workgroups a CU; rounds of K-group tiles past the first.
     (("w8a8", 3912, 3072, 0, 256, 24, 0), "128"), (("w8a8", 1975, 6144, 0, 256, 24, 0), "128"),
     (("w8a8", 3277, 1024, 1, 256, 8, 0), "g128x128k2"), (("w8a8", 239, 16000, 0, 256, 8, 0), "g128x128k2"),
