@@ -43,18 +43,18 @@ RIDGE = PEAK_BF16_TFLOPS * 1e12 / (PEAK_HBM_GBS * 1e9)
 _TRAFFIC_SRC = "profiles/hbm_traffic_by_workload.md"
 TRAFFIC = {
     ("c1_up", "packed"): (403.6e6, _TRAFFIC_SRC),
-    ("c2_skinny", "packed"): (34.91e6, _TRAFFIC_SRC),
-    ("c0", "packed"): (56.98e6, _TRAFFIC_SRC),
+    ("c2_skinny", "packed"): (34.89e6, _TRAFFIC_SRC),
+    ("c0", "packed"): (50.70e6, _TRAFFIC_SRC),
     ("skinny_m1", "packed"): (9.68e6, _TRAFFIC_SRC),
     ("skinny_m16", "packed"): (10.52e6, _TRAFFIC_SRC),
-    ("skinny_m64", "packed"): (13.18e6, _TRAFFIC_SRC),
+    ("skinny_m64", "packed"): (13.16e6, _TRAFFIC_SRC),
     ("c1_down", "packed"): (450.35e6, _TRAFFIC_SRC),
     ("c2_qkv", "packed"): (415.51e6, _TRAFFIC_SRC),
     ("c3_gate_up", "packed"): (715.93e6, _TRAFFIC_SRC),
     ("c3_down", "packed"): (367.51e6, _TRAFFIC_SRC),
     ("c3_plain", "packed"): (478.92e6, _TRAFFIC_SRC),
     ("c1_w8a8", "packed"): (472.42e6, _TRAFFIC_SRC),
-    ("c1_q8", "packed"): (592.23e6, _TRAFFIC_SRC),
+    ("c1_q8", "packed"): (592.16e6, _TRAFFIC_SRC),
     ("c1_f32", "packed"): (1007.54e6, _TRAFFIC_SRC),
     ("c1_convrot", "packed"): (403.59e6, _TRAFFIC_SRC)}
 GAMMA = np.uint64(0x9E3779B97F4A7C15)

@@ -30,8 +30,9 @@
 // (the next step's first fragments and codes are taken during the last group). The order of every sum is unchanged.
 // Measured (µs, the groups against the plain order): one row of tiles alone, K = 3072, 52.4 → 46.5 in 128 × 256 and
 // 33.6 in 128 × 128; 1021 × 3072 × 3072 54.9 → 40.3 (128 × 128, two workgroups a CU: one's epilogue under the other's
-// MFMAs). On a full chip the clock follows the power (4096 × 3072 × 12288, the same 780 k cycles: 403 µs, with every
-// activation zero 349, with every code zero 321), so there the cycles saved come back as 2.5 % (400 → 391 µs).
+// MFMAs). On a full chip the two still add (4096 × 3072 × 12288: 81.5 cycles an MFMA, 32 + 12.7 vector instructions of 4),
+// 400 → 378 to 391 µs; a fifth of that is the clock under power (303 µs with every activation or every
+// code zero).
 // 64 × 256 tiles (two row blocks a wave: two groups a step, each widening a whole K block) serve products that leave a
 // round of the taller ones part empty: SiLU-GLU 575 × 1024 × 7040 17.5 µs (28 tiles of 128 × 256 a row 23.5), 1065 ×
 // 1536 × 7488 42.2 (128 × 128 51.5).
