@@ -106,13 +106,13 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
     // 4.10 µs against the skinny kernel's 7.44, M = 16 5.95 against 8.73; two groups, SiLU-GLU: M = 3, N = 8192 5.8
     // against 8.5, M = 16 7.3 against 9.4; three, M = 1: N = 9216 8.9 against 9.7, N = 12288 10.6 against 11.4. With the
     // activation not in its LDS, to four rows of up to two groups; one row of three to 32 steps (1 × 832 × 8447 4.7 against
-    // 6.0 for a K-group tile, 1 × 7808 × 10944 23.5 against 18.8); ten rows (the fp32 route, with three times the activation,
-    // six past ten steps: 10 × 576 × 1152 6.6 against 7.2) of one group (6 × 12160 × 166 11.3 against 14.2, 5 × 1472 × 2944 4.7 against 5.4; by 11 rows level, 16 × 6144 ×
-    // 3072 11.3 against 8.5); one group of GLU columns (SiLU-GLU 10 × 3840 × 3072 7.2 against 9.1, 5 × 1152 × 3200 4.8 against
-    // 5.9).
+    // 6.0 for a K-group tile, 1 × 7808 × 10944 23.5 against 18.8); ten rows of one group (6 × 12160 × 166 11.3 against 14.2,
+    // 5 × 1472 × 2944 4.7 against 5.4; by 11 rows level, 16 × 6144 × 3072 11.3 against 8.5; the fp32 route four: 3 % on
+    // average to six, and the K-group tiles' sums are nearer, 2.8e-7 against 3.6e-7 at K = 3136); one group of GLU columns
+    // (SiLU-GLU 10 × 3840 × 3072 7.2 against 9.1, 5 × 1152 × 3200 4.8 against 5.9).
     const int groups16 = glu ? (N / 2 + 7) / 8 : (N + 15) / 16;
     const bool staged = gemv_x_in_lds(M, kt);
-    if (M <= 16 && ((groups16 <= 2 * cus && (M <= 4 || staged)) || (groups16 <= cus && (glu || M <= (f32 && steps > 10 ? 6 : 10))) ||
+    if (M <= 16 && ((groups16 <= 2 * cus && (M <= 4 || staged)) || (groups16 <= cus && (glu || M <= (f32 ? 4 : 10))) ||
                     (M == 1 && !glu && (staged || kt <= 32) && groups16 <= 3 * cus)))
         return WD_GEMV;
     // Up to 16 rows on a weight wider than 3/4 of the CUs' 64-column slabs, the skinny kernel (a slab a workgroup, four
@@ -172,10 +172,13 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
     // Output rows that are not whole 16 bytes of bf16 are stored value by value in these kernels, not in the K-group ones
     // (1032 × 512 × 6559 33.4 µs in 128 × 256 and 25.5 in 96 × 192 tiles).
     const Two t128 = f32 ? Two{9.5f, 4.48f, 7.1f, 2.53f} : Two{8.7f, 1.464f, 5.8f, 0.921f};
-    take(WD_128, t128.of(tiles(128, 8), cus, steps, ragged ? 20.0f : 0.0f, ragged ? 14.0f : 0.0f));
+    // Where the two are within 5 % the K groups, whose sums are nearer too (K = 3072, errors against 64 bits: fp32 route 7.2e-7
+    // in one sequence, 3.8e-7 in two groups, 2.7e-7 in four; bf16 route 1.5e-7, 1.0e-7, 0.8e-7).
+    const float nearer = f32 ? 1.05f : 1.0f;
+    take(WD_128, nearer * t128.of(tiles(128, 8), cus, steps, ragged ? 20.0f : 0.0f, ragged ? 14.0f : 0.0f));
     if (whole) {
-        take(WD_256, (f32 ? One{12.8f, 3.67f, 1.0f} : One{10.7f, 1.271f, 5.2f}).of(tiles(256, 8), cus, steps));
-        take(WD_224, (f32 ? One{11.2f, 3.28f, 2.3f} : One{9.5f, 1.151f, 4.7f}).of(tiles(224, 8), cus, steps));
+        take(WD_256, nearer * (f32 ? One{12.8f, 3.67f, 1.0f} : One{10.7f, 1.271f, 5.2f}).of(tiles(256, 8), cus, steps));
+        take(WD_224, nearer * (f32 ? One{11.2f, 3.28f, 2.3f} : One{9.5f, 1.151f, 4.7f}).of(tiles(224, 8), cus, steps));
     }
     // A K-group round past the first costs 0.8 µs more.
     if (f32) {
@@ -185,8 +188,8 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
         // 64 rows without groups: 64 × 128 of one-block waves, two a CU, and for the GLU epilogues (and wide plain ones) 64 × 256.
         // They win on few K steps (139 × 384 × 17856 8.2 µs against 12.6 in 64 × 128 of two groups; SiLU-GLU 652 × 3776 ×
         // 5120 33.1 against 40.1) and where an odd count of steps leaves only the tiles of four groups (2199 × 12096 × 1728).
-        if (!glu) take(WD_64N, Two{3.5f, 0.500f, 2.8f, 0.348f}.of(tiles(64, 4), cus, steps, ragged ? 5.4f : 0.0f, ragged ? 4.6f : 0.0f));
-        take(WD_64, One{ragged ? 12.2f : 4.3f, 0.540f, -0.8f}.of(tiles(64, 8), cus, steps));
+        if (!glu) take(WD_64N, 1.05f * Two{3.5f, 0.500f, 2.8f, 0.348f}.of(tiles(64, 4), cus, steps, ragged ? 5.4f : 0.0f, ragged ? 4.6f : 0.0f));
+        take(WD_64, 1.05f * One{ragged ? 12.2f : 4.3f, 0.540f, -0.8f}.of(tiles(64, 8), cus, steps));
     }
     return tile;
 }

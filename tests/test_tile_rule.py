@@ -81,8 +81,8 @@ def test_short_products_split_k(rule):
     # Up to 16 rows of one group of GLU columns, the activation not in the short-M kernel's LDS; one row of three groups.
     (("bf16", 10, 3072, 1, 256, 60, 0), "gemv"), (("bf16", 5, 3200, 1, 256, 18, 0), "gemv"), (("bf16", 11, 256, 1, 256, 26, 0), "gemv"),
     (("bf16", 1, 10944, 0, 256, 122, 0), "g32x64k4"), (("bf16", 1, 9216, 0, 256, 48, 0), "gemv"), (("bf16", 16, 3072, 0, 256, 96, 0), "g32x32k4"),
-    # The same of one group of plain columns, to ten rows (fp32 route: six).
-    (("bf16", 6, 4043, 0, 256, 59, 0), "gemv"), (("bf16", 5, 64, 0, 256, 53, 0), "gemv"), (("fp32", 6, 2295, 0, 256, 129, 0), "gemv"),
+    # The same of one group of plain columns, to ten rows (fp32 route: four).
+    (("bf16", 6, 4043, 0, 256, 59, 0), "gemv"), (("bf16", 5, 64, 0, 256, 53, 0), "gemv"), (("fp32", 4, 2295, 0, 256, 129, 0), "gemv"),
     (("bf16", 16, 2880, 0, 256, 60, 0), "g32x32k4"), (("fp32", 13, 2295, 0, 256, 145, 0), "g32x32k4"),
     # One row of three groups on short K; the skinny kernel's slabs past half the CUs.
     (("bf16", 1, 8447, 0, 256, 13, 0), "gemv"), (("bf16", 6, 8352, 0, 256, 11, 0), "skinny"), (("bf16", 10, 9216, 0, 256, 108, 0), "g32x64k4"),
