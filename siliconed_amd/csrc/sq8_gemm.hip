@@ -156,41 +156,34 @@ int choose_wd_tile(int M, int N, bool glu, int cus, int steps, bool f32) {
     // or output type would give one call two sets of bits (launch_wdirect takes 128-row tiles, the same sums, where that
     // kernel cannot serve the product).
     const bool whole = glu ? N / 2 % 32 == 0 : N % 64 == 0;
-    // From 4096 rows on and past 1024 columns no K groups: the tall tiles sum each output's K in one sequence, so a host that
-    // chunks its rows by that many gets the bits of one call. What it costs where 128 × 192 tiles of two groups would fill
-    // the rounds better (µs): 5760 × 3072 × 3072 115.9 → 119.9, with the residual 124.6 → 141.8, fp32 route 309 → 375. Priced
-    // at the clock of long runs of such products.
-    if (M >= 4096 && N > 1024) {
-        const Two t128 = f32 ? Two{21.5f, 5.07f, 28.5f, 2.66f} : Two{8.2f, 1.605f, 7.0f, 0.905f};
-        take(WD_128, t128.of(tiles(128, 8), cus, steps, 0.0f, 0.0f));
-        if (whole) {
-            take(WD_256, (f32 ? One{35.0f, 4.56f, 0.0f} : One{9.0f, 1.445f, 0.0f}).of(tiles(256, 8), cus, steps));
-            take(WD_224, (f32 ? One{32.0f, 4.00f, 0.0f} : One{7.9f, 1.28f, 0.0f}).of(tiles(224, 8), cus, steps));
-        }
-        return tile;
-    }
     // Output rows that are not whole 16 bytes of bf16 are stored value by value in these kernels, not in the K-group ones
-    // (1032 × 512 × 6559 33.4 µs in 128 × 256 and 25.5 in 96 × 192 tiles).
-    const Two t128 = f32 ? Two{9.5f, 4.48f, 7.1f, 2.53f} : Two{8.7f, 1.464f, 5.8f, 0.921f};
-    // Where the two are within 5 % the K groups, whose sums are nearer too (K = 3072, errors against 64 bits: fp32 route 7.2e-7
-    // in one sequence, 3.8e-7 in two groups, 2.7e-7 in four; bf16 route 1.5e-7, 1.0e-7, 0.8e-7).
+    // (1032 × 512 × 6559 33.4 µs in 128 × 256 and 25.5 in 96 × 192 tiles). Where a tile of one sequence and one of K groups
+    // are within 5 % the K groups, whose sums are nearer too (K = 3072, errors against 64 bits: fp32 route 7.2e-7 in one
+    // sequence, 3.8e-7 in two groups, 2.7e-7 in four; bf16 route 1.5e-7, 1.0e-7, 0.8e-7).
     const float nearer = f32 ? 1.05f : 1.0f;
+    const Two t128 = f32 ? Two{10.2f, 4.14f, 7.3f, 2.44f} : Two{7.7f, 1.478f, 5.8f, 0.908f};
     take(WD_128, nearer * t128.of(tiles(128, 8), cus, steps, ragged ? 20.0f : 0.0f, ragged ? 14.0f : 0.0f));
     if (whole) {
-        take(WD_256, nearer * (f32 ? One{12.8f, 3.67f, 1.0f} : One{10.7f, 1.271f, 5.2f}).of(tiles(256, 8), cus, steps));
-        take(WD_224, nearer * (f32 ? One{11.2f, 3.28f, 2.3f} : One{9.5f, 1.151f, 4.7f}).of(tiles(224, 8), cus, steps));
+        take(WD_256, nearer * (f32 ? One{14.8f, 3.49f, 2.9f} : One{11.3f, 1.280f, 3.0f}).of(tiles(256, 8), cus, steps));
+        take(WD_224, nearer * (f32 ? One{13.2f, 3.14f, 2.0f} : One{10.0f, 1.149f, 3.1f}).of(tiles(224, 8), cus, steps));
     }
+    // 64 rows without groups: 64 × 128 of one-block waves, two a CU, and for the GLU epilogues (and wide plain ones) 64 × 256.
+    // They win on few K steps (139 × 384 × 17856 8.2 µs against 12.6 in 64 × 128 of two groups; SiLU-GLU 652 × 3776 × 5120 33.1
+    // against 40.1) and where an odd count of steps leaves only the tiles of four groups (2199 × 12096 × 1728). Not on the fp32
+    // route.
+    if (!f32) {
+        if (!glu) take(WD_64N, 1.05f * Two{3.4f, 0.495f, 2.8f, 0.348f}.of(tiles(64, 4), cus, steps, ragged ? 5.2f : 0.0f, ragged ? 4.6f : 0.0f));
+        take(WD_64, 1.05f * One{ragged ? 12.2f : 4.4f, 0.530f, -0.8f}.of(tiles(64, 8), cus, steps));
+    }
+    // From 4096 rows on and past 1024 columns no K groups: the tiles above sum each output's K in one sequence, so a host that
+    // chunks its rows by that many gets the bits of one call. What it costs where 128 × 192 tiles of two groups would fill
+    // the rounds better (µs): 5760 × 3072 × 3072 115.9 → 119.9, with the residual 124.6 → 141.8, fp32 route 309 → 375.
+    if (M >= 4096 && N > 1024) return tile;
     // A K-group round past the first costs 0.8 µs more.
-    if (f32) {
+    if (f32)
         each_group<GM_F32>(M, blocks, glu, cus, steps, 0.0f, 0.8f, take);
-    } else {
+    else
         each_group<GM_BF16>(M, blocks, glu, cus, steps, 0.0f, 0.8f, take);
-        // 64 rows without groups: 64 × 128 of one-block waves, two a CU, and for the GLU epilogues (and wide plain ones) 64 × 256.
-        // They win on few K steps (139 × 384 × 17856 8.2 µs against 12.6 in 64 × 128 of two groups; SiLU-GLU 652 × 3776 ×
-        // 5120 33.1 against 40.1) and where an odd count of steps leaves only the tiles of four groups (2199 × 12096 × 1728).
-        if (!glu) take(WD_64N, 1.05f * Two{3.5f, 0.500f, 2.8f, 0.348f}.of(tiles(64, 4), cus, steps, ragged ? 5.4f : 0.0f, ragged ? 4.6f : 0.0f));
-        take(WD_64, 1.05f * One{ragged ? 12.2f : 4.3f, 0.540f, -0.8f}.of(tiles(64, 8), cus, steps));
-    }
     return tile;
 }
 

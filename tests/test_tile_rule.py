@@ -91,6 +91,9 @@ def test_short_products_split_k(rule):
     (("bf16", 1119, 2944, 0, 256, 9, 0), "64n"), (("bf16", 1032, 6559, 0, 256, 8, 0), "g128x128k2"),
     (("bf16", 21, 16576, 0, 256, 46, 0), "g64x96k4"), (("bf16", 441, 12800, 1, 256, 24, 0), "128"),
     (("fp32", 855, 8064, 0, 256, 12, 0), "128"), (("fp32", 188, 4640, 0, 256, 4, 0), "g64x64k4"),
+    # Tall products, of few K steps and of many.
+    (("bf16", 7887, 7104, 0, 256, 12, 0), "128"), (("fp32", 5813, 12288, 0, 256, 16, 0), "224"),
+    (("fp32", 6054, 1408, 0, 256, 8, 0), "224"), (("bf16", 4096, 12288, 0, 256, 48, 0), "256"), (("bf16", 4608, 9216, 0, 256, 48, 0), "224"),
     # W8A8: a round of more than one and fewer than two workgroups a CU; rounds of K-group tiles past the first.
     (("w8a8", 3912, 3072, 0, 256, 24, 0), "128"), (("w8a8", 1975, 6144, 0, 256, 24, 0), "128"),
     (("w8a8", 3277, 1024, 1, 256, 8, 0), "g128x128k2"), (("w8a8", 239, 16000, 0, 256, 8, 0), "g128x128k2"),
